@@ -67,7 +67,8 @@ struct VolDesc {
     float* x[2];                 // ping-pong solution
     float* u[2];                 // ping-pong dual variable (3N each)
     float2* spec[SPEC_COUNT];    // half spectra
-    float* q;                    // rho * inv_a / N (half spectrum, real; read by RTS, TV forms it in-kernel)
+    float* q;                    // RTS: inv_a / N (half spectrum, real, tile-major; TV forms its own in-kernel)
+    size_t q_len;                // elements of the tile-major part of q (2 nz more follow: Nyquist plane)
     double* partial;             // per-block (sum d^2, sum x^2) of the C2R pass
     int npartial;
     // inputs / outputs

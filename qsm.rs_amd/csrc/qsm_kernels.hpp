@@ -1440,29 +1440,73 @@ __device__ inline double lap_stencil(int k, int n, double vs) {
     return (n == 1 ? 2.0 : (k == 0 ? 1.0 : 3.0)) / (vs * vs);
 }
 
-// Spectral terms at one index, in FP64 with every operation rounded (no
-// contraction) so threshold decisions match the reference's f64 arithmetic:
+// Spectral terms in FP64 with every operation rounded (no contraction) so
+// threshold decisions match the reference's f64 arithmetic:
 // D = 1/3 - (k.b)^2/|k|^2, 0 where |k|^2 <= 1e-20 (src/kernels/dipole.rs:
 // 24-72), and L, the DFT of the negative Laplacian stencil (lap_stencil per
 // axis; exactly 0 at DC unless an axis has length 1).
-__device__ inline void spec_terms(const VolDesc& V, int kx, int ky, int kz, double& D, double& L) {
-#pragma clang fp contract(off)
-    const double fx = fftfreq_at(kx, V.nx, V.vsx);
-    const double fy = fftfreq_at(ky, V.ny, V.vsy);
-    const double fz = fftfreq_at(kz, V.nz, V.vsz);
-    const double kdb = fx * V.bx + fy * V.by + fz * V.bz;
-    const double k2 = fx * fx + fy * fy + fz * fz;
-    D = (k2 > 1e-20) ? (1.0 / 3.0) - (kdb * kdb) / k2 : 0.0;
-    L = lap_stencil(kx, V.nx, V.vsx) + lap_stencil(ky, V.ny, V.vsy) + lap_stencil(kz, V.nz, V.vsz);
+//
+// Every sum runs over x, y, then z, so the x and y parts are formed once per
+// column (a thread's elements of a z tile share it) and the z part of L, a
+// cosine, once per block into a table.  Formed per element, the six cosines
+// of an index and its mirror bound these passes: 90.5 us for the TKD z pass
+// at 192x192x128 (0.8 TB/s), 145 / 118 us for the two RTS ones at
+// 224x224x144.  The values are the same, bit for bit.
+
+// One axis's share of L: lap_stencil, lap_closed (the Poisson filter), or
+// none where the multiplier does not use L.
+enum LapKind : int { LAP_NONE = 0, LAP_STENCIL = 1, LAP_CLOSED = 2 };
+__device__ inline double lap_axis(int kind, int k, int n, double vs) {
+    return kind == LAP_STENCIL ? lap_stencil(k, n, vs) : (kind == LAP_CLOSED ? lap_closed(k, n, vs) : 0.0);
 }
+
+// (D, L) at an index and at its mirror.
+struct SpecPair {
+    double D, L, Dm, Lm;
+};
+
+// The x and y parts of one column (kx, ky) and of its mirror.
+struct SpecXY {
+    double s, sm;    // fx bx + fy by
+    double k2;       // fx^2 + fy^2 (the same for the mirror: its f are +-f)
+    double l, lm;    // the x and y shares of L
+    double dfz, bz;  // fftfreq step along z, z component of B0
+    __device__ void init(const VolDesc& V, int kx, int ky, int lap) {
+#pragma clang fp contract(off)
+        const int mx = mirror_idx(kx, V.nx), my = mirror_idx(ky, V.ny);
+        const double fx = fftfreq_at(kx, V.nx, V.vsx), fy = fftfreq_at(ky, V.ny, V.vsy);
+        const double fxm = fftfreq_at(mx, V.nx, V.vsx), fym = fftfreq_at(my, V.ny, V.vsy);
+        s = fx * V.bx + fy * V.by;
+        sm = fxm * V.bx + fym * V.by;
+        k2 = fx * fx + fy * fy;
+        l = lap_axis(lap, kx, V.nx, V.vsx) + lap_axis(lap, ky, V.ny, V.vsy);
+        lm = lap_axis(lap, mx, V.nx, V.vsx) + lap_axis(lap, my, V.ny, V.vsy);
+        dfz = 1.0 / ((double)V.nz * V.vsz);
+        bz = V.bz;
+    }
+    // lz: the block's table of z shares (lap_axis at every kz)
+    __device__ __forceinline__ SpecPair at(int kz, int nz, const double* lz) const {
+#pragma clang fp contract(off)
+        const int mz = mirror_idx(kz, nz);
+        const double fz = (double)(kz < (nz + 1) / 2 ? kz : kz - nz) * dfz;
+        const double fzm = (double)(mz < (nz + 1) / 2 ? mz : mz - nz) * dfz;
+        const double kdb = s + fz * bz, kdbm = sm + fzm * bz;
+        const double q2 = k2 + fz * fz;
+        const double kk = kdb * kdb, kkm = kdbm * kdbm;
+        SpecPair p;
+        p.D = (q2 > 1e-20) ? (1.0 / 3.0) - kk / q2 : 0.0;
+        // the mirror's k.b is -k.b but on Nyquist planes
+        p.Dm = kkm == kk ? p.D : ((q2 > 1e-20) ? (1.0 / 3.0) - kkm / q2 : 0.0);
+        p.L = lz ? l + lz[kz] : 0.0;
+        p.Lm = lz ? lm + lz[mz] : 0.0;
+        return p;
+    }
+};
 
 // TV: D inv_a and inv_a, inv_a = 1/(D^2 + rho L) or 0 where |.| <= 1e-20
 // (src/inversion/admm.rs:157-168).
-__device__ inline void tv_multipliers(const VolDesc& V, int kx, int ky, int kz, double& dinv,
-                                      double& inv) {
+__device__ inline void tv_multipliers(const VolDesc& V, double D, double L, double& dinv, double& inv) {
 #pragma clang fp contract(off)
-    double D, L;
-    spec_terms(V, kx, ky, kz, D, L);
     const double a = D * D + V.rho * L;
     inv = (fabs(a) > 1e-20) ? 1.0 / a : 0.0;
     dinv = D * inv;
@@ -1471,22 +1515,12 @@ __device__ inline void tv_multipliers(const VolDesc& V, int kx, int ky, int kz, 
 // RTS (src/inversion/rts.rs:102-183): M = mu on the cone |D| > delta, else 0;
 // inv_a = rho / (M + rho L) or 0; f^ multiplier (M / rho) inv_a where both
 // are non-zero; the ADMM step uses rho = 1, so its multiplier is inv_a.
-__device__ inline void rts_multipliers(const VolDesc& V, int kx, int ky, int kz, double& fm,
-                                       double& inv) {
+__device__ inline void rts_multipliers(const VolDesc& V, double D, double L, double& fm, double& inv) {
 #pragma clang fp contract(off)
-    double D, L;
-    spec_terms(V, kx, ky, kz, D, L);
     const double M = (fabs(D) > V.filt_a) ? V.filt_b : 0.0;
     const double a = M + V.rho * L;
     inv = (fabs(a) > 1e-20) ? V.rho / a : 0.0;
     fm = (fabs(M) > 1e-20 && fabs(inv) > 1e-20) ? (M / V.rho) * inv : 0.0;
-}
-
-// The dipole kernel alone (src/kernels/dipole.rs:24-72).
-__device__ inline double dipole_at(const VolDesc& V, int kx, int ky, int kz) {
-    double D, L;
-    spec_terms(V, kx, ky, kz, D, L);
-    return D;
 }
 
 // Closed-form spectral inversions, one multiplier per frequency:
@@ -1503,10 +1537,8 @@ __device__ inline double dipole_at(const VolDesc& V, int kx, int ky, int kz) {
 enum Filter : int { FILT_TKD = 0, FILT_TSVD = 1, FILT_TIK_ID = 2, FILT_TIK_GRAD = 3, FILT_TIK_LAP = 4,
                     FILT_RTS_X0 = 5, FILT_POISSON = 6 };
 
-__device__ inline double filter_mult(const VolDesc& V, int kx, int ky, int kz) {
+__device__ inline double filter_mult(const VolDesc& V, double D, double L) {
 #pragma clang fp contract(off)
-    double D, L;
-    spec_terms(V, kx, ky, kz, D, L);
     const double p = V.filt_a;
     switch (V.filt) {
         case FILT_TKD: {
@@ -1522,8 +1554,7 @@ __device__ inline double filter_mult(const VolDesc& V, int kx, int ky, int kz) {
             return fabs(denom) > 1e-20 ? D / denom : 0.0;
         }
         case FILT_POISSON: {
-            const double lam = -(lap_closed(kx, V.nx, V.vsx) + lap_closed(ky, V.ny, V.vsy) +
-                                 lap_closed(kz, V.nz, V.vsz));
+            const double lam = -L;
             return fabs(lam) > 1e-20 ? 1.0 / lam : 0.0;
         }
         default: {  // FILT_RTS_X0
@@ -1648,24 +1679,33 @@ struct TvQ {
     }
 };
 
+// The L that the multiplier of an FP64 z pass uses (block-uniform).
+template <int OP>
+__device__ __forceinline__ int lap_kind(const VolDesc& V) {
+    if constexpr (OP == ZOP_DIPOLE) return LAP_NONE;
+    else if constexpr (OP != ZOP_FILTER) return LAP_STENCIL;
+    else
+        return V.filt == FILT_POISSON ? LAP_CLOSED
+                                      : (V.filt == FILT_TIK_GRAD || V.filt == FILT_TIK_LAP ? LAP_STENCIL : LAP_NONE);
+}
+
 // Symmetrised multipliers of the spectral setup at one frequency, averaged
 // over k and its mirror (the reference keeps Re(IFFT(.)) of a full
 // spectrum, the inverse of its Hermitian part; on Nyquist planes D(k) !=
 // D(-k) when B0 is tilted): m for f^ and q = rho inv_a / N (TV) or
 // inv_a / N (RTS).
 template <int OP>
-__device__ inline void setup_mult(const VolDesc& V, int kx, int ky, int kz, double& m, double& qv) {
+__device__ inline void setup_mult(const VolDesc& V, const SpecPair& p, double& m, double& qv) {
     const double invN = 1.0 / ((double)V.nx * V.ny * V.nz);
-    const int mx = mirror_idx(kx, V.nx), my = mirror_idx(ky, V.ny), mz = mirror_idx(kz, V.nz);
     double d1, i1, d2, i2;
     if constexpr (OP == ZOP_TV_SETUP) {
-        tv_multipliers(V, kx, ky, kz, d1, i1);
-        tv_multipliers(V, mx, my, mz, d2, i2);
+        tv_multipliers(V, p.D, p.L, d1, i1);
+        tv_multipliers(V, p.Dm, p.Lm, d2, i2);
         m = 0.5 * (d1 + d2) * invN;
         qv = V.rho * 0.5 * (i1 + i2) * invN;
     } else {
-        rts_multipliers(V, kx, ky, kz, d1, i1);
-        rts_multipliers(V, mx, my, mz, d2, i2);
+        rts_multipliers(V, p.D, p.L, d1, i1);
+        rts_multipliers(V, p.Dm, p.Lm, d2, i2);
         m = 0.5 * (d1 + d2) * invN;
         qv = 0.5 * (i1 + i2) * invN;
     }
@@ -1673,26 +1713,20 @@ __device__ inline void setup_mult(const VolDesc& V, int kx, int ky, int kz, doub
 
 // Symmetrised multiplier of APPLYA (D inv_a / N), DIPOLE (D / N) or FILTER.
 template <int OP>
-__device__ inline double apply_mult(const VolDesc& V, int kx, int ky, int kz) {
+__device__ inline double apply_mult(const VolDesc& V, const SpecPair& p) {
     const double invN = 1.0 / ((double)V.nx * V.ny * V.nz);
-    const int mx = mirror_idx(kx, V.nx), my = mirror_idx(ky, V.ny), mz = mirror_idx(kz, V.nz);
     if constexpr (OP == ZOP_TV_APPLYA) {
         double d1, i1, d2, i2;
-        tv_multipliers(V, kx, ky, kz, d1, i1);
-        tv_multipliers(V, mx, my, mz, d2, i2);
+        tv_multipliers(V, p.D, p.L, d1, i1);
+        tv_multipliers(V, p.Dm, p.Lm, d2, i2);
         return 0.5 * (d1 + d2) * invN;
     } else if constexpr (OP == ZOP_DIPOLE) {
-        return 0.5 * (dipole_at(V, kx, ky, kz) + dipole_at(V, mx, my, mz)) * invN;
+        return 0.5 * (p.D + p.Dm) * invN;
     } else {
-        return 0.5 * (filter_mult(V, kx, ky, kz) + filter_mult(V, mx, my, mz)) * invN;
+        const double m1 = filter_mult(V, p.D, p.L);
+        const double m2 = (p.Dm == p.D && p.Lm == p.L) ? m1 : filter_mult(V, p.Dm, p.Lm);
+        return 0.5 * (m1 + m2) * invN;
     }
-}
-
-// RTS step multiplier q = inv_a / N (symmetrised), in FP64.
-__device__ inline float rts_q(const VolDesc& V, int kx, int ky, int kz) {
-    double m, qv;
-    setup_mult<ZOP_RTS_SETUP>(V, kx, ky, kz, m, qv);
-    return (float)qv;
 }
 
 // TV z pass.  SETUP: forward z of FFT(f) (after x, y), then
@@ -1705,6 +1739,13 @@ __device__ inline float rts_q(const VolDesc& V, int kx, int ky, int kz) {
 // the stored q instead.  ADJ: forward z, -q * spectrum, inverse z (q from
 // TvQ).  APPLYA / DIPOLE: forward z, times the Hermitian part of D inv_a / N
 // or of D / N (in FP64), inverse z.
+// The stored q of the Nyquist plane's half of the two doubly packed columns
+// (ky = 0 and ny / 2, nz values each) follows the tile-major array.  (Formed
+// in FP64 by the 16 threads of such a column at every RTS iteration instead,
+// it held the whole z pass: 85 us at 224x224x144, 1.0 TB/s.)
+__device__ __forceinline__ size_t q_nyq_base(const VolDesc& V, int ky) {
+    return V.q_len + (ky == 0 ? 0 : (size_t)V.nz);
+}
 // The per-iteration ops (SOLVE, SOLVE0, ADJ, RTS_SOLVE) at the lengths of
 // fft_col2.hpp: forward z from the load layout, the product in registers,
 // inverse z back to the load layout; two LDS exchanges in all.
@@ -1793,7 +1834,7 @@ __device__ __forceinline__ void z_tv_col2(const VolDesc& V, float2* lds, float2*
             if (dcol) {
                 const int kz = j + R0 * r;
                 float qB;
-                if constexpr (Q_MEM) qB = rts_q(V, V.nx / 2, ky, kz);
+                if constexpr (Q_MEM) qB = glb(V.q)[q_nyq_base(V, ky) + kz];
                 else qB = tqB.at_plane(kz, N, zqt[kz]);
                 qs = pk_apply(v[r], lds[mirror_idx(kz, N)], qr[r], qB);
             }
@@ -1854,6 +1895,22 @@ __global__ __launch_bounds__(kThreads) void k_z_tv(const VolDesc* __restrict__ v
         return;
     }
     col_load<EMAX, TW>(lds, buf, zs, nz, kx0, nxh);
+    // FP64 multipliers: the z shares of L once per block, in flight of the
+    // tile loads
+    constexpr bool FP64_MULT = OP == ZOP_TV_SETUP || OP == ZOP_RTS_SETUP || OP == ZOP_TV_APPLYA ||
+                               OP == ZOP_DIPOLE || OP == ZOP_FILTER;
+    __shared__ double lzt[FP64_MULT && OP != ZOP_DIPOLE ? tw_lds(N) : 1];
+    const double* const lz = OP == ZOP_DIPOLE ? nullptr : lzt;
+    SpecXY xy, xyB;
+    if constexpr (FP64_MULT) {
+        const int lap = lap_kind<OP>(V);
+        if constexpr (OP != ZOP_DIPOLE)
+            for (int kz = threadIdx.x; kz < nz; kz += kThreads) lzt[kz] = lap_axis(lap, kz, nz, V.vsz);
+        int fx, fy;
+        pk_freq(V, min(kx0 + (int)(threadIdx.x & (TW - 1)), nxh - 1), ky, fx, fy);
+        xy.init(V, fx, fy, lap);
+        if (dpk && (threadIdx.x & (TW - 1)) == 0) xyB.init(V, V.nx / 2, ky, lap);
+    }
     // x-update operands, in flight during the forward FFT
     constexpr bool HAS_F = OP == ZOP_TV_SOLVE || OP == ZOP_RTS_SOLVE;
     constexpr bool Q_MEM = OP == ZOP_RTS_SOLVE;
@@ -1892,7 +1949,7 @@ __global__ __launch_bounds__(kThreads) void k_z_tv(const VolDesc* __restrict__ v
     }
     if constexpr (OP == ZOP_TV_SETUP || OP == ZOP_RTS_SETUP) {
         QSM_GLOBAL float2* F = glb(V.spec[SPEC_A]) + fb;
-        QSM_GLOBAL float* Q = glb(V.q) + fb;
+        [[maybe_unused]] QSM_GLOBAL float* Q = glb(V.q) + fb;
 #pragma unroll
         for (int t = 0; t < EMAX; ++t) {
             const int e = threadIdx.x + t * kThreads;
@@ -1901,21 +1958,19 @@ __global__ __launch_bounds__(kThreads) void k_z_tv(const VolDesc* __restrict__ v
             if (e < total && kx < nxh) {
                 const float2 sv = lds[e];
                 float2 fv;
-                double qv;
+                double m, qv;
+                setup_mult<OP>(V, xy.at(kz, nz, lz), m, qv);
                 if (dcol) {
-                    double mA, mB, qB;
-                    setup_mult<OP>(V, 0, ky, kz, mA, qv);
-                    setup_mult<OP>(V, V.nx / 2, ky, kz, mB, qB);
-                    fv = pk_apply_d(sv, zmir[t], mA, mB);
+                    double mB, qB;
+                    setup_mult<OP>(V, xyB.at(kz, nz, lz), mB, qB);
+                    fv = pk_apply_d(sv, zmir[t], m, mB);
+                    if constexpr (OP == ZOP_RTS_SETUP) glb(V.q)[q_nyq_base(V, ky) + kz] = (float)qB;
                 } else {
-                    int fx, fy;
-                    pk_freq(V, kx, ky, fx, fy);
-                    double m;
-                    setup_mult<OP>(V, fx, fy, kz, m, qv);
                     fv = make_float2((float)((double)sv.x * m), (float)((double)sv.y * m));
                 }
                 stg2(F + kx + kz * TW, fv);
-                Q[kx + kz * TW] = (float)qv;  // (RTS recomputes q in the doubly packed column)
+                // (only RTS reads q back; TV forms it where it is used)
+                if constexpr (OP == ZOP_RTS_SETUP) Q[kx + kz * TW] = (float)qv;
             }
         }
     } else {
@@ -1929,13 +1984,10 @@ __global__ __launch_bounds__(kThreads) void k_z_tv(const VolDesc* __restrict__ v
                     const float2 sv = lds[e];
                     float2 out = make_float2(0.0f, 0.0f);
                     if (kx < nxh) {
+                        const double m = apply_mult<OP>(V, xy.at(kz, nz, lz));
                         if (dcol) {
-                            out = pk_apply_d(sv, zmir[t], apply_mult<OP>(V, 0, ky, kz),
-                                             apply_mult<OP>(V, V.nx / 2, ky, kz));
+                            out = pk_apply_d(sv, zmir[t], m, apply_mult<OP>(V, xyB.at(kz, nz, lz)));
                         } else {
-                            int fx, fy;
-                            pk_freq(V, kx, ky, fx, fy);
-                            const double m = apply_mult<OP>(V, fx, fy, kz);
                             out = make_float2((float)((double)sv.x * m), (float)((double)sv.y * m));
                         }
                     }
@@ -1960,8 +2012,8 @@ __global__ __launch_bounds__(kThreads) void k_z_tv(const VolDesc* __restrict__ v
                     if (dcol) {
                         float qA, qB;
                         if constexpr (Q_MEM) {
-                            qA = rts_q(V, 0, ky, kz);
-                            qB = rts_q(V, V.nx / 2, ky, kz);
+                            qA = qr[t];
+                            qB = glb(V.q)[q_nyq_base(V, ky) + kz];
                         } else {
                             const float2 tz = ztw<N>(V, twl, kz, nz);
                             qA = tq.at(kz, nz, tz);

@@ -594,8 +594,11 @@ static int tv_batch_create_impl(const qsm_tv_volume* vols, size_t n_vols, const 
         // f^ and q: tile-major z-pass operands (zop_base in the kernels)
         if ((rc = dev_alloc(&V.spec[SPEC_A], zop_elems(V)))) return cleanup(rc);
         B->allocs.push_back(V.spec[SPEC_A]);
-        if ((rc = dev_alloc(&V.q, zop_elems(V)))) return cleanup(rc);
-        B->allocs.push_back(V.q);
+        V.q_len = zop_elems(V);
+        if (rts) {
+            if ((rc = dev_alloc(&V.q, V.q_len + 2 * (size_t)V.nz))) return cleanup(rc);
+            B->allocs.push_back(V.q);
+        }
         if ((rc = dev_alloc(&V.partial, 2 * (size_t)pb.cpass))) return cleanup(rc);
         B->allocs.push_back(V.partial);
     }
