@@ -37,10 +37,14 @@ struct Plan {
     int nstages;
     int radix[kMaxStages];
     int ns[kMaxStages];          // product of the radices before stage s
+    int nb[kMaxStages];          // n / radix[s]
+    int tst[kMaxStages];         // n / (ns[s] radix[s]), the twiddle step
     uint64_t m_nb[kMaxStages];   // magic for division by n / radix[s]
     uint64_t m_ns[kMaxStages];   // magic for division by ns[s]
     int tw_off;  // offset (in float2) of this length's table exp(-2 pi i q/n), q<n
     int bl_n, bl_chirp, bl_filt;
+    int dense;      // 1: the stages of fft_dense.hpp
+    int dn_off[3];  // its dense radices' tables (float2 offsets)
 };
 
 __host__ __device__ __forceinline__ float2 cmul(float2 a, float2 b) {
@@ -258,11 +262,10 @@ __host__ __device__ inline StageGeom make_geom(int n, int ncols, int es, int cs,
 // Stage geometry from a plan's precomputed per-stage values (no divisions).
 __host__ __device__ __forceinline__ StageGeom plan_geom(const Plan& P, int s, int ncols, int es, int cs) {
     StageGeom g;
-    const int R = P.radix[s];
     g.n = P.n; g.ncols = ncols; g.es = es; g.cs = cs;
     g.Ns = P.ns[s];
-    g.nb = P.n / R;
-    g.tstep = g.nb / g.Ns;
+    g.nb = P.nb[s];
+    g.tstep = P.tst[s];
     g.m_nb = P.m_nb[s];
     g.m_Ns = P.m_ns[s];
     return g;
@@ -493,6 +496,8 @@ inline bool make_plan_stages(int n, Plan& p) {
     int ns = 1;
     for (int s = 0; s < p.nstages; ++s) {
         p.ns[s] = ns;
+        p.nb[s] = n / p.radix[s];
+        p.tst[s] = n / (ns * p.radix[s]);
         p.m_nb[s] = magic_for((uint32_t)(n / p.radix[s]));
         p.m_ns[s] = magic_for((uint32_t)ns);
         ns *= p.radix[s];

@@ -23,6 +23,8 @@
 // to about R = 200, and the tile stays at n rows.
 #pragma once
 
+#include <cmath>
+
 #include "fft_col2.hpp"
 
 namespace qsmfft {
@@ -37,13 +39,23 @@ template <bool INV> struct Dft<6, INV> : DftSplit<2, 3, INV> {};
 
 __host__ __device__ constexpr int dense_row_tiles(int R) { return (R / 2 + 16) / 16; }  // of the h + 1 rows
 __host__ __device__ constexpr int dense_k_steps(int R) { return (R / 2 + 3) / 4; }
-// float2 entries of a dense radix's coefficient table
-__host__ __device__ constexpr int dense_table_len(int R) { return dense_row_tiles(R) * dense_k_steps(R) * 64; }
+// MFMA steps (of four r) summed before they join the total, whose operands
+// are loaded together: in one chain the error grows with R, 1.9e-7 at 211
+// points against the chirp-z transform's 1.5e-7 (relative, random input); in
+// blocks of 16 r it stays at 1.0e-7.
+constexpr int kDenseBlock = 4;
+// blocks of a radix, and float2 entries of its coefficient table (whole blocks)
+__host__ __device__ constexpr int dense_blocks(int R) { return (dense_k_steps(R) + kDenseBlock - 1) / kDenseBlock; }
+__host__ __device__ constexpr int dense_table_len(int R) {
+    return dense_row_tiles(R) * dense_blocks(R) * kDenseBlock * 64;
+}
 
 // Geometry of one dense stage over a tile.
 struct DenseGeom {
     int R, h, mt, k4;    // rows 0 ... h in mt tiles of 16, k4 steps of four r
+    int kb;              // blocks of kDenseBlock steps
     int items, units;    // butterflies of the tile; (item tile, row tile) pairs
+    int m_mt;            // ceil(2^16 / mt): unit / mt = unit * m_mt >> 16
     int nb, Ns, tstep;   // as StageGeom
     int es, cs, se;      // element and sequence strides, input stride nb * es
     uint64_t m_nb, m_Ns;
@@ -54,11 +66,13 @@ __host__ __device__ __forceinline__ DenseGeom dense_geom(const Plan& P, int s, i
     g.h = g.R / 2;
     g.mt = dense_row_tiles(g.R);
     g.k4 = dense_k_steps(g.R);
-    g.nb = P.n / g.R;
+    g.kb = dense_blocks(g.R);
+    g.nb = P.nb[s];
     g.Ns = P.ns[s];
-    g.tstep = g.nb / g.Ns;
+    g.tstep = P.tst[s];
     g.items = g.nb * ncols;
     g.units = ((g.items + 15) >> 4) * g.mt;
+    g.m_mt = (65536 + g.mt - 1) / g.mt;
     g.es = es;
     g.cs = cs;
     g.se = g.nb * es;
@@ -83,6 +97,11 @@ __host__ __device__ __forceinline__ void dense_item(const DenseGeom& g, int b, i
     in = j * g.es + c * g.cs;
     out = (grp * g.Ns * g.R + k) * g.es + c * g.cs;
     ts = k * g.tstep;
+}
+// Item tile and row tile of a unit (unit < 32).
+__host__ __device__ __forceinline__ void dense_unit(const DenseGeom& g, int unit, int& nt, int& mt) {
+    nt = (unit * g.m_mt) >> 16;
+    mt = unit - nt * g.mt;
 }
 // Lane roles of a unit: operands of step kk at r = dense_r, results v = 0..3
 // at row q = dense_q, item (lane & 15) of the unit's item tile.
@@ -147,72 +166,111 @@ typedef float mfma_f4 __attribute__((ext_vector_type(4)));
 // entry (mt, kk, lane) = (cos, sin)(2 pi q r / R) for the row q = 16 mt +
 // (lane & 15) and the r of dense_r (zero past either end).  All lanes of a
 // wave take part in every MFMA; items past the tile's last repeat it and are
-// not written.  Barriers: the caller's before, one between the reads and the
-// writes, one after.
+// not written.  A block's coefficients are fetched one block ahead (the next
+// unit's included): fetched a step ahead they held each step for an L2 round
+// trip.  Barriers: the caller's before, one between the reads and the writes,
+// one after.
 template <bool COLFAST, int LOG2C, bool INV>
 __device__ __forceinline__ void dense_stage(float2* lds, const DenseGeom& g, const float2* tw,
                                             const float2* __restrict__ coef) {
     const int lane = (int)(threadIdx.x & 63);
     const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int bstep = kDenseBlock * 64;
     mfma_f4 are[kDenseUnits], aim[kDenseUnits], bre[kDenseUnits], bim[kDenseUnits];
+    const mfma_f4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+    float2 w[kDenseBlock];
+    auto fetch = [&](int unit, int kb) {  // in bounds for every unit (mt < g.mt) and kb < g.kb
+        int nt, mt;
+        dense_unit(g, unit, nt, mt);
+        const float2* __restrict__ cf = coef + (mt * g.kb + kb) * bstep;
+#pragma unroll
+        for (int t = 0; t < kDenseBlock; ++t) w[t] = (cf + t * 64)[(unsigned)lane];
+    };
+    fetch(wv, 0);
+    const int se4 = 4 * g.se;
 #pragma unroll
     for (int u = 0; u < kDenseUnits; ++u) {
         const int unit = wv + u * (kThreads / 64);
         if (unit < g.units) {
-            const int nt = unit / g.mt, mt = unit - nt * g.mt;
-            int in, out, ts;
+            int nt, mt, in, out, ts;
+            dense_unit(g, unit, nt, mt);
             dense_item<COLFAST, LOG2C>(g, min(nt * 16 + (lane & 15), g.items - 1), in, out, ts);
             const float2 x0 = lds[in];
-            mfma_f4 ar = {x0.x, x0.x, x0.x, x0.x}, ai = {x0.y, x0.y, x0.y, x0.y};
-            mfma_f4 br = {0.0f, 0.0f, 0.0f, 0.0f}, bi = {0.0f, 0.0f, 0.0f, 0.0f};
-            const float2* __restrict__ cf = coef + mt * g.k4 * 64 + lane;
-            float2 w = *cf;
-            for (int kk = 0; kk < g.k4; ++kk) {
-                const int r = min(dense_r(kk, lane), g.h);  // (coefficients are 0 past h)
-                float2 xa = lds[in + r * g.se], xb = lds[in + (g.R - r) * g.se];
-                cf += 64;
-                const float2 wn = kk + 1 < g.k4 ? *cf : w;  // the next step's, in flight
-                if (g.Ns > 1) {
-                    float2 wa = tw[r * ts], wb = tw[(g.R - r) * ts];
-                    if (INV) {
-                        wa = cconj(wa);
-                        wb = cconj(wb);
+            are[u] = mfma_f4{x0.x, x0.x, x0.x, x0.x};
+            aim[u] = mfma_f4{x0.y, x0.y, x0.y, x0.y};
+            bre[u] = bim[u] = zero;
+            // inputs r and R - r of step 0, stepped by 4; past h (where the
+            // coefficients are 0) they stay inside the butterfly: a whole
+            // block ends at r <= R - 1 for every R >= 17
+            const int r0 = dense_r(0, lane);
+            const float2* pa = lds + in + r0 * g.se;
+            const float2* pb = lds + in + (g.R - r0) * g.se;
+            const float2* ta = tw + r0 * ts;
+            const float2* tb = tw + (g.R - r0) * ts;
+            for (int kb = 0; kb < g.kb; ++kb) {
+                float2 xa[kDenseBlock], xb[kDenseBlock], wc[kDenseBlock];
+#pragma unroll
+                for (int t = 0; t < kDenseBlock; ++t) {
+                    xa[t] = *pa;
+                    xb[t] = *pb;
+                    pa += se4;
+                    pb -= se4;
+                    if (g.Ns > 1) {
+                        float2 wa = *ta, wb = *tb;
+                        ta += 4 * ts;
+                        tb -= 4 * ts;
+                        if (INV) {
+                            wa = cconj(wa);
+                            wb = cconj(wb);
+                        }
+                        xa[t] = cmul(xa[t], wa);
+                        xb[t] = cmul(xb[t], wb);
                     }
-                    xa = cmul(xa, wa);
-                    xb = cmul(xb, wb);
+                    wc[t] = w[t];
                 }
-                const float2 s = cadd(xa, xb), d = csub(xa, xb);
-                ar = __builtin_amdgcn_mfma_f32_16x16x4f32(w.x, s.x, ar, 0, 0, 0);
-                ai = __builtin_amdgcn_mfma_f32_16x16x4f32(w.x, s.y, ai, 0, 0, 0);
-                br = __builtin_amdgcn_mfma_f32_16x16x4f32(w.y, d.x, br, 0, 0, 0);
-                bi = __builtin_amdgcn_mfma_f32_16x16x4f32(w.y, d.y, bi, 0, 0, 0);
-                w = wn;
+                if (kb + 1 < g.kb) fetch(unit, kb + 1);
+                else fetch(unit + kThreads / 64, 0);
+                mfma_f4 ar = zero, ai = zero, br = zero, bi = zero;
+#pragma unroll
+                for (int t = 0; t < kDenseBlock; ++t) {
+                    if (t == 0 || kb * kDenseBlock + t < g.k4) {
+                        const float2 s = cadd(xa[t], xb[t]), d = csub(xa[t], xb[t]);
+                        ar = __builtin_amdgcn_mfma_f32_16x16x4f32(wc[t].x, s.x, ar, 0, 0, 0);
+                        ai = __builtin_amdgcn_mfma_f32_16x16x4f32(wc[t].x, s.y, ai, 0, 0, 0);
+                        br = __builtin_amdgcn_mfma_f32_16x16x4f32(wc[t].y, d.x, br, 0, 0, 0);
+                        bi = __builtin_amdgcn_mfma_f32_16x16x4f32(wc[t].y, d.y, bi, 0, 0, 0);
+                    }
+                }
+                are[u] += ar;
+                aim[u] += ai;
+                bre[u] += br;
+                bim[u] += bi;
             }
-            are[u] = ar;
-            aim[u] = ai;
-            bre[u] = br;
-            bim[u] = bi;
         }
     }
     __syncthreads();
+    const int so = g.Ns * g.es;
 #pragma unroll
     for (int u = 0; u < kDenseUnits; ++u) {
         const int unit = wv + u * (kThreads / 64);
         if (unit < g.units) {
-            const int nt = unit / g.mt, mt = unit - nt * g.mt;
+            int nt, mt, in, out, ts;
+            dense_unit(g, unit, nt, mt);
             const int b = nt * 16 + (lane & 15);
-            int in, out, ts;
             dense_item<COLFAST, LOG2C>(g, min(b, g.items - 1), in, out, ts);
-            const int so = g.Ns * g.es;
+            const int q0 = dense_q(mt, lane, 0);
+            float2* oq = lds + out + q0 * so;
+            float2* om = lds + out + (g.R - q0) * so;
+            const int hv = b < g.items ? g.h : -1;  // (items past the last write nothing)
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
-                const int q = dense_q(mt, lane, v);
-                if (q <= g.h && b < g.items) {
-                    const float2 m = make_float2(are[u][v] + bim[u][v], aim[u][v] - bre[u][v]);  // A - i B
-                    const float2 p = make_float2(are[u][v] - bim[u][v], aim[u][v] + bre[u][v]);  // A + i B
-                    lds[out + q * so] = INV ? p : m;
-                    if (q > 0 && 2 * q != g.R) lds[out + (g.R - q) * so] = INV ? m : p;
-                }
+                const int q = q0 + v;
+                const float2 m = make_float2(are[u][v] + bim[u][v], aim[u][v] - bre[u][v]);  // A - i B
+                const float2 p = make_float2(are[u][v] - bim[u][v], aim[u][v] + bre[u][v]);  // A + i B
+                if (q <= hv) *oq = INV ? p : m;
+                if (q <= hv && q > 0 && 2 * q != g.R) *om = INV ? m : p;
+                oq += so;
+                om -= so;
             }
         }
     }
@@ -262,9 +320,16 @@ __device__ __forceinline__ void lds_fft_dense(float2* lds, const Plan& P, int nc
 
 // --------------------------------------------------------- host planning --
 // Cost of a stage per element, in clocks of one CU: the LDS round trip and
-// its barriers, and for a dense radix its MFMAs (2 mt k4 / R).
+// its barriers, and for a dense radix its MFMAs (2 mt k4 / R).  0: no such
+// stage.  A dense radix has a prime factor above 13: where register radices
+// suffice their fewer roundings are kept (at 40 points 1.2e-7 of the largest
+// output against 1.7e-7 for the dense matrix).
 inline double dense_stage_cost(int R) {
     if (R <= kMaxRegRadix) return 0.55 + 0.004 * R;
+    int m = R;
+    for (int p : {2, 3, 5, 7, 11, 13})
+        while (m % p == 0) m /= p;
+    if (m == 1 || R > kMaxDenseRadix) return 0.0;
     return 0.45 + 2.0 * dense_row_tiles(R) * dense_k_steps(R) / R;
 }
 
@@ -280,9 +345,9 @@ inline bool dense_factorize(int n, int* radix, int* nstages) {
     double best = 0.0;
     *nstages = 0;
     auto offer = [&](int a, int b, int c) {
-        double cost = dense_stage_cost(a);
-        if (b > 1) cost += dense_stage_cost(b);
-        if (c > 1) cost += dense_stage_cost(c);
+        const double ca = dense_stage_cost(a), cb = b > 1 ? dense_stage_cost(b) : 0.0,
+                     cc = c > 1 ? dense_stage_cost(c) : 0.0, cost = ca + cb + cc;
+        if (ca == 0.0 || (b > 1 && cb == 0.0) || (c > 1 && cc == 0.0)) return;
         if (*nstages && cost >= best) return;
         best = cost;
         *nstages = 1 + (b > 1) + (c > 1);
@@ -290,17 +355,11 @@ inline bool dense_factorize(int n, int* radix, int* nstages) {
         radix[1] = b;
         radix[2] = c;
     };
-    for (int a = 2; a <= n && a <= kMaxDenseRadix; ++a) {
+    for (int a = 2; a <= n; ++a) {
         if (n % a) continue;
         const int m = n / a;
-        for (int b = 1; b <= a && b <= m; ++b) {
-            if (m % b) continue;
-            const int c = m / b;
-            if (c <= b || b == 1) {
-                if (b == 1 && c != 1) continue;
-                offer(a, b, c);
-            }
-        }
+        for (int b = 1; b <= a && b <= m; ++b)
+            if (m % b == 0 && m / b <= b) offer(a, b, m / b);  // a >= b >= c
     }
     return *nstages > 0;
 }
@@ -312,6 +371,8 @@ inline bool make_dense_plan(int n, Plan& p) {
     int ns = 1;
     for (int s = 0; s < p.nstages; ++s) {
         p.ns[s] = ns;
+        p.nb[s] = n / p.radix[s];
+        p.tst[s] = n / (ns * p.radix[s]);
         p.m_nb[s] = magic_for((uint32_t)(n / p.radix[s]));
         p.m_ns[s] = magic_for((uint32_t)ns);
         ns *= p.radix[s];
@@ -326,17 +387,21 @@ inline bool make_dense_plan(int n, Plan& p) {
 inline void dense_table(int R, float2* out) {
     const long double two_pi = 6.283185307179586476925286766559L;
     const int h = R / 2;
+    float2 root[kMaxDenseRadix];
+    for (int m = 0; m < R; ++m) {
+        const long double a = two_pi * m / R;
+        root[m] = make_float2((float)cosl(a), (float)sinl(a));
+    }
     for (int mt = 0; mt < dense_row_tiles(R); ++mt)
-        for (int kk = 0; kk < dense_k_steps(R); ++kk)
+        for (int kk = 0; kk < dense_blocks(R) * kDenseBlock; ++kk)
             for (int lane = 0; lane < 64; ++lane) {
                 const int q = 16 * mt + (lane & 15), r = dense_r(kk, lane);
                 float2 w = make_float2(0.0f, 0.0f);
                 if (q <= h && r <= h) {
-                    const long double a = two_pi * ((q * r) % R) / R;
-                    const long double half = 2 * r == R ? 0.5L : 1.0L;
-                    w = make_float2((float)(half * cosl(a)), 2 * r == R ? 0.0f : (float)sinl(a));
+                    w = root[(q * r) % R];
+                    if (2 * r == R) w = make_float2(0.5f * w.x, 0.0f);
                 }
-                out[(mt * dense_k_steps(R) + kk) * 64 + lane] = w;
+                out[(mt * dense_blocks(R) * kDenseBlock + kk) * 64 + lane] = w;
             }
 }
 

@@ -19,7 +19,7 @@
 
 #include <type_traits>
 
-#include "fft_col2.hpp"
+#include "fft_dense.hpp"
 #include "qsm_internal.hpp"
 
 namespace qsm {
@@ -52,19 +52,24 @@ __device__ __forceinline__ void stg2(QSM_GLOBAL float2* p, float2 a) {
     *(QSM_GLOBAL qsm_f2v*)p = v;
 }
 
-// elements per thread of an x (row) pass / a column pass
-__host__ __device__ constexpr int x_emax(int n) {
-    return n > 0 ? (qsmfft::fixed_rows(n) * n + kThreads - 1) / kThreads : kRowEmaxRt;
-}
-__host__ __device__ constexpr int xc_emax(int n) {
-    return n > 0 ? (qsmfft::fixed_rows_c(n) * n + kThreads - 1) / kThreads : kRowEmaxRt;
+// Waves per SIMD that the dense kernels are held to (the others: no bound).
+constexpr int eg_waves(int eg, int w) { return 1; }
+
+// elements per thread of an x (row) pass / a column pass, LDS tile sizes and
+// twiddle entries (n: compiled length or 0; eg: a run-time kernel's EG)
+__host__ __device__ constexpr int x_emax(int n, int eg) {
+    return n > 0 ? (qsmfft::fixed_rows(n) * n + kThreads - 1) / kThreads : (eg_dense(eg) ? eg_elems(eg) : kRowEmaxRt);
 }
 __host__ __device__ constexpr int col_emax(int n, int eg) {
-    return n > 0 ? (kTile * n + kThreads - 1) / kThreads : eg;
+    return n > 0 ? (kTile * n + kThreads - 1) / kThreads : eg_elems(eg);
 }
-__host__ __device__ constexpr int x_lds(int n) { return n > 0 ? qsmfft::fixed_rows(n) * n : kThreads * kRowEmaxRt; }
-__host__ __device__ constexpr int col_lds(int n, int eg) { return n > 0 ? kTile * n : kThreads * eg; }
-__host__ __device__ constexpr int tw_lds(int n) { return n > 0 ? n : kMaxLen; }
+__host__ __device__ constexpr int x_lds(int n, int eg) {
+    return n > 0 ? qsmfft::fixed_rows(n) * n : kThreads * x_emax(n, eg);
+}
+__host__ __device__ constexpr int col_lds(int n, int eg) { return n > 0 ? kTile * n : kThreads * eg_elems(eg); }
+__host__ __device__ constexpr int tw_lds(int n, int eg) {
+    return n > 0 ? n : (eg_dense(eg) ? qsmfft::kMaxDenseLen : kMaxLen);
+}
 // column passes of the lengths fft_col2.hpp covers use its padded layout
 __host__ __device__ constexpr int col_lds2(int n, int eg) {
     return qsmfft::col2_ok(n) ? 16 * n + 256 : col_lds(n, eg);
@@ -78,46 +83,36 @@ __device__ __forceinline__ float2* pp_buffer() {
     return pp;
 }
 
-// The M-point transform of a runtime plan (P.n == M: a chirp-z convolution
-// or a direct length) on the compile-time stages (fft_fixed.hpp), in place
+// The transform of a runtime plan of work length 1024 (a chirp-z convolution,
+// or that length itself) on the compile-time stages (fft_fixed.hpp), in place
 // in buf, when the tile holds the sequences those stages are built for:
 // column tiles of 2^LOG2C columns (layout e * 2^LOG2C + c), or row tiles of
-// kThreads * EMAX / M sequences at stride M.  Returns false (nothing done)
-// otherwise.
-template <int EMAX, bool COLFAST, int LOG2C, bool INV, int M>
-__device__ __forceinline__ bool fixed_pow2_stages(float2* buf, const qsmfft::Plan& P, int ncols,
-                                                  const float2* twl) {
-    constexpr int NC = COLFAST ? (1 << LOG2C) : (kThreads * EMAX) / M;
-    if constexpr (NC < 1 || NC * M > kThreads * EMAX) {
-        return false;
-    } else {
-        if (P.n != M || ncols != NC) return false;
-        qsmfft::fixed_fft<M, NC, COLFAST, INV>(buf, twl);
-        return true;
-    }
+// kThreads * EMAX / 1024 sequences at stride 1024.  Returns false (nothing
+// done) otherwise.
+template <int EMAX, bool COLFAST, int LOG2C, bool INV>
+__device__ __forceinline__ bool fixed_1024_stages(float2* buf, const qsmfft::Plan& P, int ncols, const float2* twl) {
+    constexpr int M = 1024, NC = COLFAST ? (1 << LOG2C) : (kThreads * EMAX) / M;
+    if (P.n != M || ncols != NC) return false;
+    qsmfft::fixed_fft<M, NC, COLFAST, INV>(buf, twl);
+    return true;
 }
 
 // twl: the pass's twiddle table in LDS; twg: the twiddle bank in global
 // memory (the chirp-z tables of runtime-planned lengths).
-template <int N, int EMAX, bool COLFAST, int LOG2C, bool INV, int NC = 0>
+template <int N, int EG, int EMAX, bool COLFAST, int LOG2C, bool INV, int NC = 0>
 __device__ __forceinline__ void run_fft(float2* lds, const qsmfft::Plan& P, int ncols, int es, int cs,
                                         const float2* twl, const float2* twg) {
     if constexpr (N > 0) {
         qsmfft::fixed_fft<N, NC ? NC : (COLFAST ? kTile : qsmfft::fixed_rows(N)), COLFAST, INV>(lds, twl);
+    } else if constexpr (eg_dense(EG)) {
+        qsmfft::lds_fft_dense<COLFAST, LOG2C, INV>(lds, P, ncols, es, cs, twl, twg);
     } else {
-        // runtime-planned lengths: out-of-place stages between the kernel's
-        // tile (kThreads * EMAX elements in every such kernel) and a second
-        // buffer of that size; a transform of length 128, 256, 512 or 1024 (a
-        // chirp-z convolution, or a direct 1024) runs on the compile-time
-        // stages instead, in place, when the tile holds exactly the sequences
-        // they are built for
+        // runtime-planned lengths (513 ... 1024, and chirp-z primes above 256):
+        // out-of-place stages between the kernel's tile (kThreads * EMAX
+        // elements in every such kernel) and a second buffer of that size
         auto inner = [&](float2* src, float2* dst, auto inv, int wes, int wcs) -> float2* {
             constexpr bool I = decltype(inv)::value;
-            if (fixed_pow2_stages<EMAX, COLFAST, LOG2C, I, 128>(src, P, ncols, twl) ||
-                fixed_pow2_stages<EMAX, COLFAST, LOG2C, I, 256>(src, P, ncols, twl) ||
-                fixed_pow2_stages<EMAX, COLFAST, LOG2C, I, 512>(src, P, ncols, twl) ||
-                fixed_pow2_stages<EMAX, COLFAST, LOG2C, I, 1024>(src, P, ncols, twl))
-                return src;
+            if (fixed_1024_stages<EMAX, COLFAST, LOG2C, I>(src, P, ncols, twl)) return src;
             return qsmfft::plan_stages<COLFAST, LOG2C, I>(src, dst, P, ncols, wes, wcs, twl);
         };
         qsmfft::lds_fft_any<COLFAST, LOG2C, INV>(lds, pp_buffer<kThreads * EMAX>(), P, ncols, es, cs, twg, inner);
@@ -130,9 +125,9 @@ __device__ __forceinline__ void run_fft(float2* lds, const qsmfft::Plan& P, int 
 // for one memory round trip before its tile loads went out.
 // The table of plan P (its length P.n: the axis length, or the chirp-z
 // convolution length).
-template <int N>
+template <int N, int EG = 0>
 struct TwStage {
-    static constexpr int K = (tw_lds(N) + kThreads - 1) / kThreads;
+    static constexpr int K = (tw_lds(N, EG) + kThreads - 1) / kThreads;
     float2 r[K];
     int n;
     __device__ __forceinline__ void fetch(const float2* __restrict__ tw, const qsmfft::Plan& P) {
@@ -158,6 +153,18 @@ __device__ __forceinline__ float2 ztw(const VolDesc& V, const float2* twl, int k
         return make_float2(cs, sn);
     }
     return twl[kz];
+}
+
+// e / nx and e / nxh for an element of a row tile (e < 2^16)
+template <int N>
+__device__ __forceinline__ int div_nx(int e, const VolDesc& V) {
+    if constexpr (N > 0) return e / N;
+    else return (int)fastdiv((uint32_t)e, V.m_nx);
+}
+template <int N>
+__device__ __forceinline__ int div_nxh(int e, const VolDesc& V) {
+    if constexpr (N > 0) return e / ((N + 1) / 2);
+    else return (int)fastdiv((uint32_t)e, V.m_nxh);
 }
 
 __device__ __forceinline__ float shrinkf(float x, float t) {
@@ -461,7 +468,7 @@ __device__ __forceinline__ float simple_src(const VolDesc& V, int i, int r, int 
 }
 
 // lds[p*nx + i] = (row 2p, row 2p+1) of the block's rows.
-template <int EMAX, int SRC>
+template <int N, int EMAX, int SRC>
 __device__ __forceinline__ void fill_simple(float2* lds, const VolDesc& V, int nx, int RB, int row0,
                                             int nrows, int aux) {
     const int total = RB * nx;
@@ -469,7 +476,7 @@ __device__ __forceinline__ void fill_simple(float2* lds, const VolDesc& V, int n
 #pragma unroll
     for (int t = 0; t < EMAX; ++t) {
         const int e = threadIdx.x + t * kThreads;
-        const int p = e / nx;
+        const int p = div_nx<N>(e, V);
         const int i = e - p * nx;
         const int ra = row0 + 2 * p, rb = ra + 1;
         r[t].x = (e < total && ra < nrows) ? simple_src<SRC>(V, i, ra, aux) : 0.0f;
@@ -1025,6 +1032,109 @@ __device__ __forceinline__ void fill_tvdiv_rows(float2* lds, const VolDesc& V, i
     }
 }
 
+// The operands of one row of fill_tvdiv_strip in one column.
+struct TvStripRow {
+    float xc, xyp, xym, xzp, xzm, ux, uy, uz, uym, uzm;
+};
+
+// fill_tvdiv for row lengths known only at run time: wave w takes the rows
+// [w nr / 4, (w + 1) nr / 4) of the block's nr = 2 RB, in groups of 62
+// columns.  Lane l of a group holds column c0 + l - 1 (periodic), so the
+// in-row neighbours are lane rotations and lanes 1 ... 62 write.  Row indices
+// are scalar and every load is unconditional; the loads of (group, row) steps
+// run two steps ahead of the arithmetic, across the groups, which keeps some
+// 5 KB per wave in flight (one row ahead, restarted in each group: 86.6 us at
+// 164x205x205).  10 loads a voxel against the element-wise fill's 13, no
+// index division, and a third of its registers.
+__device__ __forceinline__ void fill_tvdiv_strip(float2* lds, const VolDesc& V, int nx, int RB, int row0,
+                                                 int nrows, const QSM_GLOBAL float* __restrict__ x,
+                                                 const QSM_GLOBAL float* __restrict__ u,
+                                                 QSM_GLOBAL float* __restrict__ uo) {
+    constexpr int W = 62;
+    const int ny = V.ny, nz = V.nz;
+    const int nxy = nx * ny, N = nxy * nz;
+    const float t = V.thr, hx = V.hx, hy = V.hy, hz = V.hz;
+    const int lane = (int)(threadIdx.x & 63);
+    const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int q0 = (wv * 2 * RB) >> 2, q1 = ((wv + 1) * 2 * RB) >> 2;
+    const int qe = min(q1, nrows - row0);  // first of the wave's rows past the volume
+    float* ldsf = reinterpret_cast<float*>(lds);
+    // rows past the volume (the last block)
+    for (int q = max(q0, qe); q < q1; ++q)
+        for (int i = lane; i < nx; i += 64) ldsf[2 * ((q >> 1) * nx + i) + (q & 1)] = 0.0f;
+    if (q0 >= qe) return;
+    const int r0 = row0 + q0, k0 = r0 / ny, j0 = r0 - k0 * ny;
+    // load cursor: group column, row, in-plane and plane index
+    int lc = 0, lq = q0, lj = j0, lk = k0;
+    auto load = [&](TvStripRow& R) {
+        const int r = row0 + lq;
+        int ic = lc + lane - 1;
+        ic = ic < 0 ? nx - 1 : (ic < nx ? ic : (ic == nx ? 0 : nx - 1));
+        const unsigned i = (unsigned)ic & (kMaxLen - 1);  // (a bound the compiler sees: scalar base, 32-bit offset)
+        const int dzp = (lk + 1 < nz) ? nxy : nxy - N, dzm = (lk > 0) ? -nxy : N - nxy;
+        const int dyp = (lj + 1 < ny) ? nx : nx - nxy, dym = (lj > 0) ? -nx : nxy - nx;
+        const QSM_GLOBAL float* xr = x + r * nx;
+        const QSM_GLOBAL float* ur = u + r * nx;
+        R.xc = xr[i];
+        R.xyp = (xr + dyp)[i];
+        R.xym = (xr + dym)[i];
+        R.xzp = (xr + dzp)[i];
+        R.xzm = (xr + dzm)[i];
+        R.ux = ur[i];
+        R.uy = (ur + N)[i];
+        R.uz = (ur + 2 * N)[i];
+        R.uym = (ur + N + dym)[i];
+        R.uzm = (ur + 2 * N + dzm)[i];
+        // the next step: its row, or the first row of the next group (past
+        // the last group: the last one again, not used)
+        ++lq;
+        if (++lj == ny) {
+            lj = 0;
+            ++lk;
+        }
+        if (lq == qe) {
+            lq = q0;
+            lj = j0;
+            lk = k0;
+            lc = min(lc + W, (nx - 1) / W * W);
+        }
+    };
+    const int steps = ((nx + W - 1) / W) * (qe - q0);
+    int cc = 0, cq = q0, left = steps;  // step being computed, steps left
+    auto compute = [&](const TvStripRow& R) {
+        const int i = cc + lane - 1;
+        float ox, oy, oz;
+        const float d = tv_voxel(R.xc, lane_next(R.xc), lane_prev(R.xc), R.xyp, R.xym, R.xzp, R.xzm, R.ux, R.uy, R.uz,
+                                 lane_prev(R.ux), R.uym, R.uzm, t, hx, hy, hz, ox, oy, oz);
+        if (lane >= 1 && lane <= W && i < nx && left > 0) {
+            QSM_GLOBAL float* o = uo + (row0 + cq) * nx;
+            const unsigned iu = (unsigned)i & (kMaxLen - 1);
+            o[iu] = ox;
+            (o + N)[iu] = oy;
+            (o + 2 * N)[iu] = oz;
+            ldsf[2 * ((cq >> 1) * nx + i) + (cq & 1)] = d;
+        }
+        if (++cq == qe) {
+            cq = q0;
+            cc += W;
+        }
+        --left;
+    };
+    // (whole rounds of three: under a branch, the merge of its two sides
+    // would wait for the loads in flight)
+    TvStripRow A, B, C;
+    load(A);
+    load(B);
+    for (int s = 0; s < steps; s += 3) {
+        load(C);
+        compute(A);
+        load(A);
+        compute(B);
+        load(B);
+        compute(C);
+    }
+}
+
 // First step of an NLTV Newton round after the first (src/inversion/
 // nltv.rs:86-120): the previous round ended either at convergence (no z/u
 // update) or after max_iter steps (a z/u update with the previous weights is
@@ -1203,15 +1313,15 @@ __device__ __forceinline__ int plane_fast_block(int lb, int ny, int nz, int R) {
 // RBS: the block takes fixed_rows(N) >> RBS pair-rows (small volumes: more,
 // smaller blocks); the host sizes rows_x and the launch the same way.
 template <int N, int EG, int SRC, int RBS = 0>
-__global__ __launch_bounds__(kThreads) void k_r2c_x(const VolDesc* __restrict__ vols, LaunchTable lt,
+__global__ __launch_bounds__(kThreads, eg_waves(EG, 4)) void k_r2c_x(const VolDesc* __restrict__ vols, LaunchTable lt,
                                                     const float2* __restrict__ tw, int out_sel, int aux,
                                                     const VolStatus* status, VolStatus* status_rw,
                                                     VolStatus* mirror, int ck) {
     constexpr int RBX = N > 0 ? (qsmfft::fixed_rows(N) >> RBS) : 0;
     static_assert(N == 0 || RBX >= 1, "row shift too large for this length");
-    constexpr int EMAX = N > 0 ? (RBX * N + kThreads - 1) / kThreads : kRowEmaxRt;
-    __shared__ float2 lds[N > 0 ? RBX * N : x_lds(0)];
-    __shared__ float2 twl[tw_lds(N)];
+    constexpr int EMAX = N > 0 ? (RBX * N + kThreads - 1) / kThreads : x_emax(0, EG);
+    __shared__ float2 lds[N > 0 ? RBX * N : x_lds(0, EG)];
+    __shared__ float2 twl[tw_lds(N, EG)];
     const int bid = xcd_remap(blockIdx.x, gridDim.x);
     int lb;
     const int gv = locate(lt, bid, lb);
@@ -1234,10 +1344,12 @@ __global__ __launch_bounds__(kThreads) void k_r2c_x(const VolDesc* __restrict__ 
                        ? plane_fast_block(lb, V.ny, V.nz, 2 * RB)
                        : lb;
     const int row0 = rb * RB * 2;
-    TwStage<N> tws;
+    TwStage<N, EG> tws;
     tws.fetch(tw, V.px);
     if constexpr (SRC == SRC_TVDIV && tvdiv_rows_form(N, RBX)) {
         fill_tvdiv_rows<N, RBX>(lds, V, row0, nrows, glb(V.x[aux]), glb(V.u[aux ^ 1]), glb(V.u[aux]));
+    } else if constexpr (SRC == SRC_TVDIV && N == 0 && eg_dense(EG)) {
+        fill_tvdiv_strip(lds, V, nx, RB, row0, nrows, glb(V.x[aux]), glb(V.u[aux ^ 1]), glb(V.u[aux]));
     } else if constexpr (SRC == SRC_TVDIV) {
         fill_tvdiv<EMAX, false>(lds, V, nx, RB, glb(V.x[aux]), glb(V.u[aux ^ 1]), glb(V.u[aux]), row0,
                                 nrows, nullptr);
@@ -1262,11 +1374,11 @@ __global__ __launch_bounds__(kThreads) void k_r2c_x(const VolDesc* __restrict__ 
             if (threadIdx.x == 0) glb(V.adj_tpart)[(size_t)ck * V.adj_nblk + lb] = bt;
         }
     } else {
-        fill_simple<EMAX, SRC>(lds, V, nx, RB, row0, nrows, aux);
+        fill_simple<N, EMAX, SRC>(lds, V, nx, RB, row0, nrows, aux);
     }
     tws.commit(twl);
     __syncthreads();
-    run_fft<N, EMAX, false, 0, false, RBX>(lds, V.px, RB, 1, nx, twl, tw);
+    run_fft<N, EG, EMAX, false, 0, false, RBX>(lds, V.px, RB, 1, nx, twl, tw);
     QSM_GLOBAL float2* __restrict__ out = glb(V.spec[out_sel]);
     const int total = RB * nxh;
     if constexpr (N > 0 && N % 4 == 0) {
@@ -1309,7 +1421,7 @@ __global__ __launch_bounds__(kThreads) void k_r2c_x(const VolDesc* __restrict__ 
     for (int t = 0; t < EMAX; ++t) {
         const int e = threadIdx.x + t * kThreads;
         if (e < total) {
-            const int p = e / nxh;
+            const int p = div_nxh<N>(e, V);
             const int k = e - p * nxh;
             const int ra = row0 + 2 * p, rb = ra + 1;
             const float2 zk = lds[p * nx + k];
@@ -1335,14 +1447,14 @@ __global__ __launch_bounds__(kThreads) void k_r2c_x(const VolDesc* __restrict__ 
 // SCHED 0: two-stage column FFT (fft_col2.hpp) where the length allows;
 // SCHED 1: the LDS-staged Stockham stages (less LDS per block).
 template <int N, int EG, bool INV, int SCHED, int TW = kTile>
-__global__ __launch_bounds__(kThreads) void k_y_pass(const VolDesc* __restrict__ vols, LaunchTable lt,
+__global__ __launch_bounds__(kThreads, eg_waves(EG, 4)) void k_y_pass(const VolDesc* __restrict__ vols, LaunchTable lt,
                                                      const float2* __restrict__ tw, int sel, int sel2,
                                                      const VolStatus* __restrict__ status) {
     static_assert(TW == kTile || N == 0, "compiled lengths use tiles of kTile columns");
     constexpr int EMAX = col_emax(N, EG);
     constexpr bool TWO = SCHED == 0 && qsmfft::col2_ok(N);
     __shared__ float2 lds[TWO ? col_lds2(N, EG) : col_lds(N, EG)];
-    __shared__ float2 twl[tw_lds(N)];
+    __shared__ float2 twl[tw_lds(N, EG)];
     const int bid = xcd_remap(blockIdx.x, gridDim.x);
     int lb;
     const int gv = locate(lt, bid, lb);
@@ -1358,7 +1470,7 @@ __global__ __launch_bounds__(kThreads) void k_y_pass(const VolDesc* __restrict__
     const int nxh = V.nxh;
     const int ny = N > 0 ? N : V.ny;
     QSM_GLOBAL float2* buf = glb(V.spec[s]) + (size_t)kz * nxh * ny;
-    TwStage<N> tws;
+    TwStage<N, EG> tws;
     tws.fetch(tw, V.py);
     // tile 0 of an even-nx volume: column 0 is packed (DC and Nyquist planes)
     const bool pkc = tx == 0 && packed_x(V);
@@ -1411,7 +1523,7 @@ __global__ __launch_bounds__(kThreads) void k_y_pass(const VolDesc* __restrict__
         tws.commit(twl);
         __syncthreads();
         if (INV && pkc) ypk_lds<true, TW>(lds, ny);
-        run_fft<N, EMAX, true, tile_log2(TW), INV>(lds, V.py, TW, TW, 1, twl, tw);
+        run_fft<N, EG, EMAX, true, tile_log2(TW), INV>(lds, V.py, TW, TW, 1, twl, tw);
         if (!INV && pkc) ypk_lds<false, TW>(lds, ny);
         col_store<EMAX, TW>(lds, buf, nxh, ny, kx0, nxh);
     }
@@ -1749,8 +1861,8 @@ __device__ __forceinline__ size_t q_nyq_base(const VolDesc& V, int ky) {
 // The per-iteration ops (SOLVE, SOLVE0, ADJ, RTS_SOLVE) at the lengths of
 // fft_col2.hpp: forward z from the load layout, the product in registers,
 // inverse z back to the load layout; two LDS exchanges in all.
-template <int N, int OP>
-__device__ __forceinline__ void z_tv_col2(const VolDesc& V, float2* lds, float2* twl, const TwStage<N>& tws,
+template <int N, int EG, int OP>
+__device__ __forceinline__ void z_tv_col2(const VolDesc& V, float2* lds, float2* twl, const TwStage<N, EG>& tws,
                                           int ky, int kx0, bool dpk) {
     constexpr int R0 = N / 16;
     using C = qsmfft::Col2<R0>;
@@ -1850,14 +1962,14 @@ __device__ __forceinline__ void z_tv_col2(const VolDesc& V, float2* lds, float2*
 }
 
 template <int N, int EG, int OP, int SCHED, int TW = kTile>
-__global__ __launch_bounds__(kThreads) void k_z_tv(const VolDesc* __restrict__ vols, LaunchTable lt,
+__global__ __launch_bounds__(kThreads, eg_waves(EG, 3)) void k_z_tv(const VolDesc* __restrict__ vols, LaunchTable lt,
                                                    const float2* __restrict__ tw,
                                                    const VolStatus* __restrict__ status) {
     constexpr int EMAX = col_emax(N, EG);
     constexpr bool TWO = SCHED == 0 && qsmfft::col2_ok(N) &&
                          (OP == ZOP_TV_SOLVE || OP == ZOP_TV_SOLVE0 || OP == ZOP_TV_ADJ || OP == ZOP_RTS_SOLVE);
     __shared__ float2 lds[TWO ? col_lds2(N, EG) : col_lds(N, EG)];
-    __shared__ float2 twl[tw_lds(N)];
+    __shared__ float2 twl[tw_lds(N, EG)];
     const int bid = xcd_remap(blockIdx.x, gridDim.x);
     int lb;
     const int gv = locate(lt, bid, lb);
@@ -1879,10 +1991,10 @@ __global__ __launch_bounds__(kThreads) void k_z_tv(const VolDesc* __restrict__ v
     // column 0 holds two z spectra (the DC and Nyquist planes at ky = 0, ny/2)
     const bool dpk = pk_double(V, tx, ky);
     QSM_GLOBAL float2* buf = glb(V.spec[SPEC_WORK]) + base;
-    TwStage<N> tws;
+    TwStage<N, EG> tws;
     tws.fetch(tw, V.pz);
     if constexpr (TWO) {
-        z_tv_col2<N, OP>(V, lds, twl, tws, ky, kx0, dpk);
+        z_tv_col2<N, EG, OP>(V, lds, twl, tws, ky, kx0, dpk);
         return;
     }
     if constexpr (OP == ZOP_TV_SOLVE0) {
@@ -1890,7 +2002,7 @@ __global__ __launch_bounds__(kThreads) void k_z_tv(const VolDesc* __restrict__ v
         col_load<EMAX, TW>(lds, glb(V.spec[SPEC_A]) + fb, TW, nz, kx0, nxh);
         tws.commit(twl);
         __syncthreads();
-        run_fft<N, EMAX, true, L2, true>(lds, V.pz, TW, TW, 1, twl, tw);
+        run_fft<N, EG, EMAX, true, L2, true>(lds, V.pz, TW, TW, 1, twl, tw);
         col_store<EMAX, TW>(lds, buf, zs, nz, kx0, nxh);
         return;
     }
@@ -1899,7 +2011,7 @@ __global__ __launch_bounds__(kThreads) void k_z_tv(const VolDesc* __restrict__ v
     // tile loads
     constexpr bool FP64_MULT = OP == ZOP_TV_SETUP || OP == ZOP_RTS_SETUP || OP == ZOP_TV_APPLYA ||
                                OP == ZOP_DIPOLE || OP == ZOP_FILTER;
-    __shared__ double lzt[FP64_MULT && OP != ZOP_DIPOLE ? tw_lds(N) : 1];
+    __shared__ double lzt[FP64_MULT && OP != ZOP_DIPOLE ? tw_lds(N, EG) : 1];
     const double* const lz = OP == ZOP_DIPOLE ? nullptr : lzt;
     SpecXY xy, xyB;
     if constexpr (FP64_MULT) {
@@ -1931,7 +2043,7 @@ __global__ __launch_bounds__(kThreads) void k_z_tv(const VolDesc* __restrict__ v
     }
     tws.commit(twl);
     __syncthreads();
-    run_fft<N, EMAX, true, L2, false>(lds, V.pz, TW, TW, 1, twl, tw);
+    run_fft<N, EG, EMAX, true, L2, false>(lds, V.pz, TW, TW, 1, twl, tw);
     // a thread's elements all lie in column c
     const int c = threadIdx.x & (TW - 1);
     const bool dcol = dpk && c == 0;
@@ -2034,7 +2146,7 @@ __global__ __launch_bounds__(kThreads) void k_z_tv(const VolDesc* __restrict__ v
             }
         }
         __syncthreads();
-        run_fft<N, EMAX, true, L2, true>(lds, V.pz, TW, TW, 1, twl, tw);
+        run_fft<N, EG, EMAX, true, L2, true>(lds, V.pz, TW, TW, 1, twl, tw);
         col_store<EMAX, TW>(lds, buf, zs, nz, kx0, nxh);
     }
 }
@@ -2044,8 +2156,8 @@ __global__ __launch_bounds__(kThreads) void k_z_tv(const VolDesc* __restrict__ v
 // frequencies by conjugate symmetry; the imaginary parts of the DC and
 // Nyquist bins are dropped, as Re(IFFT) of a full spectrum does).
 // step 2: A, B = rows 2p, 2p+1 of sa; step 1: A = row p of sa, B = row p of sb.
-template <int EMAX>
-__device__ __forceinline__ void c2r_load(float2* lds, int nx, int nxh, int RB,
+template <int N, int EMAX>
+__device__ __forceinline__ void c2r_load(float2* lds, const VolDesc& V, int nx, int nxh, int RB,
                                          const QSM_GLOBAL float2* __restrict__ sa,
                                          const QSM_GLOBAL float2* __restrict__ sb, int row0, int step,
                                          int nrows) {
@@ -2054,7 +2166,7 @@ __device__ __forceinline__ void c2r_load(float2* lds, int nx, int nxh, int RB,
 #pragma unroll
     for (int t = 0; t < EMAX; ++t) {
         const int e = threadIdx.x + t * kThreads;
-        const int p = e / nx;
+        const int p = div_nx<N>(e, V);
         const int k = e - p * nx;
         const bool neg = (2 * k > nx);
         const int kk = neg ? nx - k : k;
@@ -2131,12 +2243,12 @@ __device__ __forceinline__ void c2r_load_pairs(float2* lds, const QSM_GLOBAL flo
 
 // c2r_load_pairs where it applies, else c2r_load.
 template <int N, int RBC, int EMAX>
-__device__ __forceinline__ void c2r_load_rows(float2* lds, int nx, int nxh, int RB,
+__device__ __forceinline__ void c2r_load_rows(float2* lds, const VolDesc& V, int nx, int nxh, int RB,
                                               const QSM_GLOBAL float2* __restrict__ sa,
                                               const QSM_GLOBAL float2* __restrict__ sb, int row0, int step,
                                               int nrows) {
     if constexpr (N > 0 && N % 4 == 0) c2r_load_pairs<N, RBC>(lds, sa, sb, row0, step, nrows);
-    else c2r_load<EMAX>(lds, nx, nxh, RB, sa, sb, row0, step, nrows);
+    else c2r_load<N, EMAX>(lds, V, nx, nxh, RB, sa, sb, row0, step, nrows);
 }
 
 // TV: x_it = Re IFFT(x^) (src/inversion/admm.rs:111-114) and the two sums of
@@ -2150,14 +2262,14 @@ __device__ __forceinline__ void c2r_load_rows(float2* lds, int nx, int nxh, int 
 enum C2RMode : int { C2R_TV = 0, C2R_ADJ = 1, C2R_F64 = 2, C2R_F64_MASKED = 3, C2R_X0 = 4 };
 
 template <int N, int EG, int MODE, int RBS = 0>
-__global__ __launch_bounds__(kThreads) void k_c2r_tv(const VolDesc* __restrict__ vols, LaunchTable lt,
+__global__ __launch_bounds__(kThreads, eg_waves(EG, 4)) void k_c2r_tv(const VolDesc* __restrict__ vols, LaunchTable lt,
                                                      const float2* __restrict__ tw, int parity,
                                                      const VolStatus* __restrict__ status) {
     // half the R2C pass's pair-rows (after its row shift RBS), at least 1
     constexpr int RBF = N > 0 ? ((qsmfft::fixed_rows(N) >> RBS) / 2 > 0 ? (qsmfft::fixed_rows(N) >> RBS) / 2 : 1) : 0;
     constexpr int EMAX = N > 0 ? (RBF * N + kThreads - 1) / kThreads : kRowEmaxRt;
-    __shared__ float2 lds[N > 0 ? RBF * N : x_lds(0)];
-    __shared__ float2 twl[tw_lds(N)];
+    __shared__ float2 lds[N > 0 ? RBF * N : kThreads * kRowEmaxRt];
+    __shared__ float2 twl[tw_lds(N, EG)];
     __shared__ double sh[kThreads / 64];
     const int bid = xcd_remap(blockIdx.x, gridDim.x);
     int lb;
@@ -2171,18 +2283,18 @@ __global__ __launch_bounds__(kThreads) void k_c2r_tv(const VolDesc* __restrict__
     const int row0 = lb * RB * 2;
     const int total = RB * nx;
     const QSM_GLOBAL float2* s = glb(V.spec[SPEC_WORK]);
-    TwStage<N> tws;
+    TwStage<N, EG> tws;
     tws.fetch(tw, V.px);
-    c2r_load_rows<N, RBF, EMAX>(lds, nx, nxh, RB, s, s, row0, 2, nrows);
+    c2r_load_rows<N, RBF, EMAX>(lds, V, nx, nxh, RB, s, s, row0, 2, nrows);
     if constexpr (MODE != C2R_TV) {
         tws.commit(twl);
         __syncthreads();
-        run_fft<N, EMAX, false, 0, true, RBF>(lds, V.px, RB, 1, nx, twl, tw);
+        run_fft<N, EG, EMAX, false, 0, true, RBF>(lds, V.px, RB, 1, nx, twl, tw);
 #pragma unroll
         for (int t = 0; t < EMAX; ++t) {
             const int e = threadIdx.x + t * kThreads;
             if (e < total) {
-                const int p = e / nx;
+                const int p = div_nx<N>(e, V);
                 const int i = e - p * nx;
                 const int ra = row0 + 2 * p, rb = ra + 1;
                 const float2 z = lds[e];
@@ -2230,7 +2342,7 @@ __global__ __launch_bounds__(kThreads) void k_c2r_tv(const VolDesc* __restrict__
         }
         tws.commit(twl);
         __syncthreads();
-        run_fft<N, EMAX, false, 0, true, RBF>(lds, V.px, RB, 1, nx, twl, tw);
+        run_fft<N, EG, EMAX, false, 0, true, RBF>(lds, V.px, RB, 1, nx, twl, tw);
         double sd = 0.0, sx = 0.0;
 #pragma unroll
         for (int t = 0; t < E4; ++t) {
@@ -2279,7 +2391,7 @@ __global__ __launch_bounds__(kThreads) void k_c2r_tv(const VolDesc* __restrict__
 #pragma unroll
     for (int t = 0; t < EMAX; ++t) {
         const int e = threadIdx.x + t * kThreads;
-        const int p = e / nx;
+        const int p = div_nx<N>(e, V);
         const int i = e - p * nx;
         // rows past the volume read its last row: always in bounds, never used
         const int ra = min(row0 + 2 * p, nrows - 1), rb = min(row0 + 2 * p + 1, nrows - 1);
@@ -2288,13 +2400,13 @@ __global__ __launch_bounds__(kThreads) void k_c2r_tv(const VolDesc* __restrict__
     }
     tws.commit(twl);
     __syncthreads();
-    run_fft<N, EMAX, false, 0, true, RBF>(lds, V.px, RB, 1, nx, twl, tw);
+    run_fft<N, EG, EMAX, false, 0, true, RBF>(lds, V.px, RB, 1, nx, twl, tw);
     double sd = 0.0, sx = 0.0;
 #pragma unroll
     for (int t = 0; t < EMAX; ++t) {
         const int e = threadIdx.x + t * kThreads;
         if (e < total) {
-            const int p = e / nx;
+            const int p = div_nx<N>(e, V);
             const int i = e - p * nx;
             const int ra = row0 + 2 * p, rb = ra + 1;
             const float2 z = lds[e];
@@ -2333,12 +2445,12 @@ __global__ __launch_bounds__(kThreads) void k_c2r_tv(const VolDesc* __restrict__
 //   -> 0 (src/bgremove/vsharp.rs:180-196; division form of
 //   src/bgremove/sharp.rs:113-123 when divide != 0), scaled by 1/N, inverse z.
 template <int N, int EG, int OP, int TW = kTile>
-__global__ __launch_bounds__(kThreads) void k_z_vs(const VolDesc* __restrict__ vols, LaunchTable lt,
+__global__ __launch_bounds__(kThreads, eg_waves(EG, 3)) void k_z_vs(const VolDesc* __restrict__ vols, LaunchTable lt,
                                                    const float2* __restrict__ tw, int sel, int ridx,
                                                    int flag) {
     constexpr int EMAX = col_emax(N, EG);
     __shared__ float2 lds[col_lds(N, EG)];
-    __shared__ float2 twl[tw_lds(N)];
+    __shared__ float2 twl[tw_lds(N, EG)];
     const int bid = xcd_remap(blockIdx.x, gridDim.x);
     int lb;
     const int gv = locate(lt, bid, lb);
@@ -2355,12 +2467,12 @@ __global__ __launch_bounds__(kThreads) void k_z_vs(const VolDesc* __restrict__ v
     const size_t base = (size_t)ky * nxh;
     const int total = nz * TW;
     QSM_GLOBAL float2* buf = glb(V.spec[OP == ZOP_VS_FWD ? sel : SPEC_WORK]) + base;
-    TwStage<N> tws;
+    TwStage<N, EG> tws;
     tws.fetch(tw, V.pz);
     col_load<EMAX, TW>(lds, buf, zs, nz, kx0, nxh);
     tws.commit(twl);
     __syncthreads();
-    run_fft<N, EMAX, true, L2, false>(lds, V.pz, TW, TW, 1, twl, tw);
+    run_fft<N, EG, EMAX, true, L2, false>(lds, V.pz, TW, TW, 1, twl, tw);
     if constexpr (OP == ZOP_VS_FWD) {
         col_store<EMAX, TW>(lds, buf, zs, nz, kx0, nxh);
     } else {
@@ -2414,7 +2526,7 @@ __global__ __launch_bounds__(kThreads) void k_z_vs(const VolDesc* __restrict__ v
                 }
             }
             __syncthreads();
-            run_fft<N, EMAX, true, L2, true>(lds, V.pz, TW, TW, 1, twl, tw);
+            run_fft<N, EG, EMAX, true, L2, true>(lds, V.pz, TW, TW, 1, twl, tw);
             col_store<EMAX, TW>(lds, buf, zs, nz, kx0, nxh);
             __syncthreads();
 #pragma unroll
@@ -2423,7 +2535,7 @@ __global__ __launch_bounds__(kThreads) void k_z_vs(const VolDesc* __restrict__ v
                 if (e < total) lds[e] = qv[t];
             }
             __syncthreads();
-            run_fft<N, EMAX, true, L2, true>(lds, V.pz, TW, TW, 1, twl, tw);
+            run_fft<N, EG, EMAX, true, L2, true>(lds, V.pz, TW, TW, 1, twl, tw);
             col_store<EMAX, TW>(lds, glb(V.spec[SPEC_C]) + base, zs, nz, kx0, nxh);
         } else {  // ZOP_VS_DECONV
             const double invN = 1.0 / ((double)V.nx * V.ny * V.nz);
@@ -2462,7 +2574,7 @@ __global__ __launch_bounds__(kThreads) void k_z_vs(const VolDesc* __restrict__ v
                 }
             }
             __syncthreads();
-            run_fft<N, EMAX, true, L2, true>(lds, V.pz, TW, TW, 1, twl, tw);
+            run_fft<N, EG, EMAX, true, L2, true>(lds, V.pz, TW, TW, 1, twl, tw);
             col_store<EMAX, TW>(lds, buf, zs, nz, kx0, nxh);
         }
     }
@@ -2477,13 +2589,13 @@ __global__ __launch_bounds__(kThreads) void k_z_vs(const VolDesc* __restrict__ v
 // value of the first (largest) radius whose eroded mask contains it
 // (src/bgremove/vsharp.rs:170-176).
 template <int N, int EG>
-__global__ __launch_bounds__(kThreads) void k_c2r_vs_select(const VolDesc* __restrict__ vols,
+__global__ __launch_bounds__(kThreads, eg_waves(EG, 4)) void k_c2r_vs_select(const VolDesc* __restrict__ vols,
                                                             LaunchTable lt,
                                                             const float2* __restrict__ tw, int ridx,
                                                             double delta) {
-    constexpr int EMAX = x_emax(N);
-    __shared__ float2 lds[x_lds(N)];
-    __shared__ float2 twl[tw_lds(N)];
+    constexpr int EMAX = x_emax(N, EG);
+    __shared__ float2 lds[x_lds(N, EG)];
+    __shared__ float2 twl[tw_lds(N, EG)];
     const int bid = xcd_remap(blockIdx.x, gridDim.x);
     int lb;
     const int gv = locate(lt, bid, lb);
@@ -2493,15 +2605,15 @@ __global__ __launch_bounds__(kThreads) void k_c2r_vs_select(const VolDesc* __res
     const int RB = N > 0 ? qsmfft::fixed_rows(N) : V.rows_x;
     const int nrows = V.ny * V.nz;
     const int row0 = lb * RB;
-    TwStage<N> tws;
+    TwStage<N, EG> tws;
     tws.fetch(tw, V.px);
-    c2r_load_rows<N, (N > 0 ? qsmfft::fixed_rows(N) : 0), EMAX>(lds, nx, nxh, RB, glb(V.spec[SPEC_WORK]),
+    c2r_load_rows<N, (N > 0 ? qsmfft::fixed_rows(N) : 0), EMAX>(lds, V, nx, nxh, RB, glb(V.spec[SPEC_WORK]),
                                                             glb(V.spec[SPEC_C]), row0, 1, nrows);
     tws.commit(twl);
     QSM_GLOBAL uint8_t* fin = glb(V.vs_final);
     QSM_GLOBAL float* loc = glb(V.vs_local);
     __syncthreads();
-    run_fft<N, EMAX, false, 0, true>(lds, V.px, RB, 1, nx, twl, tw);
+    run_fft<N, EG, EMAX, false, 0, true>(lds, V.px, RB, 1, nx, twl, tw);
     const double count = V.vs_counts[ridx];
     const float countf = (float)count;
     const double norm = 1.0 / count;
@@ -2509,7 +2621,7 @@ __global__ __launch_bounds__(kThreads) void k_c2r_vs_select(const VolDesc* __res
 #pragma unroll
     for (int t = 0; t < EMAX; ++t) {
         const int e = threadIdx.x + t * kThreads;
-        const int p = e / nx;
+        const int p = div_nx<N>(e, V);
         const int i = e - p * nx;
         const int r = row0 + p;
         if (e < total && r < nrows) {
@@ -2527,11 +2639,11 @@ __global__ __launch_bounds__(kThreads) void k_c2r_vs_select(const VolDesc* __res
 // Final rows: local = Re IFFT(.) inside the final mask, 0 outside
 // (src/bgremove/vsharp.rs:194-196); also writes the 0/1 mask.
 template <int N, int EG>
-__global__ __launch_bounds__(kThreads) void k_c2r_vs_out(const VolDesc* __restrict__ vols, LaunchTable lt,
+__global__ __launch_bounds__(kThreads, eg_waves(EG, 4)) void k_c2r_vs_out(const VolDesc* __restrict__ vols, LaunchTable lt,
                                                          const float2* __restrict__ tw) {
-    constexpr int EMAX = x_emax(N);
-    __shared__ float2 lds[x_lds(N)];
-    __shared__ float2 twl[tw_lds(N)];
+    constexpr int EMAX = x_emax(N, EG);
+    __shared__ float2 lds[x_lds(N, EG)];
+    __shared__ float2 twl[tw_lds(N, EG)];
     const int bid = xcd_remap(blockIdx.x, gridDim.x);
     int lb;
     const int gv = locate(lt, bid, lb);
@@ -2542,12 +2654,12 @@ __global__ __launch_bounds__(kThreads) void k_c2r_vs_out(const VolDesc* __restri
     const int nrows = V.ny * V.nz;
     const int row0 = lb * RB * 2;
     const QSM_GLOBAL float2* s = glb(V.spec[SPEC_WORK]);
-    TwStage<N> tws;
+    TwStage<N, EG> tws;
     tws.fetch(tw, V.px);
-    c2r_load_rows<N, (N > 0 ? qsmfft::fixed_rows(N) : 0), EMAX>(lds, nx, nxh, RB, s, s, row0, 2, nrows);
+    c2r_load_rows<N, (N > 0 ? qsmfft::fixed_rows(N) : 0), EMAX>(lds, V, nx, nxh, RB, s, s, row0, 2, nrows);
     tws.commit(twl);
     __syncthreads();
-    run_fft<N, EMAX, false, 0, true>(lds, V.px, RB, 1, nx, twl, tw);
+    run_fft<N, EG, EMAX, false, 0, true>(lds, V.px, RB, 1, nx, twl, tw);
     const int total = RB * nx;
     const QSM_GLOBAL uint8_t* fin = glb(V.vs_final);
     QSM_GLOBAL double* out = glb(V.out);
@@ -2556,7 +2668,7 @@ __global__ __launch_bounds__(kThreads) void k_c2r_vs_out(const VolDesc* __restri
     for (int t = 0; t < EMAX; ++t) {
         const int e = threadIdx.x + t * kThreads;
         if (e < total) {
-            const int p = e / nx;
+            const int p = div_nx<N>(e, V);
             const int i = e - p * nx;
             const int ra = row0 + 2 * p, rb = ra + 1;
             const float2 z = lds[e];

@@ -1,13 +1,13 @@
 // One translation unit per specialised axis length: compiled with
 // -DQSM_PASS_N=<length> it defines launch_fixed_<length>(), with
-// -DQSM_PASS_N=0 the runtime-plan fallback launch_generic().
+// -DQSM_PASS_N=0 the kernels of run-time lengths and launch_generic().
 #include "qsm_kernels.hpp"
 
 #ifndef QSM_PASS_N
 #error "compile with -DQSM_PASS_N=<axis length> (0 for the runtime-plan kernels)"
 #endif
 #if QSM_PASS_N == 0 && !defined(QSM_GENERIC_PART)
-#error "the runtime-plan kernels compile with -DQSM_GENERIC_PART=0..3"
+#error "the run-time-length kernels compile with -DQSM_GENERIC_PART=0..4"
 #endif
 
 namespace qsm {
@@ -132,26 +132,32 @@ void QSM_CAT(launch_fixed_, QSM_PASS_N)(int kind, const LaunchTable& lt, const P
     else launch_cols<QSM_PASS_N, 0>(kind, lt, a);
 }
 #elif QSM_GENERIC_PART == 0
-// The runtime-plan kernels are compiled in four parts (this one with the row
-// kernels and the dispatcher) so that they build in parallel.
-void launch_generic_cols(int kind, const LaunchTable& lt, const PassArgs& a);
-void launch_generic_cols_long16(int kind, const LaunchTable& lt, const PassArgs& a);
-void launch_generic_cols_long32(int kind, const LaunchTable& lt, const PassArgs& a);
+// The run-time-length kernels are compiled in five parts (this one with the
+// runtime-plan row kernels and the dispatcher) so that they build in parallel.
+void launch_plan_cols(int kind, const LaunchTable& lt, const PassArgs& a);
+void launch_dense_rows(int kind, const LaunchTable& lt, const PassArgs& a);
+void launch_dense_cols(int kind, const LaunchTable& lt, const PassArgs& a);
+void launch_dense_cols_long(int kind, const LaunchTable& lt, const PassArgs& a);
 void launch_generic(int kind, int emax, const LaunchTable& lt, const PassArgs& a) {
-    if (is_row_kind(kind)) launch_rows<0, 16>(kind, lt, a);
-    else if (emax == kColLongTile + 16) launch_generic_cols_long16(kind, lt, a);  // work length <= 512
-    else if (emax > kColLongTile) launch_generic_cols_long32(kind, lt, a);        // <= 1024
-    else launch_generic_cols(kind, lt, a);                                        // <= 256
+    if (eg_dense(emax)) {
+        if (is_row_kind(kind)) launch_dense_rows(kind, lt, a);
+        else if (eg_elems(emax) > kColLongTile) launch_dense_cols_long(kind, lt, a);  // 257 ... 512
+        else launch_dense_cols(kind, lt, a);                                          // <= 256
+    } else if (is_row_kind(kind)) {
+        launch_rows<0, 16>(kind, lt, a);
+    } else {
+        launch_plan_cols(kind, lt, a);  // work lengths 513 ... 1024
+    }
 }
 #elif QSM_GENERIC_PART == 1
-void launch_generic_cols(int kind, const LaunchTable& lt, const PassArgs& a) { launch_cols<0, 16>(kind, lt, a); }
+void launch_plan_cols(int kind, const LaunchTable& lt, const PassArgs& a) { launch_cols<0, 32, kTileLong>(kind, lt, a); }
 #elif QSM_GENERIC_PART == 2
-void launch_generic_cols_long16(int kind, const LaunchTable& lt, const PassArgs& a) {
-    launch_cols<0, 16, kTileLong>(kind, lt, a);
-}
+void launch_dense_rows(int kind, const LaunchTable& lt, const PassArgs& a) { launch_rows<0, kEgDense + 16>(kind, lt, a); }
+#elif QSM_GENERIC_PART == 3
+void launch_dense_cols(int kind, const LaunchTable& lt, const PassArgs& a) { launch_cols<0, kEgDense + 16>(kind, lt, a); }
 #else
-void launch_generic_cols_long32(int kind, const LaunchTable& lt, const PassArgs& a) {
-    launch_cols<0, 32, kTileLong>(kind, lt, a);
+void launch_dense_cols_long(int kind, const LaunchTable& lt, const PassArgs& a) {
+    launch_cols<0, kEgDense + 16, kTileLong>(kind, lt, a);
 }
 #endif
 

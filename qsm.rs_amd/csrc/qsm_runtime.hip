@@ -2,7 +2,7 @@
 // iteration loop with the reference's progress semantics, and the extern "C"
 // entry points declared in include/qsm_gpu.h.
 #include "qsm_internal.hpp"
-#include "fft_col2.hpp"
+#include "fft_dense.hpp"
 #include "fft_chirp.hpp"
 #include "../../include/qsm_gpu.h"
 
@@ -72,26 +72,26 @@ bool length_ok(size_t n) {
     return direct_length((int)n) || ((int)n <= kMaxChirpLen && chirp_length((int)n) > 0);
 }
 
-// Length the FFT stages of an axis of length n run at (n, or the chirp-z
-// convolution length), which sizes the LDS tiles.
-int work_length(int n) { return direct_length(n) ? n : chirp_length(n); }
-
-// Columns per tile of a column pass of length n: kTile for the compiled
-// lengths and for runtime plans of work length <= 256; kTileLong above (half
-// the LDS per block of the two-buffer transform, so twice the blocks per
-// CU).  Measured, one volume: 164x205x205 (chirp-z on every axis) 4.29 ->
-// 5.14 solves/s and 232x232x160 4.30 -> 4.69 with kTileLong, 130^3 (work
-// length 130) 27.8 -> 26.7, so kTile stays there.
-int col_tile(int n) {
-    if (has_fixed_kernels(n) || work_length(n) <= 256) return kTile;
-    return kTileLong;
+bool dense_length(int n) {
+    int r[3], st;
+    return !has_fixed_kernels(n) && qsmfft::dense_factorize(n, r, &st);
 }
 
-// Runtime-plan column kernel of length n: its elements per thread (EG),
-// plus kColLongTile when it runs in tiles of kTileLong columns.
-int emax_for_col(int n) {
-    if (col_tile(n) == kTileLong) return kColLongTile + (work_length(n) <= 512 ? 16 : 32);
-    return 16;
+// Length the FFT stages of an axis of length n run at (n, or the chirp-z
+// convolution length), which sizes the LDS tiles.
+int work_length(int n) { return dense_length(n) || direct_length(n) ? n : chirp_length(n); }
+
+// Columns per tile of a column pass of length n: kTile up to 256 and for the
+// compiled lengths, kTileLong above (a tile of 4096 elements at most, so four
+// blocks fit a CU's LDS).
+int col_tile(int n) { return has_fixed_kernels(n) || work_length(n) <= 256 ? kTile : kTileLong; }
+
+// Launch size of a pass of length n (compiled kernels ignore it): the EG of
+// the kernels that serve it, plus kColLongTile for dense column kernels in
+// tiles of kTileLong columns.
+int emax_for(int n, bool column) {
+    if (dense_length(n)) return kEgDense + 16 + (column && col_tile(n) == kTileLong ? kColLongTile : 0);
+    return column ? 32 : 16;
 }
 
 // Elements of the tile-major TV / RTS z-pass operands (f^, q) of a volume:
@@ -110,13 +110,23 @@ inline float2 twiddle_entry(int q, int n) {
 
 struct TwiddleBank {
     std::vector<float2> host;
-    std::map<int, int> off, chirp_off, filt_off;
+    std::map<int, int> off, chirp_off, filt_off, dense_off;
     int add(int n) {
         auto it = off.find(n);
         if (it != off.end()) return it->second;
         int o = (int)host.size();
         for (int q = 0; q < n; ++q) host.push_back(twiddle_entry(q, n));
         off[n] = o;
+        return o;
+    }
+    // coefficient table of a dense radix
+    int add_dense(int R) {
+        auto it = dense_off.find(R);
+        if (it != dense_off.end()) return it->second;
+        const int o = (int)host.size();
+        host.resize(o + qsmfft::dense_table_len(R));
+        qsmfft::dense_table(R, host.data() + o);
+        dense_off[R] = o;
         return o;
     }
     // chirp (n entries) and filter (M entries) offsets of length n
@@ -138,44 +148,15 @@ struct TwiddleBank {
     }
 };
 
-// The same tables for one volume (three axes, each at most a length-1024
-// table, or a length-M table plus a chirp of n <= 512 and a filter of M)
-// in fixed storage, for the entry point that allocates nothing.
-struct FixedTwiddleBank {
-    static constexpr int kCap = 3 * (2 * kMaxLen + kMaxChirpLen);
-    float2 host[kCap];
-    int len[6] = {0, 0, 0, 0, 0, 0}, off[6] = {0, 0, 0, 0, 0, 0};
-    int nlen = 0, count = 0;
-    int add(int n) {
-        for (int i = 0; i < nlen; ++i)
-            if (len[i] == n) return off[i];
-        const int o = count;
-        for (int q = 0; q < n; ++q) host[count++] = twiddle_entry(q, n);
-        len[nlen] = n;
-        off[nlen++] = o;
-        return o;
-    }
-    void add_chirp(int n, int M, int& oc, int& of) {
-        for (int i = 0; i < nlen; ++i)
-            if (len[i] == -n) {  // chirp tables are keyed by -n
-                oc = off[i];
-                of = oc + n;
-                return;
-            }
-        std::vector<float2> c, f;
-        chirp_tables(n, M, c, f);
-        oc = count;
-        for (const float2& v : c) host[count++] = v;
-        of = count;
-        for (const float2& v : f) host[count++] = v;
-        len[nlen] = -n;
-        off[nlen++] = oc;
-    }
-};
-
-template <class TB>
-qsmfft::Plan make_plan(int n, TB& tb) {
+qsmfft::Plan make_plan(int n, TwiddleBank& tb) {
     qsmfft::Plan p{};
+    if (dense_length(n)) {
+        qsmfft::make_dense_plan(n, p);
+        p.tw_off = tb.add(n);
+        for (int s = 0; s < p.nstages; ++s)
+            if (p.radix[s] > qsmfft::kMaxRegRadix) p.dn_off[s] = tb.add_dense(p.radix[s]);
+        return p;
+    }
     if (direct_length(n)) {
         qsmfft::make_plan_stages(n, p);
         p.tw_off = tb.add(n);
@@ -225,23 +206,22 @@ struct PassBlocks {
 // Pair-rows per block of the x passes: as many as 16 elements per thread
 // hold (kRowEmaxRt for the runtime-plan kernels), at most 32.
 static int default_rows_x(int nx) {
-    const int tile = qsmfft::kThreads * (has_fixed_kernels(nx) ? 16 : kRowEmaxRt);
+    const int tile = qsmfft::kThreads * (has_fixed_kernels(nx) || dense_length(nx) ? 16 : kRowEmaxRt);
     return std::max(1, std::min(32, tile / work_length(nx)));
 }
 
-// xshift / cshift 2 (compiled lengths only): the R2C / TV C2R passes take a
+// xshift / cshift 2 (compiled and dense lengths): the R2C / TV C2R passes take a
 // quarter of their default rows per block, as the kernels launched with
 // PassArgs::xshift = 2 do (C2R: half the R2C pass's rows before its shift).
-template <class TB>
-PassBlocks fill_geometry(VolDesc& V, const qsm_grid& g, TB& tb, int xshift = 0, int cshift = 0) {
+PassBlocks fill_geometry(VolDesc& V, const qsm_grid& g, TwiddleBank& tb, int xshift = 0, int cshift = 0) {
     V.nx = (int)g.nx; V.ny = (int)g.ny; V.nz = (int)g.nz;
     V.nxh = (V.nx + 1) / 2;  // even nx: DC and Nyquist share column 0
     V.rows_x = default_rows_x(V.nx) >> xshift;
-    // compiled C2R kernels take half the R2C pass's pair-rows (the previous
-    // iterate stays in registers across the transform); the runtime-plan one
-    // its whole tile, whose 8 elements per thread cover it
-    V.rows_c = has_fixed_kernels(V.nx) ? std::max(1, (default_rows_x(V.nx) >> cshift) / 2)
-                                       : default_rows_x(V.nx);
+    // compiled and dense C2R kernels take half the R2C pass's pair-rows (the
+    // previous iterate stays in registers across the transform); the
+    // runtime-plan one its whole tile, whose 8 elements per thread cover it
+    V.rows_c = has_fixed_kernels(V.nx) || dense_length(V.nx) ? std::max(1, (default_rows_x(V.nx) >> cshift) / 2)
+                                                             : default_rows_x(V.nx);
     V.ntx = (V.nxh + kTile - 1) / kTile;
     V.ntx_long = (V.nxh + kTileLong - 1) / kTileLong;
     V.m_nx = qsmfft::magic_for((uint32_t)V.nx);
@@ -289,7 +269,7 @@ Groups make_groups(const std::vector<int>& len, const std::vector<int>& blocks, 
             gs.push_back(PassGroup{});
             g = &gs.back();
             g->n = len[v];
-            g->emax = column ? emax_for_col(len[v]) : 16;
+            g->emax = emax_for(len[v], column);
             g->xshift = sh;
             g->lt.nvol = 0;
             g->lt.start[0] = 0;
@@ -540,7 +520,7 @@ static int tv_batch_create_impl(const qsm_tv_volume* vols, size_t n_vols, const 
     TwiddleBank tb;
     std::vector<int> lx, ly, lz, bx, bc, by, bz, bo;
     auto cleanup = [&](int rc) { batch_free(B); return rc; };
-    // A small volume of a compiled x length, whose R2C pass would launch
+    // A small volume of a compiled or dense x length, whose R2C pass would launch
     // fewer than 1024 blocks (128 for 128x128x64 against ~768 resident), runs
     // that pass with a quarter of the rows per block, and its TV C2R pass
     // likewise, where either keeps at least 4 pair-rows per block (fewer made
@@ -551,7 +531,7 @@ static int tv_batch_create_impl(const qsm_tv_volume* vols, size_t n_vols, const 
     for (size_t v = 0; v < n_vols; ++v) {
         const int nx = (int)vols[v].grid.nx, r0 = default_rows_x(nx), rc = std::max(1, r0 / 2);
         const long npairs = ((long)vols[v].grid.ny * (long)vols[v].grid.nz + 1) / 2;
-        const bool fixed = has_fixed_kernels(nx);
+        const bool fixed = has_fixed_kernels(nx) || dense_length(nx);
         xshift[v] = (fixed && (npairs + r0 - 1) / r0 < 1024 && (r0 >> 2) >= 4) ? 2 : 0;
         cshift[v] = (fixed && (npairs + rc - 1) / rc < 1024 && (r0 >> 2) / 2 >= 4) ? 2 : 0;
     }
@@ -1083,7 +1063,7 @@ static void enqueue_round_trip(int src_kind, int zkind, const VolDesc& V, const 
     a.xshift = 0;
     auto run = [&](int kind, int n, bool column, const LaunchTable& lt) {
         a.sched = column_schedule(kind, n);
-        launch_pass(kind, n, column ? emax_for_col(n) : 16, lt, a);
+        launch_pass(kind, n, emax_for(n, column), lt, a);
     };
     run(src_kind, V.nx, false, tx);
     run(P_Y_FWD, V.ny, true, ty);
@@ -1620,14 +1600,16 @@ int qsm_dipole_adjoint(const double* d_field, const qsm_grid* grid, const double
 
 // ------------------------------------- dipole operator, no allocation ----
 // Workspace of qsm_dipole_forward_noalloc in a file-scope device array: the
-// volume descriptor, the twiddle tables (three lengths <= 1024) and one half
-// spectrum.  Each device holds its own copy until the process ends.  Host
+// volume descriptor, the FFT tables of three lengths and one half spectrum.  Each device holds its own copy until the process ends.  Host
 // code never passes `scratch` itself to a kernel or a copy: its device
 // address comes from hipGetSymbolAddress, once per device.
 namespace {
 constexpr size_t kScratchDescBytes = 4096;
-constexpr size_t kScratchTwBytes = sizeof(float2) * FixedTwiddleBank::kCap;
-constexpr size_t kScratchSpecOff = 65536;
+// three axes, each at most a length-1024 table with a chirp and its filter, or
+// a length-512 table with two dense tables
+constexpr size_t kScratchTwBytes =
+    sizeof(float2) * 3 * (2 * kMaxLen + kMaxChirpLen + 2 * (size_t)qsmfft::dense_table_len(qsmfft::kMaxDenseRadix));
+constexpr size_t kScratchSpecOff = 1 << 20;
 constexpr size_t kScratchSpecBytes = (size_t)72 << 20;
 constexpr size_t kScratchBytes = kScratchSpecOff + kScratchSpecBytes;
 static_assert(sizeof(VolDesc) <= kScratchDescBytes, "descriptor does not fit its scratch slot");
@@ -1667,7 +1649,7 @@ int qsm_dipole_forward_noalloc(const double* d_chi, const qsm_grid* grid, const 
     if (!(bn > 0)) return fail(QSM_EPARAM, "B0 direction has zero length");
     VolDesc V;
     std::memset(&V, 0, sizeof V);
-    FixedTwiddleBank tb;
+    TwiddleBank tb;
     PassBlocks pb = fill_geometry(V, *grid, tb);
     const size_t spec_bytes = (size_t)V.nxh * V.ny * V.nz * sizeof(float2);
     if (spec_bytes > kScratchSpecBytes)
@@ -1687,7 +1669,7 @@ int qsm_dipole_forward_noalloc(const double* d_chi, const qsm_grid* grid, const 
     hipStream_t st = (hipStream_t)stream;
     // The R2C pass writes the whole spectrum, so nothing needs clearing.
     QSM_HIP(hipMemcpyAsync(d_vols, &V, sizeof V, hipMemcpyHostToDevice, st));
-    QSM_HIP(hipMemcpyAsync(d_tw, tb.host, tb.count * sizeof(float2), hipMemcpyHostToDevice, st));
+    QSM_HIP(hipMemcpyAsync(d_tw, tb.host.data(), tb.host.size() * sizeof(float2), hipMemcpyHostToDevice, st));
     enqueue_round_trip(P_R2C_F64, P_Z_DIPOLE, V, pb, d_vols, d_tw, st);
     QSM_CHECK_LAUNCH();
     // the host-side tables above live on this stack frame: wait before returning
