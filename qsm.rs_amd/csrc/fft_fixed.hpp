@@ -174,10 +174,19 @@ __device__ __forceinline__ void fixed_fft(float2* lds, const float2* tw) {
 #endif
 
 // Sequences per block for a row (x) pass of length N: pairs of real rows,
-// at most 32 and at most 16 elements per thread.
+// at most 32 and at most 16 elements per thread; a multiple of 4 up to length
+// 256, so that the four waves of the wave-row fill have the same rows (21 at
+// 192 gave one wave six and the others five).
 constexpr int fixed_rows(int n) {
     int rb = (kThreads * 16) / n;
-    return rb < 1 ? 1 : (rb > 32 ? 32 : rb);
+    rb = rb < 1 ? 1 : (rb > 32 ? 32 : rb);
+    return rb >= 16 ? rb & ~3 : rb;
+}
+// The same with about a quarter of the rows (shift 2: small volumes), 4 or 8:
+// with 5 pair-rows at 192 three waves waited for the fourth's second.
+constexpr int shifted_rows(int n, int shift) {
+    const int rb = fixed_rows(n) >> shift;
+    return shift > 0 && rb >= 4 ? (rb + 2) & ~3 : rb;
 }
 
 // Pair-rows per block of the TV C2R pass: half of the other row passes, so

@@ -40,6 +40,10 @@ constexpr int kEgDense = 1024;
 constexpr bool eg_dense(int eg) { return eg >= kEgDense; }
 constexpr int eg_elems(int eg) { return eg & (kEgDense - 1); }
 
+// Floats allocated past the end of x and u: the run-time-length divergence
+// fill loads up to four columns from any column of a row.
+constexpr int kRowSlack = 4;
+
 struct LaunchTable {
     int nvol;
     int start[kMaxVolumes + 1];  // start[v] = first block of entry v; start[nvol] = total

@@ -674,16 +674,14 @@ __host__ __device__ constexpr bool tvdiv_rows_form(int n, int rb) {
     return n > 0 && n <= 256 && rb >= 4;
 }
 
-// Columns per lane of the wave-row form (VW): 4 or 2 where groups of 256 or
-// 128 columns pad the row no further than groups of 64 do (no more idle
-// lanes), so that every load and store moves 16 or 8 bytes per lane
-// (measured at 256: 277.9 -> 274.8 us per 4-volume launch with 2, 268.2
-// with 4; 151 -> 118 -> 104 VGPRs); otherwise 1.
-__host__ __device__ constexpr int tv_pad(int n, int g) { return (n + g - 1) / g * g; }
+// Columns per lane of the wave-row form (VW): 4 above 128 columns and 2 above
+// 64, one group of lanes for the row, so that every load and store moves 16 or
+// 8 bytes per lane.  Measured at 256, one column per lane against 2 and 4:
+// 277.9, 274.8 and 268.2 us per 4-volume launch; at 144 (three groups of 64
+// columns against 36 lanes of 4) 78.8 and 71.6 us for two 144x192x160 volumes,
+// at 160 81.4 and 79.0, at 176 91.7 and 88.1, at 192 the same.
 __host__ __device__ constexpr int tvdiv_rows_vw(int n) {
-    return (n % 4 == 0 && tv_pad(n, 256) == tv_pad(n, 64))
-               ? 4
-               : ((n % 2 == 0 && tv_pad(n, 128) == tv_pad(n, 64)) ? 2 : 1);
+    return n % 4 == 0 && n > 128 ? 4 : (n % 2 == 0 && n > 64 ? 2 : 1);
 }
 
 template <int VW>
@@ -778,41 +776,25 @@ __device__ __forceinline__ void tvrow_load(TvRow<NX, VW>& R, int r, int k, int n
     }
 }
 
-// The z/u update and the divergence at one voxel (the arithmetic of
-// tvdiv_compute): x and its six neighbours, u and the components of u at
-// the three lower neighbours; writes u' = v - shrink(v), returns div(2z - v).
-__device__ __forceinline__ float tv_voxel(float xc, float xp, float xm, float xyp, float xym, float xzp,
-                                          float xzm, float ux, float uy, float uz, float uxm, float uym,
-                                          float uzm, float t, float hx, float hy, float hz, float& ox,
-                                          float& oy, float& oz) {
-    const float vx = (xp - xc) * hx + ux;
-    const float vy = (xyp - xc) * hy + uy;
-    const float vz = (xzp - xc) * hz + uz;
-    const float vxm = (xc - xm) * hx + uxm;
-    const float vym = (xc - xym) * hy + uym;
-    const float vzm = (xc - xzm) * hz + uzm;
-    const float zx = shrinkf(vx, t), zy = shrinkf(vy, t), zz = shrinkf(vz, t);
-    ox = vx - zx;
-    oy = vy - zy;
-    oz = vz - zz;
-    const float gx = 2.0f * zx - vx, gy = 2.0f * zy - vy, gz = 2.0f * zz - vz;
-    const float gxm = 2.0f * shrinkf(vxm, t) - vxm;
-    const float gym = 2.0f * shrinkf(vym, t) - vym;
-    const float gzm = 2.0f * shrinkf(vzm, t) - vzm;
-    return (gx - gxm) * hx + (gy - gym) * hy + (gz - gzm) * hz;
-}
+// One component of the z/u update for a threshold t >= 0: with z =
+// shrink(v, t), u' = v - z is v clamped to [-t, t] (one v_med3) and g = 2z - v
+// = v - 2u'.  tvdiv_compute's form (two compares and selects, then v - z and
+// 2z - v) took 7 instructions more per component, six components a voxel,
+// and VALU issue was a third of the pass's time.
+__device__ __forceinline__ float tv_clamp(float v, float t) { return __builtin_amdgcn_fmed3f(v, -t, t); }
+__device__ __forceinline__ float tv_g(float v, float u) { return fmaf(-2.0f, u, v); }
+__device__ __forceinline__ float tv_gv(float v, float t) { return tv_g(v, tv_clamp(v, t)); }
 
-// fill_tvdiv with the block's RB pair-rows split over its four waves: wave w
-// takes pair-rows [w RB / 4, (w + 1) RB / 4), lane l the columns VW l ...
-// VW l + VW - 1 (+ 64 VW m).  Row indices are then the same in every lane
-// (scalar), the in-row neighbours come from the lane's own columns and, at
-// their ends, from lane rotations (x and u_x left of the lane's first
-// column from lane l - 1, x right of its last from lane l + 1; with a
-// partial last column group, the periodic wrap between columns NX - 1 and 0
-// from lane broadcasts) and the y neighbours from the wave's neighbouring
-// rows in registers; only the rows above and below the wave's rows, and
-// y-wrapping rows, are loaded again.  Loads per voxel: 7 plus 3 / (rows per
-// wave), against 13.
+// fill_tvdiv (t >= 0) with the block's RB pair-rows split over its four
+// waves: wave w takes pair-rows [w RB / 4, (w + 1) RB / 4), lane l the columns
+// VW l ... VW l + VW - 1 (+ 64 VW m).  Row indices are then the same in every
+// lane (scalar).  x right of the lane's last column comes from a lane rotation
+// (lane l + 1); g's x component left of its first column from lane l - 1, and
+// its y component one row up from the wave's previous row, both already
+// formed (with a partial last column group, the periodic wrap between columns
+// NX - 1 and 0 from lane broadcasts); only the rows above and below the wave's
+// rows, and y-wrapping rows, are loaded again.  Loads per voxel: 7 plus 3 /
+// (rows per wave), against 13.
 template <int NX, int RB>
 __device__ __forceinline__ void fill_tvdiv_rows(float2* lds, const VolDesc& V, int row0, int nrows,
                                                 const QSM_GLOBAL float* __restrict__ x,
@@ -854,7 +836,7 @@ __device__ __forceinline__ void fill_tvdiv_rows(float2* lds, const VolDesc& V, i
 #pragma unroll
         for (int m = 0; m < C; ++m) hym_x[m] = hym_uy[m] = vzero<VW>();
     }
-    vt pxc[C], puy[C], dev[C];
+    vt pgy[C], dev[C];  // g's y component in the previous row; the pair's first row
     // row q of the wave from cur, with the next row's loads issued into nxt;
     // ODD: the second row of a pair-row (the pair goes to LDS)
     auto step = [&](TvRow<NX, VW>& cur, TvRow<NX, VW>& nxt, const int q, auto odd) {
@@ -878,12 +860,19 @@ __device__ __forceinline__ void fill_tvdiv_rows(float2* lds, const VolDesc& V, i
 #pragma unroll
             for (int m = 0; m < C; ++m) hyp_x[m] = okl ? ldv<VW>(xr + tv_col<NX, VW>(lane, m)) : vzero<VW>();
         }
-        vt xym[C], uym[C], xyp[C];
+        vt gym[C], xyp[C];
+        // g's y component at y - 1 where it is not the wave's previous row
+        auto gy_at = [&](const vt& xc, const vt& xm, const vt& um) {
+            float g[VW];
+#pragma unroll
+            for (int e = 0; e < VW; ++e) g[e] = tv_gv((vel<VW>(xc, e) - vel<VW>(xm, e)) * hy + vel<VW>(um, e), t);
+            return vpack<VW>(g);
+        };
         if (!ok) {
             // rows past the volume (the last block): d = 0, nothing stored
 #pragma unroll
             for (int m = 0; m < C; ++m) {
-                xym[m] = uym[m] = xyp[m] = vzero<VW>();
+                gym[m] = xyp[m] = vzero<VW>();
                 cur.xc[m] = cur.ux[m] = cur.uy[m] = cur.uz[m] = vzero<VW>();
                 cur.xzp[m] = cur.xzm[m] = cur.uzm[m] = vzero<VW>();
             }
@@ -891,23 +880,16 @@ __device__ __forceinline__ void fill_tvdiv_rows(float2* lds, const VolDesc& V, i
             // y - 1
             if (q == 0) {
 #pragma unroll
-                for (int m = 0; m < C; ++m) {
-                    xym[m] = hym_x[m];
-                    uym[m] = hym_uy[m];
-                }
+                for (int m = 0; m < C; ++m) gym[m] = gy_at(cur.xc[m], hym_x[m], hym_uy[m]);
             } else if (j == 0) {
                 const int ra = r + ny - 1;
 #pragma unroll
-                for (int m = 0; m < C; ++m) {
-                    xym[m] = ldv<VW>(x + ra * NX + tv_col<NX, VW>(lane, m));
-                    uym[m] = ldv<VW>(u + N + ra * NX + tv_col<NX, VW>(lane, m));
-                }
+                for (int m = 0; m < C; ++m)
+                    gym[m] = gy_at(cur.xc[m], ldv<VW>(x + ra * NX + tv_col<NX, VW>(lane, m)),
+                                   ldv<VW>(u + N + ra * NX + tv_col<NX, VW>(lane, m)));
             } else {
 #pragma unroll
-                for (int m = 0; m < C; ++m) {
-                    xym[m] = pxc[m];
-                    uym[m] = puy[m];
-                }
+                for (int m = 0; m < C; ++m) gym[m] = pgy[m];
             }
             // y + 1
             if (q + 1 == nrw) {
@@ -922,83 +904,69 @@ __device__ __forceinline__ void fill_tvdiv_rows(float2* lds, const VolDesc& V, i
                 for (int m = 0; m < C; ++m) xyp[m] = nxt.xc[m];
             }
         }
-        // in-row neighbours at the ends of the lane's columns: x right of
-        // its last column from lane l + 1 (lane 63: lane 0 of the next
-        // column group), x and u_x left of its first column from lane l - 1
-        // (lane 0: lane 63 of the previous group); columns NX - 1 and 0 are
-        // neighbours (periodic), through lane broadcasts when the last group
-        // is partial
-        float rn[C], rp[C], rpu[C];
+        // x right of the lane's last column from lane l + 1 (lane 63: lane 0
+        // of the next column group); column NX - 1's right neighbour is
+        // column 0 (whole groups: the rotation wraps by itself; a partial
+        // last group: from a lane broadcast)
+        float rn[C];
 #pragma unroll
-        for (int m = 0; m < C; ++m) {
-            rn[m] = lane_next(vfirst<VW>(cur.xc[m]));
-            rp[m] = lane_prev(vlast<VW>(cur.xc[m]));
-            rpu[m] = lane_prev(vlast<VW>(cur.ux[m]));
-        }
-        // (whole groups: the rotations already wrap column NX - 1 to 0)
-        float x0 = 0.0f, xl = 0.0f, uxl = 0.0f;
-        if constexpr (NX % G != 0) {
+        for (int m = 0; m < C; ++m) rn[m] = lane_next(vfirst<VW>(cur.xc[m]));
+        [[maybe_unused]] float x0 = 0.0f;
+        if constexpr (NX % G != 0)
             x0 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, vfirst<VW>(cur.xc[0])), 0));
-            xl = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, vlast<VW>(cur.xc[C - 1])), LV - 1));
-            uxl = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, vlast<VW>(cur.ux[C - 1])), LV - 1));
-        }
-        vt d[C];
+        // the x component of every column of the row, then its left neighbour
+        // (lane l - 1; lane 0: lane 63 of the previous group)
+        float gx[C][VW], ox[C][VW], gl[C];
 #pragma unroll
         for (int m = 0; m < C; ++m) {
             float xp = lane == 63 ? rn[(m + 1) % C] : rn[m];
-            float xm = lane == 0 ? rp[(m + C - 1) % C] : rp[m];
-            float uxm = lane == 0 ? rpu[(m + C - 1) % C] : rpu[m];
             if constexpr (NX % G != 0) {
-                if (m == C - 1 && lane == LV - 1) xp = x0;  // column NX - 1
-                if (m == 0 && lane == 0) {                  // column 0
-                    xm = xl;
-                    uxm = uxl;
-                }
+                if (m == C - 1 && lane == LV - 1) xp = x0;
+            }
+#pragma unroll
+            for (int e = 0; e < VW; ++e) {
+                const float xr = e + 1 < VW ? vel<VW>(cur.xc[m], e + 1) : xp;
+                const float vx = (xr - vel<VW>(cur.xc[m], e)) * hx + vel<VW>(cur.ux[m], e);
+                ox[m][e] = tv_clamp(vx, t);
+                gx[m][e] = tv_g(vx, ox[m][e]);
+            }
+        }
+#pragma unroll
+        for (int m = 0; m < C; ++m) gl[m] = lane_prev(gx[m][VW - 1]);
+        [[maybe_unused]] float glast = 0.0f;
+        if constexpr (NX % G != 0)
+            glast = __builtin_bit_cast(
+                float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, gx[C - 1][VW - 1]), LV - 1));
+        vt d[C];
+#pragma unroll
+        for (int m = 0; m < C; ++m) {
+            float gxm0 = lane == 0 ? gl[(m + C - 1) % C] : gl[m];
+            if constexpr (NX % G != 0) {
+                if (m == 0 && lane == 0) gxm0 = glast;
             }
             const bool col_ok = NX % G == 0 || m < C - 1 || lane < LV;
             QSM_GLOBAL float* o = uo + r * NX + VW * lane + G * m;
-            if constexpr (VW == 1) {
-                // (tv_voxel written out: the same arithmetic, with the stores
-                // between the two halves, in fewer registers)
-                const float xc = cur.xc[m];
-                const float vx = (xp - xc) * hx + cur.ux[m];
-                const float vy = (xyp[m] - xc) * hy + cur.uy[m];
-                const float vz = (cur.xzp[m] - xc) * hz + cur.uz[m];
-                const float vxm = (xc - xm) * hx + uxm;
-                const float vym = (xc - xym[m]) * hy + uym[m];
-                const float vzm = (xc - cur.xzm[m]) * hz + cur.uzm[m];
-                const float zx = shrinkf(vx, t), zy = shrinkf(vy, t), zz = shrinkf(vz, t);
-                if (ok && col_ok) {
-                    o[0] = vx - zx;
-                    o[N] = vy - zy;
-                    o[2 * N] = vz - zz;
-                }
-                const float gx = 2.0f * zx - vx, gy = 2.0f * zy - vy, gz = 2.0f * zz - vz;
-                const float gxm = 2.0f * shrinkf(vxm, t) - vxm;
-                const float gym = 2.0f * shrinkf(vym, t) - vym;
-                const float gzm = 2.0f * shrinkf(vzm, t) - vzm;
-                d[m] = ok ? (gx - gxm) * hx + (gy - gym) * hy + (gz - gzm) * hz : 0.0f;
-            } else {
-                // the lane's columns e = 0 ... VW - 1: in-row neighbours
-                // from its own registers except at the two ends
-                float ox[VW], oy[VW], oz[VW], dd[VW];
+            float oy[VW], oz[VW], gyv[VW], dd[VW];
 #pragma unroll
-                for (int e = 0; e < VW; ++e) {
-                    const float xpe = e + 1 < VW ? vel<VW>(cur.xc[m], e + 1) : xp;
-                    const float xme = e > 0 ? vel<VW>(cur.xc[m], e - 1) : xm;
-                    const float uxme = e > 0 ? vel<VW>(cur.ux[m], e - 1) : uxm;
-                    dd[e] = tv_voxel(vel<VW>(cur.xc[m], e), xpe, xme, vel<VW>(xyp[m], e), vel<VW>(xym[m], e),
-                                     vel<VW>(cur.xzp[m], e), vel<VW>(cur.xzm[m], e), vel<VW>(cur.ux[m], e),
-                                     vel<VW>(cur.uy[m], e), vel<VW>(cur.uz[m], e), uxme, vel<VW>(uym[m], e),
-                                     vel<VW>(cur.uzm[m], e), t, hx, hy, hz, ox[e], oy[e], oz[e]);
-                }
-                if (ok && col_ok) {
-                    stv<VW>(o, vpack<VW>(ox));
-                    stv<VW>(o + N, vpack<VW>(oy));
-                    stv<VW>(o + 2 * N, vpack<VW>(oz));
-                }
-                d[m] = ok ? vpack<VW>(dd) : vzero<VW>();
+            for (int e = 0; e < VW; ++e) {
+                const float xc = vel<VW>(cur.xc[m], e);
+                const float vy = (vel<VW>(xyp[m], e) - xc) * hy + vel<VW>(cur.uy[m], e);
+                const float vz = (vel<VW>(cur.xzp[m], e) - xc) * hz + vel<VW>(cur.uz[m], e);
+                const float vzm = (xc - vel<VW>(cur.xzm[m], e)) * hz + vel<VW>(cur.uzm[m], e);
+                oy[e] = tv_clamp(vy, t);
+                oz[e] = tv_clamp(vz, t);
+                gyv[e] = tv_g(vy, oy[e]);
+                const float gz = tv_g(vz, oz[e]), gzm = tv_gv(vzm, t);
+                const float gxm = e > 0 ? gx[m][e - 1] : gxm0;
+                dd[e] = (gx[m][e] - gxm) * hx + (gyv[e] - vel<VW>(gym[m], e)) * hy + (gz - gzm) * hz;
             }
+            if (ok && col_ok) {
+                stv<VW>(o, vpack<VW>(ox[m]));
+                stv<VW>(o + N, vpack<VW>(oy));
+                stv<VW>(o + 2 * N, vpack<VW>(oz));
+            }
+            pgy[m] = vpack<VW>(gyv);
+            d[m] = ok ? vpack<VW>(dd) : vzero<VW>();
         }
         if constexpr (ODD) {
             const int p = p0 + (q >> 1);
@@ -1015,11 +983,6 @@ __device__ __forceinline__ void fill_tvdiv_rows(float2* lds, const VolDesc& V, i
 #pragma unroll
             for (int m = 0; m < C; ++m) dev[m] = d[m];
         }
-#pragma unroll
-        for (int m = 0; m < C; ++m) {
-            pxc[m] = cur.xc[m];
-            puy[m] = cur.uy[m];
-        }
         j = jn;
         k = kn;
     };
@@ -1032,25 +995,63 @@ __device__ __forceinline__ void fill_tvdiv_rows(float2* lds, const VolDesc& V, i
     }
 }
 
-// The operands of one row of fill_tvdiv_strip in one column.
-struct TvStripRow {
-    float xc, xyp, xym, xzp, xzm, ux, uy, uz, uym, uzm;
+// VW floats at a 4-byte aligned address (one load / store; global memory
+// takes dword alignment).
+template <int VW>
+struct alignas(4) FloatsU {
+    float v[VW];
+};
+template <int VW>
+__device__ __forceinline__ FloatsU<VW> ldu(const QSM_GLOBAL float* p) {
+    if constexpr (VW == 1) {
+        return FloatsU<VW>{{*p}};
+    } else {
+        typedef float vt __attribute__((ext_vector_type(VW), aligned(4)));
+        const vt w = *(const QSM_GLOBAL vt*)p;
+        FloatsU<VW> r;
+#pragma unroll
+        for (int e = 0; e < VW; ++e) r.v[e] = w[e];
+        return r;
+    }
+}
+template <int VW>
+__device__ __forceinline__ void stu(QSM_GLOBAL float* p, const float (&a)[VW]) {
+    if constexpr (VW == 1) {
+        *p = a[0];
+    } else {
+        typedef float vt __attribute__((ext_vector_type(VW), aligned(4)));
+        vt w;
+#pragma unroll
+        for (int e = 0; e < VW; ++e) w[e] = a[e];
+        *(QSM_GLOBAL vt*)p = w;
+    }
+}
+
+// The operands of one row of fill_tvdiv_any in a lane's VW columns, and x and
+// u_x at the row's ends (x0, xl, ul: columns 0 and nx - 1), every lane the same.
+template <int VW>
+struct TvAnyRow {
+    FloatsU<VW> xc, ux, uy, uz, xzp, xzm, uzm;
+    float x0, xl, ul;
 };
 
-// fill_tvdiv for row lengths known only at run time: wave w takes the rows
-// [w nr / 4, (w + 1) nr / 4) of the block's nr = 2 RB, in groups of 62
-// columns.  Lane l of a group holds column c0 + l - 1 (periodic), so the
-// in-row neighbours are lane rotations and lanes 1 ... 62 write.  Row indices
-// are scalar and every load is unconditional; the loads of (group, row) steps
-// run two steps ahead of the arithmetic, across the groups, which keeps some
-// 5 KB per wave in flight (one row ahead, restarted in each group: 86.6 us at
-// 164x205x205).  10 loads a voxel against the element-wise fill's 13, no
-// index division, and a third of its registers.
-__device__ __forceinline__ void fill_tvdiv_strip(float2* lds, const VolDesc& V, int nx, int RB, int row0,
-                                                 int nrows, const QSM_GLOBAL float* __restrict__ x,
-                                                 const QSM_GLOBAL float* __restrict__ u,
-                                                 QSM_GLOBAL float* __restrict__ uo) {
-    constexpr int W = 62;
+// fill_tvdiv (t >= 0) for row lengths known only at run time, in the manner of
+// fill_tvdiv_rows: wave w takes the rows [w nr / 4, (w + 1) nr / 4) of the
+// block's nr = 2 RB, lane l VW consecutive columns.  Rows up to 64 VW columns
+// are one group; longer ones run group by group, 63 VW columns in the first
+// (its last lane only lends its x to the right) and 62 VW in each further one
+// (lane 0 lends g's x component besides).  A lane's columns past the row's end
+// are the next row's first ones: loaded (the buffers end in kRowSlack floats),
+// never used.  The periodic neighbours of columns 0 and nx - 1 come from the
+// row's end values.  Rows need not be aligned.
+// One column per lane with the in-row neighbours loaded took 300 instructions
+// per row of 164 columns and 84 us of a pass whose bytes take 36 us.
+template <int VW>
+__device__ __forceinline__ void fill_tvdiv_any(float2* lds, const VolDesc& V, int nx, int RB, int row0,
+                                               int nrows, const QSM_GLOBAL float* __restrict__ x,
+                                               const QSM_GLOBAL float* __restrict__ u,
+                                               QSM_GLOBAL float* __restrict__ uo) {
+    using Row = TvAnyRow<VW>;
     const int ny = V.ny, nz = V.nz;
     const int nxy = nx * ny, N = nxy * nz;
     const float t = V.thr, hx = V.hx, hy = V.hy, hz = V.hz;
@@ -1063,76 +1064,134 @@ __device__ __forceinline__ void fill_tvdiv_strip(float2* lds, const VolDesc& V, 
     for (int q = max(q0, qe); q < q1; ++q)
         for (int i = lane; i < nx; i += 64) ldsf[2 * ((q >> 1) * nx + i) + (q & 1)] = 0.0f;
     if (q0 >= qe) return;
-    const int r0 = row0 + q0, k0 = r0 / ny, j0 = r0 - k0 * ny;
-    // load cursor: group column, row, in-plane and plane index
-    int lc = 0, lq = q0, lj = j0, lk = k0;
-    auto load = [&](TvStripRow& R) {
-        const int r = row0 + lq;
-        int ic = lc + lane - 1;
-        ic = ic < 0 ? nx - 1 : (ic < nx ? ic : (ic == nx ? 0 : nx - 1));
-        const unsigned i = (unsigned)ic & (kMaxLen - 1);  // (a bound the compiler sees: scalar base, 32-bit offset)
-        const int dzp = (lk + 1 < nz) ? nxy : nxy - N, dzm = (lk > 0) ? -nxy : N - nxy;
-        const int dyp = (lj + 1 < ny) ? nx : nx - nxy, dym = (lj > 0) ? -nx : nxy - nx;
-        const QSM_GLOBAL float* xr = x + r * nx;
-        const QSM_GLOBAL float* ur = u + r * nx;
-        R.xc = xr[i];
-        R.xyp = (xr + dyp)[i];
-        R.xym = (xr + dym)[i];
-        R.xzp = (xr + dzp)[i];
-        R.xzm = (xr + dzm)[i];
-        R.ux = ur[i];
-        R.uy = (ur + N)[i];
-        R.uz = (ur + 2 * N)[i];
-        R.uym = (ur + N + dym)[i];
-        R.uzm = (ur + 2 * N + dzm)[i];
-        // the next step: its row, or the first row of the next group (past
-        // the last group: the last one again, not used)
-        ++lq;
-        if (++lj == ny) {
-            lj = 0;
-            ++lk;
+    const int k0 = (row0 + q0) / ny, j0 = row0 + q0 - k0 * ny;
+    for (int c0 = 0; c0 < nx;) {
+        const int hl = c0 > 0 ? 1 : 0;                          // halo lane on the left
+        const bool last = nx - c0 <= (64 - hl) * VW;            // no halo lane on the right
+        const int c = c0 + VW * (lane - hl);                    // the lane's first column
+        const bool own = lane >= hl && (last || lane < 63) && c < nx;
+        const unsigned cu = (unsigned)min(c, nx - 1) & (kMaxLen - 1);  // (a bound the compiler sees)
+        const int el = nx - 1 - c;                              // element that is the row's last column
+        auto load = [&](Row& R, int r, int k) {
+            const int dzp = (k + 1 < nz) ? nxy : nxy - N, dzm = (k > 0) ? -nxy : N - nxy;
+            const QSM_GLOBAL float* xr = x + r * nx;
+            const QSM_GLOBAL float* ur = u + r * nx;
+            R.xc = ldu<VW>(xr + cu);
+            R.ux = ldu<VW>(ur + cu);
+            R.uy = ldu<VW>(ur + N + cu);
+            R.uz = ldu<VW>(ur + 2 * N + cu);
+            R.xzp = ldu<VW>(xr + dzp + cu);
+            R.xzm = ldu<VW>(xr + dzm + cu);
+            R.uzm = ldu<VW>(ur + 2 * N + dzm + cu);
+            R.x0 = xr[0];
+            R.xl = xr[nx - 1];
+            R.ul = ur[nx - 1];
+        };
+        int j = j0, k = k0;
+        Row A, B;
+        FloatsU<VW> hx_m, hu_m, hx_p;  // rows above / below the wave's rows
+        {
+            const int r = row0 + q0, ra = j > 0 ? r - 1 : r + ny - 1;
+            load(A, r, k);
+            hx_m = ldu<VW>(x + ra * nx + cu);
+            hu_m = ldu<VW>(u + N + ra * nx + cu);
         }
-        if (lq == qe) {
-            lq = q0;
-            lj = j0;
-            lk = k0;
-            lc = min(lc + W, (nx - 1) / W * W);
+        float gym[VW];  // g's y component at y - 1
+        auto gy_from = [&](const FloatsU<VW>& xc, const FloatsU<VW>& xm, const FloatsU<VW>& um) {
+#pragma unroll
+            for (int e = 0; e < VW; ++e) gym[e] = tv_gv((xc.v[e] - xm.v[e]) * hy + um.v[e], t);
+        };
+        // row q from cur, the next row's loads into nxt
+        auto step = [&](const Row& cur, Row& nxt, int q) {
+            const int r = row0 + q;
+            int jn = j + 1, kn = k;
+            if (jn == ny) {
+                jn = 0;
+                ++kn;
+            }
+            const bool more = q + 1 < qe;
+            if (more) load(nxt, r + 1, kn);
+            if (q + 2 >= qe) {  // the row after the wave's last row (or after this one), periodic in y
+                const int rl = more ? r + 1 : r, jl = more ? jn : j;
+                if (q + 2 == qe || q == q0) hx_p = ldu<VW>(x + (jl + 1 < ny ? rl + 1 : rl - ny + 1) * nx + cu);
+            }
+            if (q == q0) {
+                gy_from(cur.xc, hx_m, hu_m);
+            } else if (j == 0) {
+                const int ra = r + ny - 1;
+                gy_from(cur.xc, ldu<VW>(x + ra * nx + cu), ldu<VW>(u + N + ra * nx + cu));
+            }
+            FloatsU<VW> xyp;
+            if (!more) xyp = hx_p;
+            else if (jn == 0) xyp = ldu<VW>(x + (r - ny + 1) * nx + cu);
+            else xyp = nxt.xc;
+            const float rn = lane_next(cur.xc.v[0]);
+            float ox[VW], oy[VW], oz[VW], gx[VW], gy[VW], d[VW];
+#pragma unroll
+            for (int e = 0; e < VW; ++e) {
+                float xp = e + 1 < VW ? cur.xc.v[e + 1 < VW ? e + 1 : 0] : rn;
+                xp = el == e ? cur.x0 : xp;
+                const float vx = (xp - cur.xc.v[e]) * hx + cur.ux.v[e];
+                ox[e] = tv_clamp(vx, t);
+                gx[e] = tv_g(vx, ox[e]);
+            }
+            float gl = lane_prev(gx[VW - 1]);
+            gl = c == 0 ? tv_gv((cur.x0 - cur.xl) * hx + cur.ul, t) : gl;
+#pragma unroll
+            for (int e = 0; e < VW; ++e) {
+                const float xc = cur.xc.v[e];
+                const float vy = (xyp.v[e] - xc) * hy + cur.uy.v[e];
+                const float vz = (cur.xzp.v[e] - xc) * hz + cur.uz.v[e];
+                const float vzm = (xc - cur.xzm.v[e]) * hz + cur.uzm.v[e];
+                oy[e] = tv_clamp(vy, t);
+                oz[e] = tv_clamp(vz, t);
+                gy[e] = tv_g(vy, oy[e]);
+                d[e] = (gx[e] - (e > 0 ? gx[e > 0 ? e - 1 : 0] : gl)) * hx + (gy[e] - gym[e]) * hy +
+                       (tv_g(vz, oz[e]) - tv_gv(vzm, t)) * hz;
+                gym[e] = gy[e];
+            }
+            if (own) {
+                QSM_GLOBAL float* o = uo + r * nx + cu;
+                float* l = ldsf + 2 * ((q >> 1) * nx + c) + (q & 1);
+                if (el >= VW - 1) {
+                    stu<VW>(o, ox);
+                    stu<VW>(o + N, oy);
+                    stu<VW>(o + 2 * N, oz);
+#pragma unroll
+                    for (int e = 0; e < VW; ++e) l[2 * e] = d[e];
+                } else {
+#pragma unroll
+                    for (int e = 0; e < VW - 1; ++e) {
+                        if (e <= el) {
+                            o[e] = ox[e];
+                            (o + N)[e] = oy[e];
+                            (o + 2 * N)[e] = oz[e];
+                            l[2 * e] = d[e];
+                        }
+                    }
+                }
+            }
+            j = jn;
+            k = kn;
+        };
+        int q = q0;
+        for (; q + 1 < qe; q += 2) {
+            step(A, B, q);
+            step(B, A, q + 1);
         }
-    };
-    const int steps = ((nx + W - 1) / W) * (qe - q0);
-    int cc = 0, cq = q0, left = steps;  // step being computed, steps left
-    auto compute = [&](const TvStripRow& R) {
-        const int i = cc + lane - 1;
-        float ox, oy, oz;
-        const float d = tv_voxel(R.xc, lane_next(R.xc), lane_prev(R.xc), R.xyp, R.xym, R.xzp, R.xzm, R.ux, R.uy, R.uz,
-                                 lane_prev(R.ux), R.uym, R.uzm, t, hx, hy, hz, ox, oy, oz);
-        if (lane >= 1 && lane <= W && i < nx && left > 0) {
-            QSM_GLOBAL float* o = uo + (row0 + cq) * nx;
-            const unsigned iu = (unsigned)i & (kMaxLen - 1);
-            o[iu] = ox;
-            (o + N)[iu] = oy;
-            (o + 2 * N)[iu] = oz;
-            ldsf[2 * ((cq >> 1) * nx + i) + (cq & 1)] = d;
-        }
-        if (++cq == qe) {
-            cq = q0;
-            cc += W;
-        }
-        --left;
-    };
-    // (whole rounds of three: under a branch, the merge of its two sides
-    // would wait for the loads in flight)
-    TvStripRow A, B, C;
-    load(A);
-    load(B);
-    for (int s = 0; s < steps; s += 3) {
-        load(C);
-        compute(A);
-        load(A);
-        compute(B);
-        load(B);
-        compute(C);
+        if (q < qe) step(A, B, q);
+        c0 += (64 - hl - (last ? 0 : 1)) * VW;
     }
+}
+
+// Columns per lane of fill_tvdiv_any: rows up to 256 columns in one group.
+__device__ __forceinline__ void fill_tvdiv_runtime(float2* lds, const VolDesc& V, int nx, int RB, int row0, int nrows,
+                                                   const QSM_GLOBAL float* __restrict__ x,
+                                                   const QSM_GLOBAL float* __restrict__ u,
+                                                   QSM_GLOBAL float* __restrict__ uo) {
+    if (nx <= 64) fill_tvdiv_any<1>(lds, V, nx, RB, row0, nrows, x, u, uo);
+    else if (nx <= 128) fill_tvdiv_any<2>(lds, V, nx, RB, row0, nrows, x, u, uo);
+    else fill_tvdiv_any<4>(lds, V, nx, RB, row0, nrows, x, u, uo);
 }
 
 // First step of an NLTV Newton round after the first (src/inversion/
@@ -1310,14 +1369,14 @@ __device__ __forceinline__ int plane_fast_block(int lb, int ny, int nz, int R) {
 // aux: TV iteration parity for SRC_TVDIV, radius index for SRC_SPHERE.
 // ck: checkpoint index (SRC_TVDIV_REC: the record written; SRC_TVADJ: the
 // record read, and the row of adj_tpart written).
-// RBS: the block takes fixed_rows(N) >> RBS pair-rows (small volumes: more,
+// RBS: the block takes shifted_rows(N, RBS) pair-rows (small volumes: more,
 // smaller blocks); the host sizes rows_x and the launch the same way.
 template <int N, int EG, int SRC, int RBS = 0>
 __global__ __launch_bounds__(kThreads, eg_waves(EG, 4)) void k_r2c_x(const VolDesc* __restrict__ vols, LaunchTable lt,
                                                     const float2* __restrict__ tw, int out_sel, int aux,
                                                     const VolStatus* status, VolStatus* status_rw,
                                                     VolStatus* mirror, int ck) {
-    constexpr int RBX = N > 0 ? (qsmfft::fixed_rows(N) >> RBS) : 0;
+    constexpr int RBX = N > 0 ? qsmfft::shifted_rows(N, RBS) : 0;
     static_assert(N == 0 || RBX >= 1, "row shift too large for this length");
     constexpr int EMAX = N > 0 ? (RBX * N + kThreads - 1) / kThreads : x_emax(0, EG);
     __shared__ float2 lds[N > 0 ? RBX * N : x_lds(0, EG)];
@@ -1349,7 +1408,7 @@ __global__ __launch_bounds__(kThreads, eg_waves(EG, 4)) void k_r2c_x(const VolDe
     if constexpr (SRC == SRC_TVDIV && tvdiv_rows_form(N, RBX)) {
         fill_tvdiv_rows<N, RBX>(lds, V, row0, nrows, glb(V.x[aux]), glb(V.u[aux ^ 1]), glb(V.u[aux]));
     } else if constexpr (SRC == SRC_TVDIV && N == 0 && eg_dense(EG)) {
-        fill_tvdiv_strip(lds, V, nx, RB, row0, nrows, glb(V.x[aux]), glb(V.u[aux ^ 1]), glb(V.u[aux]));
+        fill_tvdiv_runtime(lds, V, nx, RB, row0, nrows, glb(V.x[aux]), glb(V.u[aux ^ 1]), glb(V.u[aux]));
     } else if constexpr (SRC == SRC_TVDIV) {
         fill_tvdiv<EMAX, false>(lds, V, nx, RB, glb(V.x[aux]), glb(V.u[aux ^ 1]), glb(V.u[aux]), row0,
                                 nrows, nullptr);

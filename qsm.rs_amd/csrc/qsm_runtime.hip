@@ -206,7 +206,8 @@ struct PassBlocks {
 // Pair-rows per block of the x passes: as many as 16 elements per thread
 // hold (kRowEmaxRt for the runtime-plan kernels), at most 32.
 static int default_rows_x(int nx) {
-    const int tile = qsmfft::kThreads * (has_fixed_kernels(nx) || dense_length(nx) ? 16 : kRowEmaxRt);
+    if (has_fixed_kernels(nx)) return qsmfft::fixed_rows(nx);
+    const int tile = qsmfft::kThreads * (dense_length(nx) ? 16 : kRowEmaxRt);
     return std::max(1, std::min(32, tile / work_length(nx)));
 }
 
@@ -216,7 +217,8 @@ static int default_rows_x(int nx) {
 PassBlocks fill_geometry(VolDesc& V, const qsm_grid& g, TwiddleBank& tb, int xshift = 0, int cshift = 0) {
     V.nx = (int)g.nx; V.ny = (int)g.ny; V.nz = (int)g.nz;
     V.nxh = (V.nx + 1) / 2;  // even nx: DC and Nyquist share column 0
-    V.rows_x = default_rows_x(V.nx) >> xshift;
+    V.rows_x = has_fixed_kernels(V.nx) ? qsmfft::shifted_rows(V.nx, xshift) : default_rows_x(V.nx) >> xshift;
+    if (dense_length(V.nx) && V.rows_x > 2) V.rows_x &= ~1;  // the same rows for each of the fill's four waves
     // compiled and dense C2R kernels take half the R2C pass's pair-rows (the
     // previous iterate stays in registers across the transform); the
     // runtime-plan one its whole tile, whose 8 elements per thread cover it
@@ -350,6 +352,10 @@ using namespace qsm;
 struct qsm_tv_batch {
     int nvol = 0;
     int method = 0;  // 0 TV-ADMM (src/inversion/tv.rs), 1 RTS (src/inversion/rts.rs)
+    // The fused z/u update clamps to [-t, t], t = lambda / rho >= 0; for any
+    // other t (a negative lambda, say) the recording kernel, which forms
+    // shrink itself, runs in its place with a scratch record.
+    bool plain_shrink = false;
     qsm_tv_params params{};
     std::vector<VolDesc> h;
     VolDesc* d_vols = nullptr;
@@ -552,6 +558,7 @@ static int tv_batch_create_impl(const qsm_tv_volume* vols, size_t n_vols, const 
             V.filt_b = rts->mu;
             V.lsmr_iter = (int)rts->lsmr_iter;
         }
+        if (!(V.thr >= 0.0f)) B->plain_shrink = true;
         V.field = vols[v].d_field;
         V.mask = vols[v].d_mask;
         V.out = vols[v].d_chi;
@@ -564,9 +571,9 @@ static int tv_batch_create_impl(const qsm_tv_volume* vols, size_t n_vols, const 
         const size_t Nh = (size_t)V.nxh * V.ny * V.nz;
         int rc;
         for (int p = 0; p < 2; ++p) {
-            if ((rc = dev_alloc(&V.x[p], N))) return cleanup(rc);
+            if ((rc = dev_alloc(&V.x[p], N + kRowSlack))) return cleanup(rc);
             B->allocs.push_back(V.x[p]);
-            if ((rc = dev_alloc(&V.u[p], 3 * N))) return cleanup(rc);
+            if ((rc = dev_alloc(&V.u[p], 3 * N + kRowSlack))) return cleanup(rc);
             B->allocs.push_back(V.u[p]);
         }
         if ((rc = dev_alloc(&V.spec[SPEC_WORK], Nh))) return cleanup(rc);
@@ -581,6 +588,13 @@ static int tv_batch_create_impl(const qsm_tv_volume* vols, size_t n_vols, const 
         }
         if ((rc = dev_alloc(&V.partial, 2 * (size_t)pb.cpass))) return cleanup(rc);
         B->allocs.push_back(V.partial);
+    }
+    if (B->plain_shrink) {
+        for (auto& V : B->h) {
+            int rc;
+            if ((rc = dev_alloc(&V.ckpt, 3 * (size_t)V.nx * V.ny * V.nz))) return cleanup(rc);
+            B->allocs.push_back(V.ckpt);
+        }
     }
     B->gx = make_groups(lx, bx, false, &xshift);
     B->gxc = make_groups(lx, bc, false, &cshift);
@@ -689,9 +703,10 @@ static int enqueue_iteration(qsm_tv_batch* B, size_t it, hipEvent_t closed, int 
         a.status_rw = B->d_status;
         a.mirror = B->h_status_dev;
     }
-    a.ridx = rec;
+    const bool record = rec >= 0 || B->plain_shrink;
+    a.ridx = std::max(rec, 0);
     int rc;
-    if ((rc = run_pass(B, 0, rec >= 0 ? P_R2C_TVDIV_REC : P_R2C_TVDIV, B->gx, a))) return rc;
+    if ((rc = run_pass(B, 0, record ? P_R2C_TVDIV_REC : P_R2C_TVDIV, B->gx, a))) return rc;
     if (closed) QSM_HIP(hipEventRecord(closed, B->stream));
     a.status_rw = nullptr;
     a.mirror = nullptr;
@@ -869,7 +884,7 @@ static int tv_batch_profile_impl(qsm_tv_batch* B, size_t iters, double* ms_out, 
         a.parity = (int)((it - 1) & 1);
         a.status_rw = it >= 2 ? B->d_status : nullptr;
         QSM_HIP(hipEventRecord(ev[0], st));
-        run_groups(P_R2C_TVDIV, B->gx, a);
+        run_groups(B->plain_shrink ? P_R2C_TVDIV_REC : P_R2C_TVDIV, B->gx, a);
         a.status_rw = nullptr;
         QSM_HIP(hipEventRecord(ev[1], st));
         run_groups(P_Y_FWD, B->gy, a);
