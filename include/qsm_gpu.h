@@ -311,6 +311,11 @@ int qsm_memcpy_htod(void* dst, const void* src, size_t bytes);
 int qsm_memcpy_dtoh(void* dst, const void* src, size_t bytes);
 int qsm_memcpy_dtod(void* dst, const void* src, size_t bytes);
 int qsm_device_synchronize(void);
+/* The library keeps device workspaces (at most 2 GiB over all devices),
+ * streams and pinned staging buffers (at most 16 MiB a device) of finished
+ * calls for later ones; they are given back when the device runs out of
+ * memory, and by this call. */
+void qsm_release_cached_memory(void);
 /* Achievable HBM rate reference: a one-element-per-thread device copy of
  * `bytes`, read + write counted, best of `reps` launches (GB/s). */
 int qsm_hbm_copy_probe(size_t bytes, int reps, double* gbps);

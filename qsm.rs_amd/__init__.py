@@ -202,6 +202,7 @@ _SIGS = {
     "qsm_memcpy_dtoh": (C.c_int, [C.c_void_p, C.c_void_p, _SZ]),
     "qsm_memcpy_dtod": (C.c_int, [C.c_void_p, C.c_void_p, _SZ]),
     "qsm_device_synchronize": (C.c_int, []),
+    "qsm_release_cached_memory": (None, []),
     "qsm_hbm_copy_probe": (C.c_int, [_SZ, C.c_int, _D]),
     "qsm_hbm_stream_probe": (C.c_int, [_SZ, C.c_int, C.c_int, C.c_int, _D]),
 }
@@ -818,6 +819,11 @@ def fft_schedule(axis: str, n: int) -> str:
 
 def synchronize():
     _check(_lib.qsm_device_synchronize())
+
+
+def release_cached_memory():
+    """Give back the workspaces, streams and pinned buffers kept of finished calls."""
+    _lib.qsm_release_cached_memory()
 
 
 def copy_device(dst: DeviceArray, src: DeviceArray):

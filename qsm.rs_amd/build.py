@@ -23,7 +23,7 @@ FIXED_LENGTHS = [48, 64, 72, 80, 96, 112, 120, 128, 144, 150, 160, 168, 176, 180
                  224, 240, 256, 288, 320, 384, 416, 448, 480, 512]
 UNITS = ([("qsm_pass.hip", f"qsm_pass_0_{k}", ["-DQSM_PASS_N=0", f"-DQSM_GENERIC_PART={k}"]) for k in range(5)]
          + [("qsm_pass.hip", f"qsm_pass_{n}", [f"-DQSM_PASS_N={n}"]) for n in FIXED_LENGTHS]
-         + [("qsm_misc.hip", "qsm_misc", []), ("qsm_runtime.hip", "qsm_runtime", []),
+         + [("qsm_misc.hip", "qsm_misc", []), ("qsm_runtime.hip", "qsm_runtime", []), ("qsm_hostmem.hip", "qsm_hostmem", []),
             ("qsm_nifti.hip", "qsm_nifti", [])])
 
 HIPCC_FLAGS = [

@@ -85,6 +85,7 @@ struct VolDesc {
     const double* field;         // f64 input (device)
     const uint8_t* mask;         // u8 mask (device)
     double* out;                 // f64 output (device)
+    float* out32;                // f32 output in its place (host entry points), or null
     uint8_t* mask_out;           // u8 mask output (device, V-SHARP)
     // V-SHARP state
     float* vs_local;             // selected high-passed field (N)

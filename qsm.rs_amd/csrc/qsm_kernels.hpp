@@ -2722,6 +2722,11 @@ __global__ __launch_bounds__(kThreads, eg_waves(EG, 4)) void k_c2r_vs_out(const 
     const int total = RB * nx;
     const QSM_GLOBAL uint8_t* fin = glb(V.vs_final);
     QSM_GLOBAL double* out = glb(V.out);
+    QSM_GLOBAL float* out32 = glb(V.out32);
+    auto put = [&](size_t idx, float v) {
+        if (V.out32) out32[idx] = v;
+        else out[idx] = (double)v;
+    };
     QSM_GLOBAL uint8_t* mout = glb(V.mask_out);
 #pragma unroll
     for (int t = 0; t < EMAX; ++t) {
@@ -2734,13 +2739,13 @@ __global__ __launch_bounds__(kThreads, eg_waves(EG, 4)) void k_c2r_vs_out(const 
             if (ra < nrows) {
                 const size_t idx = i + (size_t)ra * nx;
                 const uint8_t fm = fin[idx];
-                out[idx] = fm == 1 ? (double)z.x : 0.0;
+                put(idx, fm == 1 ? z.x : 0.0f);
                 mout[idx] = fm;
             }
             if (rb < nrows) {
                 const size_t idx = i + (size_t)rb * nx;
                 const uint8_t fm = fin[idx];
-                out[idx] = fm == 1 ? (double)z.y : 0.0;
+                put(idx, fm == 1 ? z.y : 0.0f);
                 mout[idx] = fm;
             }
         }

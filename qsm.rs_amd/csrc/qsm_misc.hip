@@ -155,8 +155,12 @@ __global__ __launch_bounds__(kThreads) void k_tv_output(const VolDesc* __restric
     const size_t N = (size_t)V.nx * V.ny * V.nz;
     const float* x = V.x[status[gv].iters & 1];
     const size_t end = (size_t)(lb + 1) * kThreads * 4;
-    for (size_t i = (size_t)lb * kThreads * 4 + threadIdx.x; i < N && i < end; i += kThreads)
-        V.out[i] = V.mask[i] ? (double)x[i] : 0.0;
+    float* const o32 = V.out32;
+    for (size_t i = (size_t)lb * kThreads * 4 + threadIdx.x; i < N && i < end; i += kThreads) {
+        const float v = V.mask[i] ? x[i] : 0.0f;
+        if (o32) o32[i] = v;
+        else V.out[i] = (double)v;
+    }
 }
 
 __global__ __launch_bounds__(kThreads) void k_vs_init(const VolDesc* __restrict__ vols, LaunchTable lt) {

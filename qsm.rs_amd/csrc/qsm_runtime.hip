@@ -4,6 +4,7 @@
 #include "qsm_internal.hpp"
 #include "fft_dense.hpp"
 #include "fft_chirp.hpp"
+#include "qsm_hostmem.hpp"
 #include "../../include/qsm_gpu.h"
 
 #include <algorithm>
@@ -108,43 +109,50 @@ inline float2 twiddle_entry(int q, int n) {
     return make_float2((float)cosl(a), (float)sinl(a));
 }
 
+// The FFT tables of a length, formed in long double once per process (60 us
+// for a 192x192x128 volume, 10 ms for a chirp-z filter of 1024) and kept:
+// there are at most kMaxLen lengths, and kMaxDenseRadix dense radices.
+// Kinds: 0 the twiddles of length n, 1 a dense radix's coefficients, 2 the
+// chirp of length n and then its filter.
+const std::vector<float2>& fft_table(int kind, int n) {
+    static std::mutex mu;
+    static std::map<std::pair<int, int>, std::vector<float2>> tab;
+    std::lock_guard<std::mutex> lk(mu);
+    std::vector<float2>& t = tab[{kind, n}];  // (references stay valid as the map grows)
+    if (t.empty()) {
+        if (kind == 0) {
+            for (int q = 0; q < n; ++q) t.push_back(twiddle_entry(q, n));
+        } else if (kind == 1) {
+            t.resize(qsmfft::dense_table_len(n));
+            qsmfft::dense_table(n, t.data());
+        } else {
+            std::vector<float2> f;
+            chirp_tables(n, chirp_length(n), t, f);
+            t.insert(t.end(), f.begin(), f.end());
+        }
+    }
+    return t;
+}
+
+// The tables of the lengths of a set of volumes, end to end.
 struct TwiddleBank {
     std::vector<float2> host;
-    std::map<int, int> off, chirp_off, filt_off, dense_off;
-    int add(int n) {
-        auto it = off.find(n);
+    std::map<std::pair<int, int>, int> off;
+    int put(int kind, int n) {
+        auto it = off.find({kind, n});
         if (it != off.end()) return it->second;
-        int o = (int)host.size();
-        for (int q = 0; q < n; ++q) host.push_back(twiddle_entry(q, n));
-        off[n] = o;
-        return o;
-    }
-    // coefficient table of a dense radix
-    int add_dense(int R) {
-        auto it = dense_off.find(R);
-        if (it != dense_off.end()) return it->second;
         const int o = (int)host.size();
-        host.resize(o + qsmfft::dense_table_len(R));
-        qsmfft::dense_table(R, host.data() + o);
-        dense_off[R] = o;
+        const std::vector<float2>& t = fft_table(kind, n);
+        host.insert(host.end(), t.begin(), t.end());
+        off[{kind, n}] = o;
         return o;
     }
+    int add(int n) { return put(0, n); }
+    int add_dense(int R) { return put(1, R); }
     // chirp (n entries) and filter (M entries) offsets of length n
-    void add_chirp(int n, int M, int& oc, int& of) {
-        auto it = chirp_off.find(n);
-        if (it != chirp_off.end()) {
-            oc = it->second;
-            of = filt_off[n];
-            return;
-        }
-        std::vector<float2> c, f;
-        chirp_tables(n, M, c, f);
-        oc = (int)host.size();
-        host.insert(host.end(), c.begin(), c.end());
-        of = (int)host.size();
-        host.insert(host.end(), f.begin(), f.end());
-        chirp_off[n] = oc;
-        filt_off[n] = of;
+    void add_chirp(int n, int& oc, int& of) {
+        oc = put(2, n);
+        of = oc + n;
     }
 };
 
@@ -167,17 +175,36 @@ qsmfft::Plan make_plan(int n, TwiddleBank& tb) {
     qsmfft::make_plan_stages(M, p);
     p.tw_off = tb.add(M);
     p.bl_n = n;
-    tb.add_chirp(n, M, p.bl_chirp, p.bl_filt);
+    tb.add_chirp(n, p.bl_chirp, p.bl_filt);
     return p;
 }
 
 template <class T>
 int dev_alloc(T** p, size_t count) {
     if (count == 0) count = 1;
-    hipError_t e = hipMalloc((void**)p, count * sizeof(T));
+    hipError_t e = workspace_alloc((void**)p, count * sizeof(T));
     if (e != hipSuccess)
         return fail(e == hipErrorOutOfMemory ? QSM_ENOMEM : QSM_EHIP, "hipMalloc(%zu bytes): %s",
                     count * sizeof(T), hipGetErrorString(e));
+    return QSM_OK;
+}
+
+// Volume descriptors and FFT tables in one block, uploaded by one copy on the
+// null stream (which, as ever, waits for work the caller left there).
+int upload_plan(const VolDesc* vols, size_t n_vols, const TwiddleBank& tb, void** block, VolDesc** d_vols,
+                float2** d_tw) {
+    const size_t head = (n_vols * sizeof(VolDesc) + 255) / 256 * 256, tw = tb.host.size() * sizeof(float2);
+    std::vector<unsigned char> host(head + tw);
+    std::memcpy(host.data(), vols, n_vols * sizeof(VolDesc));
+    if (tw) std::memcpy(host.data() + head, tb.host.data(), tw);
+    unsigned char* d = nullptr;
+    const int rc = dev_alloc(&d, host.size());
+    if (rc) return rc;
+    *block = d;
+    *d_vols = reinterpret_cast<VolDesc*>(d);
+    *d_tw = reinterpret_cast<float2*>(d + head);
+    const hipError_t e = hipMemcpy(d, host.data(), host.size(), hipMemcpyHostToDevice);
+    if (e != hipSuccess) return fail(QSM_EHIP, "hipMemcpy of plan tables: %s", hipGetErrorString(e));
     return QSM_OK;
 }
 
@@ -356,6 +383,9 @@ struct qsm_tv_batch {
     // other t (a negative lambda, say) the recording kernel, which forms
     // shrink itself, runs in its place with a scratch record.
     bool plain_shrink = false;
+    bool field32 = false;  // the field is VolDesc::vs_local, in f32 (host entry points)
+    void* host_out = nullptr;  // their result array, made ready while the device works
+    size_t host_bytes = 0;
     qsm_tv_params params{};
     std::vector<VolDesc> h;
     VolDesc* d_vols = nullptr;
@@ -405,18 +435,18 @@ static void batch_free(qsm_tv_batch* b) {
         if (g) (void)hipGraphExecDestroy(g);
     for (auto& st : b->side)
         if (st) (void)hipStreamSynchronize(st);
-    for (void* p : b->allocs) (void)hipFree(p);
+    for (void* p : b->allocs) workspace_free(p);
     for (auto& e : b->ev_fork)
         if (e) (void)hipEventDestroy(e);
     for (auto& row : b->ev_join)
         for (auto& e : row)
             if (e) (void)hipEventDestroy(e);
     for (auto& st : b->side)
-        if (st) (void)hipStreamDestroy(st);
-    if (b->h_status) (void)hipHostFree(b->h_status);
+        stream_give(st);
+    pinned_give(b->h_status);
     for (auto& e : b->ev)
         if (e) (void)hipEventDestroy(e);
-    if (b->own_stream && b->stream) (void)hipStreamDestroy(b->stream);
+    if (b->own_stream && b->stream) stream_give(b->stream);
     delete b;
 }
 
@@ -491,8 +521,18 @@ static int tune_column_schedules(qsm_tv_batch* B) {
 
 // rts != null selects RTS: its rho, tol, max_iter replace params' (params
 // may then be null).
+// io: the host entry points' one volume, whose field and output are f32 on the
+// device (the volume's own d_field and d_chi are then null).
+struct HostVolume {
+    float* field = nullptr;
+    float* chi = nullptr;
+    uint8_t* mask = nullptr;
+    double* out = nullptr;  // the caller's result array of n values
+    size_t n = 0;
+};
 static int tv_batch_create_impl(const qsm_tv_volume* vols, size_t n_vols, const qsm_tv_params* params_in,
-                                void* stream, qsm_tv_batch** out, const qsm_rts_params* rts = nullptr) {
+                                void* stream, qsm_tv_batch** out, const qsm_rts_params* rts = nullptr,
+                                const HostVolume* io = nullptr) {
     qsm_tv_params rts_as_tv{};
     if (rts) {
         if (!(rts->rho > 0) || std::isnan(rts->delta) || std::isnan(rts->mu))
@@ -512,7 +552,7 @@ static int tv_batch_create_impl(const qsm_tv_volume* vols, size_t n_vols, const 
     for (size_t v = 0; v < n_vols; ++v) {
         int rc = validate_grid(&vols[v].grid);
         if (rc) return rc;
-        if (!vols[v].d_field || !vols[v].d_mask || !vols[v].d_chi)
+        if (!io && (!vols[v].d_field || !vols[v].d_mask || !vols[v].d_chi))
             return fail(QSM_EPARAM, "volume %zu has a null device pointer", v);
         const double* b = vols[v].bdir;
         double bn = std::sqrt(b[0] * b[0] + b[1] * b[1] + b[2] * b[2]);
@@ -562,6 +602,12 @@ static int tv_batch_create_impl(const qsm_tv_volume* vols, size_t n_vols, const 
         V.field = vols[v].d_field;
         V.mask = vols[v].d_mask;
         V.out = vols[v].d_chi;
+        if (io) {
+            V.vs_local = io->field;
+            V.mask = io->mask;
+            V.out32 = io->chi;
+            B->field32 = true;
+        }
         lx.push_back(V.nx); bx.push_back(pb.xpass); bc.push_back(pb.cpass);
         ly.push_back(V.ny); by.push_back(pb.ypass);
         lz.push_back(V.nz); bz.push_back(pb.zpass);
@@ -602,15 +648,11 @@ static int tv_batch_create_impl(const qsm_tv_volume* vols, size_t n_vols, const 
     B->gz = make_groups(lz, bz, true);
     B->lt_out = identity_table(bo);
     int rc;
-    if ((rc = dev_alloc(&B->d_tw, tb.host.size()))) return cleanup(rc);
-    B->allocs.push_back(B->d_tw);
-    if ((rc = dev_alloc(&B->d_vols, n_vols))) return cleanup(rc);
-    B->allocs.push_back(B->d_vols);
     if ((rc = dev_alloc(&B->d_status, n_vols))) return cleanup(rc);
     B->allocs.push_back(B->d_status);
     {
-        hipError_t e = hipHostMalloc((void**)&B->h_status, n_vols * sizeof(VolStatus),
-                                     hipHostMallocMapped | hipHostMallocCoherent);
+        static_assert(kMaxVolumes * sizeof(VolStatus) <= kPinnedBlock, "status mirror block");
+        hipError_t e = pinned_take((void**)&B->h_status);
         if (e != hipSuccess) { B->h_status = nullptr; return cleanup(fail(QSM_EHIP, "hipHostMalloc: %s", hipGetErrorString(e))); }
         e = hipHostGetDevicePointer((void**)&B->h_status_dev, B->h_status, 0);
         if (e != hipSuccess) return cleanup(fail(QSM_EHIP, "hipHostGetDevicePointer: %s", hipGetErrorString(e)));
@@ -619,7 +661,7 @@ static int tv_batch_create_impl(const qsm_tv_volume* vols, size_t n_vols, const 
     if (stream) {
         B->stream = (hipStream_t)stream;
     } else {
-        hipError_t e = hipStreamCreateWithFlags(&B->stream, hipStreamNonBlocking);
+        hipError_t e = stream_take(&B->stream);
         if (e != hipSuccess) { B->stream = nullptr; return cleanup(fail(QSM_EHIP, "hipStreamCreate: %s", hipGetErrorString(e))); }
         B->own_stream = true;
     }
@@ -627,18 +669,19 @@ static int tv_batch_create_impl(const qsm_tv_volume* vols, size_t n_vols, const 
         hipError_t he = hipEventCreateWithFlags(&e, hipEventDisableTiming);
         if (he != hipSuccess) { e = nullptr; return cleanup(fail(QSM_EHIP, "hipEventCreate: %s", hipGetErrorString(he))); }
     }
-    hipError_t e1 = hipMemcpy(B->d_tw, tb.host.data(), tb.host.size() * sizeof(float2), hipMemcpyHostToDevice);
-    hipError_t e2 = hipMemcpy(B->d_vols, B->h.data(), n_vols * sizeof(VolDesc), hipMemcpyHostToDevice);
-    if (e1 != hipSuccess || e2 != hipSuccess)
-        return cleanup(fail(QSM_EHIP, "hipMemcpy of plan tables: %s",
-                            hipGetErrorString(e1 != hipSuccess ? e1 : e2)));
+    {
+        void* block = nullptr;
+        rc = upload_plan(B->h.data(), n_vols, tb, &block, &B->d_vols, &B->d_tw);
+        if (block) B->allocs.push_back(block);
+        if (rc) return cleanup(rc);
+    }
     {
         int rc = tune_column_schedules(B);
         if (rc) return cleanup(rc);
     }
     if (B->gx.size() > 1 || B->gy.size() > 1 || B->gz.size() > 1 || B->gxc.size() > 1) {
         for (auto& st : B->side) {
-            hipError_t e = hipStreamCreateWithFlags(&st, hipStreamNonBlocking);
+            hipError_t e = stream_take(&st);
             if (e != hipSuccess) { st = nullptr; return cleanup(fail(QSM_EHIP, "hipStreamCreate: %s", hipGetErrorString(e))); }
         }
         auto mk = [&](hipEvent_t& ev) {
@@ -729,7 +772,7 @@ static int enqueue_setup(qsm_tv_batch* B) {
         for (auto& V : B->h) launch_fill_zero(st, V.u[0], 3 * (size_t)V.nx * V.ny * V.nz);
         launch_status_reset(st, B->d_status, B->nvol);
         PassArgs a = B->args(nullptr);
-        run_groups(P_R2C_F64, B->gx, a);
+        run_groups(B->field32 ? P_R2C_F32 : P_R2C_F64, B->gx, a);
         run_groups(P_Y_FWD, B->gy, a);
         run_groups(P_Z_FILTER, B->gz, a);
         run_groups(P_Y_INV, B->gy, a);
@@ -747,7 +790,7 @@ static int enqueue_setup(qsm_tv_batch* B) {
     }
     launch_status_reset(st, B->d_status, B->nvol);
     PassArgs a = B->args(nullptr);
-    run_groups(P_R2C_F64, B->gx, a);
+    run_groups(B->field32 ? P_R2C_F32 : P_R2C_F64, B->gx, a);
     run_groups(P_Y_FWD, B->gy, a);
     run_groups(P_Z_TV_SETUP, B->gz, a);
     QSM_CHECK_LAUNCH();
@@ -823,6 +866,7 @@ static int tv_batch_run_impl(qsm_tv_batch* B, qsm_progress_fn progress, void* us
             int rc = launch_iteration(B, it, nullptr);
             if (rc) return rc;
         }
+        prefault(B->host_out, B->host_bytes);
         if (max_iter > 0) launch_tv_reduce(st, B->d_vols, B->nvol, B->d_status, B->h_status_dev);
     } else {
         // Iteration j is closed by the first pass of iteration j+1 (or by
@@ -838,6 +882,7 @@ static int tv_batch_run_impl(qsm_tv_batch* B, qsm_progress_fn progress, void* us
                 if (rc) return rc;
                 ++next;
             }
+            if (it == 1) prefault(B->host_out, B->host_bytes);
             if (it == max_iter) {
                 launch_tv_reduce(st, B->d_vols, B->nvol, B->d_status, B->h_status_dev);
                 QSM_HIP(hipEventRecord(B->ev[it % W], st));
@@ -862,7 +907,32 @@ static int tv_batch_run_impl(qsm_tv_batch* B, qsm_progress_fn progress, void* us
     return QSM_OK;
 }
 
-
+// The one volume of a host entry point: workspaces, and the field (in f32, the
+// precision of the first pass) and mask uploaded.
+static int host_volume_upload(HostVolume& hv, const double* field, const uint8_t* mask, size_t N) {
+    int rc;
+    if ((rc = dev_alloc(&hv.field, N)) || (rc = dev_alloc(&hv.chi, N)) || (rc = dev_alloc(&hv.mask, N))) return rc;
+    hipError_t e = copy_to_device_f32(hv.field, field, N);
+    if (e == hipSuccess) e = copy_to_device(hv.mask, mask, N);
+    if (e != hipSuccess) return fail(QSM_EHIP, "hipMemcpy H2D: %s", hipGetErrorString(e));
+    return QSM_OK;
+}
+static int host_volume_download(const HostVolume& hv, double* chi_out, size_t N) {
+    const hipError_t e = copy_to_host_f32(chi_out, hv.chi, N);
+    if (e != hipSuccess) return fail(QSM_EHIP, "hipMemcpy D2H: %s", hipGetErrorString(e));
+    return QSM_OK;
+}
+static void host_volume_free(HostVolume& hv) {
+    workspace_free(hv.field);
+    workspace_free(hv.chi);
+    workspace_free(hv.mask);
+}
+static qsm_tv_volume host_volume(const qsm_grid* grid, const double bdir[3]) {
+    qsm_tv_volume vol{};
+    vol.grid = *grid;
+    for (int a = 0; a < 3; ++a) vol.bdir[a] = bdir[a];
+    return vol;
+}
 
 // Event-timed copy of the iteration loop: every kernel of `iters` iterations
 // is bracketed by HIP events on the batch's stream; ms_out[k] receives the
@@ -930,7 +1000,7 @@ static void unrolled_free(qsm_tv_unrolled* U) {
         if (U->B->stream) (void)hipStreamSynchronize(U->B->stream);
         batch_free(U->B);
     }
-    for (void* p : U->allocs) (void)hipFree(p);
+    for (void* p : U->allocs) workspace_free(p);
     delete U;
 }
 
@@ -1057,7 +1127,7 @@ static int unrolled_backward_impl(qsm_tv_unrolled* U, const double* const* d_chi
 // The five passes of one spectral round trip of a single volume: R2C of
 // src_kind, y, z pass zkind, inverse y, C2R to f64 (masked for filters).
 // Launch tables live on the stack.
-static void enqueue_round_trip(int src_kind, int zkind, const VolDesc& V, const PassBlocks& pb,
+static void enqueue_round_trip(int src_kind, int zkind, int out_kind, const VolDesc& V, const PassBlocks& pb,
                                const VolDesc* d_vols, const float2* d_tw, hipStream_t st) {
     auto table = [](int blocks) {
         LaunchTable lt{};
@@ -1084,15 +1154,15 @@ static void enqueue_round_trip(int src_kind, int zkind, const VolDesc& V, const 
     run(P_Y_FWD, V.ny, true, ty);
     run(zkind, V.nz, true, tz);
     run(P_Y_INV, V.ny, true, ty);
-    run(zkind == P_Z_FILTER ? P_C2R_F64_MASKED : P_C2R_F64OUT, V.nx, false, txc);
+    run(out_kind, V.nx, false, txc);
 }
 
 static int spectral_apply(int zkind, int filt, double fa, const double* d_in, const uint8_t* d_mask,
                           const qsm_grid* grid, const double bdir_in[3], double* d_out, void* stream,
-                          int src_kind = P_R2C_F64) {
+                          int src_kind = P_R2C_F64, const HostVolume* hv = nullptr) {
     static const double z_axis[3] = {0.0, 0.0, 1.0};
     const double* bdir = bdir_in ? bdir_in : z_axis;
-    if (!d_in || !grid || !d_out || (zkind == P_Z_FILTER && !d_mask))
+    if (!hv && (!d_in || !grid || !d_out || (zkind == P_Z_FILTER && !d_mask)))
         return fail(QSM_EPARAM, "null argument");
     int rc = validate_grid(grid);
     if (rc) return rc;
@@ -1107,6 +1177,11 @@ static int spectral_apply(int zkind, int filt, double fa, const double* d_in, co
     V.adj_out = d_out;
     V.out = d_out;
     V.mask = d_mask;
+    if (hv) {
+        V.vs_local = hv->field;
+        V.mask = hv->mask;
+        V.x[0] = hv->chi;
+    }
     V.filt = filt;
     V.filt_a = fa;
     const size_t Nh = (size_t)V.nxh * V.ny * V.nz;
@@ -1117,28 +1192,28 @@ static int spectral_apply(int zkind, int filt, double fa, const double* d_in, co
     bool own = false;
     auto done = [&](int code) {
         if (st) (void)hipStreamSynchronize(st);
-        for (void* p : allocs) (void)hipFree(p);
-        if (own && st) (void)hipStreamDestroy(st);
+        for (void* p : allocs) workspace_free(p);
+        if (own) stream_give(st);
         return code;
     };
     if ((rc = dev_alloc(&V.spec[SPEC_WORK], Nh))) return done(rc);
     allocs.push_back(V.spec[SPEC_WORK]);
-    if ((rc = dev_alloc(&d_tw, tb.host.size()))) return done(rc);
-    allocs.push_back(d_tw);
-    if ((rc = dev_alloc(&d_vols, 1))) return done(rc);
-    allocs.push_back(d_vols);
+    {
+        void* block = nullptr;
+        rc = upload_plan(&V, 1, tb, &block, &d_vols, &d_tw);
+        if (block) allocs.push_back(block);
+        if (rc) return done(rc);
+    }
     if (!st) {
-        hipError_t e = hipStreamCreateWithFlags(&st, hipStreamNonBlocking);
+        hipError_t e = stream_take(&st);
         if (e != hipSuccess) { st = nullptr; return done(fail(QSM_EHIP, "hipStreamCreate: %s", hipGetErrorString(e))); }
         own = true;
     }
-    hipError_t e1 = hipMemcpy(d_tw, tb.host.data(), tb.host.size() * sizeof(float2), hipMemcpyHostToDevice);
-    hipError_t e2 = hipMemcpy(d_vols, &V, sizeof V, hipMemcpyHostToDevice);
-    if (e1 != hipSuccess || e2 != hipSuccess)
-        return done(fail(QSM_EHIP, "hipMemcpy of plan tables: %s", hipGetErrorString(e1 != hipSuccess ? e1 : e2)));
-    enqueue_round_trip(src_kind, zkind, V, pb, d_vols, d_tw, st);
+    enqueue_round_trip(src_kind, zkind, hv ? P_C2R_X0 : (zkind == P_Z_FILTER ? P_C2R_F64_MASKED : P_C2R_F64OUT), V,
+                       pb, d_vols, d_tw, st);
     hipError_t le = hipGetLastError();
     if (le != hipSuccess) return done(fail(QSM_EHIP, "kernel launch: %s", hipGetErrorString(le)));
+    if (hv) prefault(hv->out, hv->n * sizeof(double));
     hipError_t se = hipStreamSynchronize(st);
     if (se != hipSuccess) return done(fail(QSM_EHIP, "hipStreamSynchronize: %s", hipGetErrorString(se)));
     return done(QSM_OK);
@@ -1183,6 +1258,9 @@ struct qsm_vsharp_batch {
     std::vector<double> radii;  // processing order (descending)
     double threshold = 0.05;
     bool sharp = false;         // one radius: sharp_core semantics
+    bool field32 = false;       // the field is in VolDesc::vs_local, in f32, until that is cleared (host entry point)
+    void* host_out = nullptr;   // its result array, made ready while the device works
+    size_t host_bytes = 0;
     Groups gx, grows, gy, gy2, gz;   // passes grouped by axis length
     LaunchTable lt_init{};
     std::vector<void*> allocs;
@@ -1203,13 +1281,14 @@ struct qsm_vsharp_batch {
 static void vs_free(qsm_vsharp_batch* b) {
     if (!b) return;
     if (b->stream) (void)hipStreamSynchronize(b->stream);
-    for (void* p : b->allocs) (void)hipFree(p);
-    if (b->own_stream && b->stream) (void)hipStreamDestroy(b->stream);
+    for (void* p : b->allocs) workspace_free(p);
+    if (b->own_stream && b->stream) stream_give(b->stream);
     delete b;
 }
 
 static int vs_create_impl(const qsm_vsharp_volume* vols, size_t n_vols, const double* radii,
-                          size_t n_radii, double threshold, void* stream, qsm_vsharp_batch** out) {
+                          size_t n_radii, double threshold, void* stream, qsm_vsharp_batch** out,
+                          const HostVolume* io = nullptr) {
     if (!vols || !out || (n_radii && !radii)) return fail(QSM_EPARAM, "null argument");
     if (n_vols == 0 || n_vols > (size_t)kMaxVolumes)
         return fail(QSM_EPARAM, "batch size %zu outside 1..%d", n_vols, kMaxVolumes);
@@ -1219,7 +1298,7 @@ static int vs_create_impl(const qsm_vsharp_volume* vols, size_t n_vols, const do
     for (size_t v = 0; v < n_vols; ++v) {
         int rc = validate_grid(&vols[v].grid);
         if (rc) return rc;
-        if (!vols[v].d_field || !vols[v].d_mask || !vols[v].d_local || !vols[v].d_mask_out)
+        if (!io && (!vols[v].d_field || !vols[v].d_mask || !vols[v].d_local || !vols[v].d_mask_out))
             return fail(QSM_EPARAM, "volume %zu has a null device pointer", v);
     }
     qsm_vsharp_batch* B = new qsm_vsharp_batch();
@@ -1247,6 +1326,11 @@ static int vs_create_impl(const qsm_vsharp_volume* vols, size_t n_vols, const do
         V.mask = vols[v].d_mask;
         V.out = vols[v].d_local;
         V.mask_out = vols[v].d_mask_out;
+        if (io) {
+            V.mask = io->mask;
+            V.out32 = io->chi;
+            B->field32 = true;
+        }
         V.vs_threshold = threshold;
         V.vs_radii = B->d_radii;
         V.vs_counts = B->d_radii + (size_t)R * (1 + v);
@@ -1277,22 +1361,21 @@ static int vs_create_impl(const qsm_vsharp_volume* vols, size_t n_vols, const do
     B->gy2 = make_groups(ly, by2, true);
     B->gz = make_groups(lz, bz, true);
     B->lt_init = identity_table(bi);
-    if ((rc = dev_alloc(&B->d_tw, tb.host.size()))) return cleanup(rc);
-    B->allocs.push_back(B->d_tw);
-    if ((rc = dev_alloc(&B->d_vols, n_vols))) return cleanup(rc);
-    B->allocs.push_back(B->d_vols);
+    {
+        void* block = nullptr;
+        rc = upload_plan(B->h.data(), n_vols, tb, &block, &B->d_vols, &B->d_tw);
+        if (block) B->allocs.push_back(block);
+        if (rc) return cleanup(rc);
+    }
     if (stream) {
         B->stream = (hipStream_t)stream;
     } else {
-        hipError_t e = hipStreamCreateWithFlags(&B->stream, hipStreamNonBlocking);
+        hipError_t e = stream_take(&B->stream);
         if (e != hipSuccess) { B->stream = nullptr; return cleanup(fail(QSM_EHIP, "hipStreamCreate: %s", hipGetErrorString(e))); }
         B->own_stream = true;
     }
-    hipError_t e1 = hipMemcpy(B->d_tw, tb.host.data(), tb.host.size() * sizeof(float2), hipMemcpyHostToDevice);
-    hipError_t e2 = hipMemcpy(B->d_vols, B->h.data(), n_vols * sizeof(VolDesc), hipMemcpyHostToDevice);
     hipError_t e3 = hipMemcpy(B->d_radii, host_tab.data(), host_tab.size() * sizeof(double), hipMemcpyHostToDevice);
-    if (e1 != hipSuccess || e2 != hipSuccess || e3 != hipSuccess)
-        return cleanup(fail(QSM_EHIP, "hipMemcpy of plan tables failed"));
+    if (e3 != hipSuccess) return cleanup(fail(QSM_EHIP, "hipMemcpy of plan tables failed"));
     *out = B;
     return QSM_OK;
 }
@@ -1305,7 +1388,7 @@ static int vs_run_impl(qsm_vsharp_batch* B, qsm_progress_fn progress, void* user
     // F^ = FFT(field) (vsharp.rs:117-122), M^ = FFT(mask) once for all radii
     PassArgs a = B->args();
     a.sel = SPEC_A;
-    run_groups(P_R2C_F64, B->gx, a);
+    run_groups(B->field32 ? P_R2C_F32 : P_R2C_F64, B->gx, a);
     run_groups(P_Y_FWD, B->gy, a);
     run_groups(P_Z_VS_FWD, B->gz, a);
     a.sel = SPEC_B;
@@ -1343,6 +1426,7 @@ static int vs_run_impl(qsm_vsharp_batch* B, qsm_progress_fn progress, void* user
     run_groups(P_Y_INV, B->gy, a);
     run_groups(P_C2R_VS_OUT, B->gx, a);
     QSM_CHECK_LAUNCH();
+    prefault(B->host_out, B->host_bytes);
     QSM_HIP(hipStreamSynchronize(st));
     return QSM_OK;
 }
@@ -1361,30 +1445,28 @@ static int vsharp_host(const double* field, const uint8_t* mask, const qsm_grid*
         std::memcpy(mask_out, mask, N);
         return QSM_OK;
     }
-    double *d_f = nullptr, *d_l = nullptr;
-    uint8_t *d_m = nullptr, *d_mo = nullptr;
+    HostVolume hv;
+    uint8_t* d_mo = nullptr;
     qsm_vsharp_batch* B = nullptr;
     auto done = [&](int code) {
         if (B) vs_free(B);
-        if (d_f) (void)hipFree(d_f);
-        if (d_l) (void)hipFree(d_l);
-        if (d_m) (void)hipFree(d_m);
-        if (d_mo) (void)hipFree(d_mo);
+        host_volume_free(hv);
+        workspace_free(d_mo);
         return code;
     };
-    if ((rc = dev_alloc(&d_f, N)) || (rc = dev_alloc(&d_l, N)) || (rc = dev_alloc(&d_m, N)) ||
-        (rc = dev_alloc(&d_mo, N)))
-        return done(rc);
-    hipError_t e = hipMemcpy(d_f, field, N * sizeof(double), hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = hipMemcpy(d_m, mask, N, hipMemcpyHostToDevice);
-    if (e != hipSuccess) return done(fail(QSM_EHIP, "hipMemcpy H2D: %s", hipGetErrorString(e)));
-    qsm_vsharp_volume vol;
+    if ((rc = dev_alloc(&hv.chi, N)) || (rc = dev_alloc(&hv.mask, N)) || (rc = dev_alloc(&d_mo, N))) return done(rc);
+    qsm_vsharp_volume vol{};
     vol.grid = *grid;
-    vol.d_field = d_f; vol.d_mask = d_m; vol.d_local = d_l; vol.d_mask_out = d_mo;
-    if ((rc = vs_create_impl(&vol, 1, radii, n_radii, threshold, nullptr, &B))) return done(rc);
+    vol.d_mask_out = d_mo;
+    if ((rc = vs_create_impl(&vol, 1, radii, n_radii, threshold, nullptr, &B, &hv))) return done(rc);
+    B->host_out = local_out;
+    B->host_bytes = N * sizeof(double);
+    hipError_t e = copy_to_device_f32(B->h[0].vs_local, field, N);
+    if (e == hipSuccess) e = copy_to_device(hv.mask, mask, N);
+    if (e != hipSuccess) return done(fail(QSM_EHIP, "hipMemcpy H2D: %s", hipGetErrorString(e)));
     if ((rc = vs_run_impl(B, progress, user))) return done(rc);
-    e = hipMemcpy(local_out, d_l, N * sizeof(double), hipMemcpyDeviceToHost);
-    if (e == hipSuccess) e = hipMemcpy(mask_out, d_mo, N, hipMemcpyDeviceToHost);
+    if ((rc = host_volume_download(hv, local_out, N))) return done(rc);
+    e = copy_to_host(mask_out, d_mo, N);
     if (e != hipSuccess) return done(fail(QSM_EHIP, "hipMemcpy D2H: %s", hipGetErrorString(e)));
     return done(QSM_OK);
 }
@@ -1521,29 +1603,21 @@ int qsm_tv_admm_ex(const double* local_field, const uint8_t* mask, const qsm_gri
     int rc = validate_grid(grid);
     if (rc) return rc;
     const size_t N = grid->nx * grid->ny * grid->nz;
-    double *d_f = nullptr, *d_chi = nullptr;
-    uint8_t* d_m = nullptr;
+    HostVolume hv;
     qsm_tv_batch* B = nullptr;
     auto done = [&](int code) {
         if (B) batch_free(B);
-        if (d_f) (void)hipFree(d_f);
-        if (d_chi) (void)hipFree(d_chi);
-        if (d_m) (void)hipFree(d_m);
+        host_volume_free(hv);
         return code;
     };
-    if ((rc = dev_alloc(&d_f, N)) || (rc = dev_alloc(&d_chi, N)) || (rc = dev_alloc(&d_m, N)))
-        return done(rc);
-    hipError_t e = hipMemcpy(d_f, local_field, N * sizeof(double), hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = hipMemcpy(d_m, mask, N, hipMemcpyHostToDevice);
-    if (e != hipSuccess) return done(fail(QSM_EHIP, "hipMemcpy H2D: %s", hipGetErrorString(e)));
-    qsm_tv_volume vol;
-    vol.grid = *grid;
-    vol.bdir[0] = bdir[0]; vol.bdir[1] = bdir[1]; vol.bdir[2] = bdir[2];
-    vol.d_field = d_f; vol.d_mask = d_m; vol.d_chi = d_chi;
-    if ((rc = tv_batch_create_impl(&vol, 1, params, nullptr, &B))) return done(rc);
+    if ((rc = host_volume_upload(hv, local_field, mask, N))) return done(rc);
+    const qsm_tv_volume vol = host_volume(grid, bdir);
+    if ((rc = tv_batch_create_impl(&vol, 1, params, nullptr, &B, nullptr, &hv))) return done(rc);
+    B->graph_state = -1;  // run once: capturing the graphs costs more than they save
+    B->host_out = chi_out;
+    B->host_bytes = N * sizeof(double);
     if ((rc = tv_batch_run_impl(B, progress, user))) return done(rc);
-    e = hipMemcpy(chi_out, d_chi, N * sizeof(double), hipMemcpyDeviceToHost);
-    if (e != hipSuccess) return done(fail(QSM_EHIP, "hipMemcpy D2H: %s", hipGetErrorString(e)));
+    if ((rc = host_volume_download(hv, chi_out, N))) return done(rc);
     if (iters_out || rel_out) {
         size_t it = 0;
         double rel = 0;
@@ -1685,7 +1759,7 @@ int qsm_dipole_forward_noalloc(const double* d_chi, const qsm_grid* grid, const 
     // The R2C pass writes the whole spectrum, so nothing needs clearing.
     QSM_HIP(hipMemcpyAsync(d_vols, &V, sizeof V, hipMemcpyHostToDevice, st));
     QSM_HIP(hipMemcpyAsync(d_tw, tb.host.data(), tb.host.size() * sizeof(float2), hipMemcpyHostToDevice, st));
-    enqueue_round_trip(P_R2C_F64, P_Z_DIPOLE, V, pb, d_vols, d_tw, st);
+    enqueue_round_trip(P_R2C_F64, P_Z_DIPOLE, P_C2R_F64OUT, V, pb, d_vols, d_tw, st);
     QSM_CHECK_LAUNCH();
     // the host-side tables above live on this stack frame: wait before returning
     QSM_HIP(hipStreamSynchronize(st));
@@ -1701,22 +1775,30 @@ static int filter_host(int filt, double fa, const double* field, const uint8_t* 
     int rc = validate_grid(grid);
     if (rc) return rc;
     const size_t N = grid->nx * grid->ny * grid->nz;
-    double *d_f = nullptr, *d_o = nullptr;
-    uint8_t* d_m = nullptr;
+    // the wrapped Laplacian takes the phase in f64; every other source is f32 on
+    // the device, and so is the output
+    double* d_f64 = nullptr;
+    HostVolume hv;
     auto done = [&](int code) {
-        if (d_f) (void)hipFree(d_f);
-        if (d_o) (void)hipFree(d_o);
-        if (d_m) (void)hipFree(d_m);
+        workspace_free(d_f64);
+        host_volume_free(hv);
         return code;
     };
-    if ((rc = dev_alloc(&d_f, N)) || (rc = dev_alloc(&d_o, N)) || (rc = dev_alloc(&d_m, N))) return done(rc);
-    hipError_t e = hipMemcpy(d_f, field, N * sizeof(double), hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = hipMemcpy(d_m, mask, N, hipMemcpyHostToDevice);
-    if (e != hipSuccess) return done(fail(QSM_EHIP, "hipMemcpy H2D: %s", hipGetErrorString(e)));
-    if ((rc = spectral_apply(P_Z_FILTER, filt, fa, d_f, d_m, grid, bdir, d_o, nullptr, src_kind)))
+    const bool wrapped = src_kind == P_R2C_WRAPLAP;
+    hv.out = chi_out;
+    hv.n = N;
+    if (wrapped) {
+        if ((rc = dev_alloc(&d_f64, N)) || (rc = dev_alloc(&hv.chi, N)) || (rc = dev_alloc(&hv.mask, N))) return done(rc);
+        hipError_t e = copy_to_device(d_f64, field, N * sizeof(double));
+        if (e == hipSuccess) e = copy_to_device(hv.mask, mask, N);
+        if (e != hipSuccess) return done(fail(QSM_EHIP, "hipMemcpy H2D: %s", hipGetErrorString(e)));
+    } else if ((rc = host_volume_upload(hv, field, mask, N))) {
         return done(rc);
-    e = hipMemcpy(chi_out, d_o, N * sizeof(double), hipMemcpyDeviceToHost);
-    if (e != hipSuccess) return done(fail(QSM_EHIP, "hipMemcpy D2H: %s", hipGetErrorString(e)));
+    }
+    if ((rc = spectral_apply(P_Z_FILTER, filt, fa, d_f64, nullptr, grid, bdir, nullptr, nullptr,
+                             wrapped ? P_R2C_WRAPLAP : P_R2C_F32, &hv)))
+        return done(rc);
+    if ((rc = host_volume_download(hv, chi_out, N))) return done(rc);
     return done(QSM_OK);
 }
 
@@ -1749,33 +1831,23 @@ int qsm_nltv(const double* local_field, const uint8_t* mask, const qsm_grid* gri
     int rc = validate_grid(grid);
     if (rc) return rc;
     const size_t N = grid->nx * grid->ny * grid->nz;
-    double *d_f = nullptr, *d_chi = nullptr;
-    uint8_t* d_m = nullptr;
+    HostVolume hv;
     qsm_tv_batch* B = nullptr;
     std::vector<void*> extra;
     auto done = [&](int code) {
         if (B) batch_free(B);
-        for (void* p : extra) (void)hipFree(p);
-        if (d_f) (void)hipFree(d_f);
-        if (d_chi) (void)hipFree(d_chi);
-        if (d_m) (void)hipFree(d_m);
+        for (void* p : extra) workspace_free(p);
+        host_volume_free(hv);
         return code;
     };
-    if ((rc = dev_alloc(&d_f, N)) || (rc = dev_alloc(&d_chi, N)) || (rc = dev_alloc(&d_m, N)))
-        return done(rc);
-    hipError_t e = hipMemcpy(d_f, local_field, N * sizeof(double), hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = hipMemcpy(d_m, mask, N, hipMemcpyHostToDevice);
-    if (e != hipSuccess) return done(fail(QSM_EHIP, "hipMemcpy H2D: %s", hipGetErrorString(e)));
-    qsm_tv_volume vol;
-    vol.grid = *grid;
-    vol.bdir[0] = bdir[0]; vol.bdir[1] = bdir[1]; vol.bdir[2] = bdir[2];
-    vol.d_field = d_f; vol.d_mask = d_m; vol.d_chi = d_chi;
+    if ((rc = host_volume_upload(hv, local_field, mask, N))) return done(rc);
+    const qsm_tv_volume vol = host_volume(grid, bdir);
     qsm_tv_params tp;
     tp.lambda = params->lambda;
     tp.rho = 100.0 * params->lambda;  // src/inversion/nltv.rs:75
     tp.tol = params->tol;
     tp.max_iter = params->max_iter;
-    if ((rc = tv_batch_create_impl(&vol, 1, &tp, nullptr, &B))) return done(rc);
+    if ((rc = tv_batch_create_impl(&vol, 1, &tp, nullptr, &B, nullptr, &hv))) return done(rc);
     VolDesc& V = B->h[0];
     V.filt_b = params->mu;
     const int nb = (int)((N + qsmfft::kThreads * 4 - 1) / (qsmfft::kThreads * 4));
@@ -1834,8 +1906,7 @@ int qsm_nltv(const double* local_field, const uint8_t* mask, const qsm_grid* gri
     launch_tv_output(st, B->d_vols, B->lt_out, B->d_status);
     QSM_CHECK_LAUNCH();
     QSM_HIP(hipStreamSynchronize(st));
-    e = hipMemcpy(chi_out, d_chi, N * sizeof(double), hipMemcpyDeviceToHost);
-    if (e != hipSuccess) return done(fail(QSM_EHIP, "hipMemcpy D2H: %s", hipGetErrorString(e)));
+    if ((rc = host_volume_download(hv, chi_out, N))) return done(rc);
     return done(QSM_OK);
 }
 
@@ -1895,29 +1966,21 @@ int qsm_rts(const double* local_field, const uint8_t* mask, const qsm_grid* grid
     int rc = validate_grid(grid);
     if (rc) return rc;
     const size_t N = grid->nx * grid->ny * grid->nz;
-    double *d_f = nullptr, *d_chi = nullptr;
-    uint8_t* d_m = nullptr;
+    HostVolume hv;
     qsm_tv_batch* B = nullptr;
     auto done = [&](int code) {
         if (B) batch_free(B);
-        if (d_f) (void)hipFree(d_f);
-        if (d_chi) (void)hipFree(d_chi);
-        if (d_m) (void)hipFree(d_m);
+        host_volume_free(hv);
         return code;
     };
-    if ((rc = dev_alloc(&d_f, N)) || (rc = dev_alloc(&d_chi, N)) || (rc = dev_alloc(&d_m, N)))
-        return done(rc);
-    hipError_t e = hipMemcpy(d_f, local_field, N * sizeof(double), hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = hipMemcpy(d_m, mask, N, hipMemcpyHostToDevice);
-    if (e != hipSuccess) return done(fail(QSM_EHIP, "hipMemcpy H2D: %s", hipGetErrorString(e)));
-    qsm_tv_volume vol;
-    vol.grid = *grid;
-    vol.bdir[0] = bdir[0]; vol.bdir[1] = bdir[1]; vol.bdir[2] = bdir[2];
-    vol.d_field = d_f; vol.d_mask = d_m; vol.d_chi = d_chi;
-    if ((rc = tv_batch_create_impl(&vol, 1, nullptr, nullptr, &B, params))) return done(rc);
+    if ((rc = host_volume_upload(hv, local_field, mask, N))) return done(rc);
+    const qsm_tv_volume vol = host_volume(grid, bdir);
+    if ((rc = tv_batch_create_impl(&vol, 1, nullptr, nullptr, &B, params, &hv))) return done(rc);
+    B->graph_state = -1;  // run once: capturing the graphs costs more than they save
+    B->host_out = chi_out;
+    B->host_bytes = N * sizeof(double);
     if ((rc = tv_batch_run_impl(B, progress, user))) return done(rc);
-    e = hipMemcpy(chi_out, d_chi, N * sizeof(double), hipMemcpyDeviceToHost);
-    if (e != hipSuccess) return done(fail(QSM_EHIP, "hipMemcpy D2H: %s", hipGetErrorString(e)));
+    if ((rc = host_volume_download(hv, chi_out, N))) return done(rc);
     return done(QSM_OK);
 }
 
@@ -2096,15 +2159,15 @@ int qsm_hbm_copy_probe(size_t bytes, int reps, double* gbps) {
     float2 *a = nullptr, *b = nullptr;
     int rc;
     if ((rc = dev_alloc(&a, n)) || (rc = dev_alloc(&b, n))) {
-        if (a) (void)hipFree(a);
+        workspace_free(a);
         return rc;
     }
     launch_fill_zero(nullptr, reinterpret_cast<float*>(a), 2 * n);
     double best = 0.0;
     const hipError_t e = best_rate(reps, 2.0 * (double)n * sizeof(float2),
                                    [&] { launch_copy_probe(nullptr, a, b, n); }, best);
-    (void)hipFree(a);
-    (void)hipFree(b);
+    workspace_free(a);
+    workspace_free(b);
     if (e != hipSuccess) return fail(QSM_EHIP, "copy probe: %s", hipGetErrorString(e));
     *gbps = best;
     return QSM_OK;
@@ -2119,15 +2182,15 @@ int qsm_hbm_stream_probe(size_t n, int reads, int writes, int reps, double* gbps
     float *in = nullptr, *out = nullptr;
     int rc;
     if ((rc = dev_alloc(&in, n * reads)) || (rc = dev_alloc(&out, n * writes))) {
-        if (in) (void)hipFree(in);
+        workspace_free(in);
         return rc;
     }
     launch_fill_zero(nullptr, in, n * reads);
     double best = 0.0;
     const hipError_t e = best_rate(reps, 4.0 * (double)n * (reads + writes),
                                    [&] { launch_stream_probe(nullptr, reads, writes, in, out, n); }, best);
-    (void)hipFree(in);
-    (void)hipFree(out);
+    workspace_free(in);
+    workspace_free(out);
     if (e != hipSuccess) return fail(QSM_EHIP, "stream probe: %s", hipGetErrorString(e));
     *gbps = best;
     return QSM_OK;
@@ -2173,5 +2236,7 @@ int qsm_device_synchronize(void) {
     QSM_HIP(hipDeviceSynchronize());
     return QSM_OK;
 }
+
+void qsm_release_cached_memory(void) { workspace_trim(); }
 
 }  // extern "C"
