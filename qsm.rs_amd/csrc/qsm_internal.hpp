@@ -167,7 +167,8 @@ struct PassArgs {
                               // (TV record / adjoint passes: ridx = checkpoint index)
     double delta;             // erosion threshold
     int sched;                // column-pass FFT schedule (y / z passes): 0 two-stage, 1 LDS-staged
-    int xshift;               // x passes: 0 or 2 (fixed_rows >> xshift pair-rows per block)
+    int xshift;               // x passes: 0 or 2 (shifted_rows(n, xshift) pair-rows per block)
+    int no_change;            // TV C2R: nobody reads this iteration's relative change
 };
 
 // Axis lengths without compiled-length kernels that run fft_dense.hpp.

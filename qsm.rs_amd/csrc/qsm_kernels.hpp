@@ -52,9 +52,6 @@ __device__ __forceinline__ void stg2(QSM_GLOBAL float2* p, float2 a) {
     *(QSM_GLOBAL qsm_f2v*)p = v;
 }
 
-// Waves per SIMD that the dense kernels are held to (the others: no bound).
-constexpr int eg_waves(int eg, int w) { return 1; }
-
 // elements per thread of an x (row) pass / a column pass, LDS tile sizes and
 // twiddle entries (n: compiled length or 0; eg: a run-time kernel's EG)
 __host__ __device__ constexpr int x_emax(int n, int eg) {
@@ -1372,7 +1369,7 @@ __device__ __forceinline__ int plane_fast_block(int lb, int ny, int nz, int R) {
 // RBS: the block takes shifted_rows(N, RBS) pair-rows (small volumes: more,
 // smaller blocks); the host sizes rows_x and the launch the same way.
 template <int N, int EG, int SRC, int RBS = 0>
-__global__ __launch_bounds__(kThreads, eg_waves(EG, 4)) void k_r2c_x(const VolDesc* __restrict__ vols, LaunchTable lt,
+__global__ __launch_bounds__(kThreads) void k_r2c_x(const VolDesc* __restrict__ vols, LaunchTable lt,
                                                     const float2* __restrict__ tw, int out_sel, int aux,
                                                     const VolStatus* status, VolStatus* status_rw,
                                                     VolStatus* mirror, int ck) {
@@ -1506,7 +1503,7 @@ __global__ __launch_bounds__(kThreads, eg_waves(EG, 4)) void k_r2c_x(const VolDe
 // SCHED 0: two-stage column FFT (fft_col2.hpp) where the length allows;
 // SCHED 1: the LDS-staged Stockham stages (less LDS per block).
 template <int N, int EG, bool INV, int SCHED, int TW = kTile>
-__global__ __launch_bounds__(kThreads, eg_waves(EG, 4)) void k_y_pass(const VolDesc* __restrict__ vols, LaunchTable lt,
+__global__ __launch_bounds__(kThreads) void k_y_pass(const VolDesc* __restrict__ vols, LaunchTable lt,
                                                      const float2* __restrict__ tw, int sel, int sel2,
                                                      const VolStatus* __restrict__ status) {
     static_assert(TW == kTile || N == 0, "compiled lengths use tiles of kTile columns");
@@ -2021,7 +2018,7 @@ __device__ __forceinline__ void z_tv_col2(const VolDesc& V, float2* lds, float2*
 }
 
 template <int N, int EG, int OP, int SCHED, int TW = kTile>
-__global__ __launch_bounds__(kThreads, eg_waves(EG, 3)) void k_z_tv(const VolDesc* __restrict__ vols, LaunchTable lt,
+__global__ __launch_bounds__(kThreads) void k_z_tv(const VolDesc* __restrict__ vols, LaunchTable lt,
                                                    const float2* __restrict__ tw,
                                                    const VolStatus* __restrict__ status) {
     constexpr int EMAX = col_emax(N, EG);
@@ -2313,7 +2310,10 @@ __device__ __forceinline__ void c2r_load_rows(float2* lds, const VolDesc& V, int
 // TV: x_it = Re IFFT(x^) (src/inversion/admm.rs:111-114) and the two sums of
 // relative_change (src/utils/mod.rs:69-77) accumulated in FP64 per block;
 // the next pass's first block (or k_tv_reduce after the last iteration)
-// reduces them.
+// reduces them.  no_change: nobody reads this iteration's sums (they are 0),
+// so the previous iterate is not loaded; the pass is bound by memory, and 8
+// bytes a voxel instead of 12 take 20.7 us instead of 25.1 at 256x256x160,
+// 119 instead of 179 for two 384x384x256 volumes.
 // MODE C2R_TV: as above.  C2R_ADJ: Re IFFT to adj_c (c-bar), nothing
 // else.  C2R_F64: Re IFFT widened to f64 into adj_out.
 // C2R_F64_MASKED: f64 into out, 0 where mask == 0 (src/utils/mask.rs:47-53).
@@ -2321,9 +2321,9 @@ __device__ __forceinline__ void c2r_load_rows(float2* lds, const VolDesc& V, int
 enum C2RMode : int { C2R_TV = 0, C2R_ADJ = 1, C2R_F64 = 2, C2R_F64_MASKED = 3, C2R_X0 = 4 };
 
 template <int N, int EG, int MODE, int RBS = 0>
-__global__ __launch_bounds__(kThreads, eg_waves(EG, 4)) void k_c2r_tv(const VolDesc* __restrict__ vols, LaunchTable lt,
+__global__ __launch_bounds__(kThreads) void k_c2r_tv(const VolDesc* __restrict__ vols, LaunchTable lt,
                                                      const float2* __restrict__ tw, int parity,
-                                                     const VolStatus* __restrict__ status) {
+                                                     const VolStatus* __restrict__ status, int no_change) {
     // half the R2C pass's pair-rows (after its row shift RBS), at least 1
     constexpr int RBF = N > 0 ? ((qsmfft::fixed_rows(N) >> RBS) / 2 > 0 ? (qsmfft::fixed_rows(N) >> RBS) / 2 : 1) : 0;
     constexpr int EMAX = N > 0 ? (RBF * N + kThreads - 1) / kThreads : kRowEmaxRt;
@@ -2388,21 +2388,31 @@ __global__ __launch_bounds__(kThreads, eg_waves(EG, 4)) void k_c2r_tv(const VolD
         // four consecutive columns per thread: 16-byte loads of the previous
         // iterate and stores of the new one
         constexpr int E4 = (RBF * N / 4 + kThreads - 1) / kThreads;
-        float4 xa[E4], xb[E4];  // previous iterate, in flight during the inverse FFT
+        float4 xa[E4] = {}, xb[E4] = {};  // previous iterate, in flight during the inverse FFT
+        if (!no_change) {
 #pragma unroll
-        for (int t = 0; t < E4; ++t) {
-            const int e = 4 * (threadIdx.x + t * kThreads);
-            const int p = e / N;
-            const int i = e - p * N;
-            // rows past the volume read its last row: always in bounds, never used
-            const int ra = min(row0 + 2 * p, nrows - 1), rb = min(row0 + 2 * p + 1, nrows - 1);
-            xa[t] = ldv<4>(xo + i + (size_t)ra * N);
-            xb[t] = ldv<4>(xo + i + (size_t)rb * N);
+            for (int t = 0; t < E4; ++t) {
+                const int e = 4 * (threadIdx.x + t * kThreads);
+                const int p = e / N;
+                const int i = e - p * N;
+                // rows past the volume read its last row: always in bounds, never used
+                const int ra = min(row0 + 2 * p, nrows - 1), rb = min(row0 + 2 * p + 1, nrows - 1);
+                xa[t] = ldv<4>(xo + i + (size_t)ra * N);
+                xb[t] = ldv<4>(xo + i + (size_t)rb * N);
+            }
         }
         tws.commit(twl);
         __syncthreads();
         run_fft<N, EG, EMAX, false, 0, true, RBF>(lds, V.px, RB, 1, nx, twl, tw);
         double sd = 0.0, sx = 0.0;
+        auto add = [&](const float* z, float4 prev) {
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                const double d = (double)z[c] - (double)vel<4>(prev, c);
+                sd += d * d;
+                sx += (double)z[c] * (double)z[c];
+            }
+        };
 #pragma unroll
         for (int t = 0; t < E4; ++t) {
             const int e = 4 * (threadIdx.x + t * kThreads);
@@ -2419,21 +2429,11 @@ __global__ __launch_bounds__(kThreads, eg_waves(EG, 4)) void k_c2r_tv(const VolD
                 }
                 if (ra < nrows) {
                     stv<4>(xn + i + (size_t)ra * N, vpack<4>(za));
-#pragma unroll
-                    for (int c = 0; c < 4; ++c) {
-                        const double d = (double)za[c] - (double)vel<4>(xa[t], c);
-                        sd += d * d;
-                        sx += (double)za[c] * (double)za[c];
-                    }
+                    if (!no_change) add(za, xa[t]);
                 }
                 if (rb < nrows) {
                     stv<4>(xn + i + (size_t)rb * N, vpack<4>(zb));
-#pragma unroll
-                    for (int c = 0; c < 4; ++c) {
-                        const double d = (double)zb[c] - (double)vel<4>(xb[t], c);
-                        sd += d * d;
-                        sx += (double)zb[c] * (double)zb[c];
-                    }
+                    if (!no_change) add(zb, xb[t]);
                 }
             }
         }
@@ -2446,16 +2446,18 @@ __global__ __launch_bounds__(kThreads, eg_waves(EG, 4)) void k_c2r_tv(const VolD
         }
         return;
     }
-    float2 xp[EMAX];  // previous iterate, in flight during the inverse FFT
+    float2 xp[EMAX] = {};  // previous iterate, in flight during the inverse FFT
+    if (!no_change) {
 #pragma unroll
-    for (int t = 0; t < EMAX; ++t) {
-        const int e = threadIdx.x + t * kThreads;
-        const int p = div_nx<N>(e, V);
-        const int i = e - p * nx;
-        // rows past the volume read its last row: always in bounds, never used
-        const int ra = min(row0 + 2 * p, nrows - 1), rb = min(row0 + 2 * p + 1, nrows - 1);
-        xp[t].x = xo[i + (size_t)ra * nx];
-        xp[t].y = xo[i + (size_t)rb * nx];
+        for (int t = 0; t < EMAX; ++t) {
+            const int e = threadIdx.x + t * kThreads;
+            const int p = div_nx<N>(e, V);
+            const int i = e - p * nx;
+            // rows past the volume read its last row: always in bounds, never used
+            const int ra = min(row0 + 2 * p, nrows - 1), rb = min(row0 + 2 * p + 1, nrows - 1);
+            xp[t].x = xo[i + (size_t)ra * nx];
+            xp[t].y = xo[i + (size_t)rb * nx];
+        }
     }
     tws.commit(twl);
     __syncthreads();
@@ -2472,14 +2474,18 @@ __global__ __launch_bounds__(kThreads, eg_waves(EG, 4)) void k_c2r_tv(const VolD
             if (ra < nrows) {
                 const double d = (double)z.x - (double)xp[t].x;
                 xn[i + (size_t)ra * nx] = z.x;
-                sd += d * d;
-                sx += (double)z.x * (double)z.x;
+                if (!no_change) {
+                    sd += d * d;
+                    sx += (double)z.x * (double)z.x;
+                }
             }
             if (rb < nrows) {
                 const double d = (double)z.y - (double)xp[t].y;
                 xn[i + (size_t)rb * nx] = z.y;
-                sd += d * d;
-                sx += (double)z.y * (double)z.y;
+                if (!no_change) {
+                    sd += d * d;
+                    sx += (double)z.y * (double)z.y;
+                }
             }
         }
     }
@@ -2504,7 +2510,7 @@ __global__ __launch_bounds__(kThreads, eg_waves(EG, 4)) void k_c2r_tv(const VolD
 //   -> 0 (src/bgremove/vsharp.rs:180-196; division form of
 //   src/bgremove/sharp.rs:113-123 when divide != 0), scaled by 1/N, inverse z.
 template <int N, int EG, int OP, int TW = kTile>
-__global__ __launch_bounds__(kThreads, eg_waves(EG, 3)) void k_z_vs(const VolDesc* __restrict__ vols, LaunchTable lt,
+__global__ __launch_bounds__(kThreads) void k_z_vs(const VolDesc* __restrict__ vols, LaunchTable lt,
                                                    const float2* __restrict__ tw, int sel, int ridx,
                                                    int flag) {
     constexpr int EMAX = col_emax(N, EG);
@@ -2648,7 +2654,7 @@ __global__ __launch_bounds__(kThreads, eg_waves(EG, 3)) void k_z_vs(const VolDes
 // value of the first (largest) radius whose eroded mask contains it
 // (src/bgremove/vsharp.rs:170-176).
 template <int N, int EG>
-__global__ __launch_bounds__(kThreads, eg_waves(EG, 4)) void k_c2r_vs_select(const VolDesc* __restrict__ vols,
+__global__ __launch_bounds__(kThreads) void k_c2r_vs_select(const VolDesc* __restrict__ vols,
                                                             LaunchTable lt,
                                                             const float2* __restrict__ tw, int ridx,
                                                             double delta) {
@@ -2698,7 +2704,7 @@ __global__ __launch_bounds__(kThreads, eg_waves(EG, 4)) void k_c2r_vs_select(con
 // Final rows: local = Re IFFT(.) inside the final mask, 0 outside
 // (src/bgremove/vsharp.rs:194-196); also writes the 0/1 mask.
 template <int N, int EG>
-__global__ __launch_bounds__(kThreads, eg_waves(EG, 4)) void k_c2r_vs_out(const VolDesc* __restrict__ vols, LaunchTable lt,
+__global__ __launch_bounds__(kThreads) void k_c2r_vs_out(const VolDesc* __restrict__ vols, LaunchTable lt,
                                                          const float2* __restrict__ tw) {
     constexpr int EMAX = x_emax(N, EG);
     __shared__ float2 lds[x_lds(N, EG)];

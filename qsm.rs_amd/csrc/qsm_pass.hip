@@ -47,11 +47,11 @@ static void launch_rows_s(int kind, const LaunchTable& lt, const PassArgs& a) {
         case P_R2C_F32: k_r2c_x<N, EG, SRC_F32, RBS><<<g, b, 0, st>>>(a.vols, lt, a.tw, a.sel, 0, a.status, nullptr, nullptr, 0); break;
         case P_R2C_ACC: k_r2c_x<N, EG, SRC_ACC, RBS><<<g, b, 0, st>>>(a.vols, lt, a.tw, a.sel, 0, nullptr, nullptr, nullptr, 0); break;
         case P_R2C_SPHERE: k_r2c_x<N, EG, SRC_SPHERE, RBS><<<g, b, 0, st>>>(a.vols, lt, a.tw, a.sel, a.ridx, a.status, nullptr, nullptr, 0); break;
-        case P_C2R_TV: k_c2r_tv<N, EG, C2R_TV, RBS><<<g, b, 0, st>>>(a.vols, lt, a.tw, a.parity, a.status); break;
-        case P_C2R_ADJ: k_c2r_tv<N, EG, C2R_ADJ, RBS><<<g, b, 0, st>>>(a.vols, lt, a.tw, 0, nullptr); break;
-        case P_C2R_F64OUT: k_c2r_tv<N, EG, C2R_F64, RBS><<<g, b, 0, st>>>(a.vols, lt, a.tw, 0, nullptr); break;
-        case P_C2R_F64_MASKED: k_c2r_tv<N, EG, C2R_F64_MASKED, RBS><<<g, b, 0, st>>>(a.vols, lt, a.tw, 0, nullptr); break;
-        case P_C2R_X0: k_c2r_tv<N, EG, C2R_X0, RBS><<<g, b, 0, st>>>(a.vols, lt, a.tw, 0, nullptr); break;
+        case P_C2R_TV: k_c2r_tv<N, EG, C2R_TV, RBS><<<g, b, 0, st>>>(a.vols, lt, a.tw, a.parity, a.status, a.no_change); break;
+        case P_C2R_ADJ: k_c2r_tv<N, EG, C2R_ADJ, RBS><<<g, b, 0, st>>>(a.vols, lt, a.tw, 0, nullptr, 0); break;
+        case P_C2R_F64OUT: k_c2r_tv<N, EG, C2R_F64, RBS><<<g, b, 0, st>>>(a.vols, lt, a.tw, 0, nullptr, 0); break;
+        case P_C2R_F64_MASKED: k_c2r_tv<N, EG, C2R_F64_MASKED, RBS><<<g, b, 0, st>>>(a.vols, lt, a.tw, 0, nullptr, 0); break;
+        case P_C2R_X0: k_c2r_tv<N, EG, C2R_X0, RBS><<<g, b, 0, st>>>(a.vols, lt, a.tw, 0, nullptr, 0); break;
         case P_R2C_X0: k_r2c_x<N, EG, SRC_X0, RBS><<<g, b, 0, st>>>(a.vols, lt, a.tw, a.sel, 0, nullptr, nullptr, nullptr, 0); break;
         case P_R2C_TVDIV_W:
             k_r2c_x<N, EG, SRC_TVDIV_W, RBS><<<g, b, 0, st>>>(a.vols, lt, a.tw, a.sel, a.parity, a.status,

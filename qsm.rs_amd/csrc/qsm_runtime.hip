@@ -728,6 +728,12 @@ static int run_pass(qsm_tv_batch* B, int slot, int kind, const Groups& gs, const
     return QSM_OK;
 }
 
+// The relative change of iteration `it` reaches nobody: no change is below a
+// tol that is not positive, and what a run reports is the last iteration's.
+static bool change_unread(const qsm_tv_batch* B, size_t it) {
+    return !(B->params.tol > 0.0) && it != B->params.max_iter;
+}
+
 // rec >= 0 also records the shrink pattern of iteration it-1 as checkpoint
 // `rec` (unrolled adjoint).
 static int enqueue_iteration(qsm_tv_batch* B, size_t it, hipEvent_t closed, int rec = -1) {
@@ -756,6 +762,7 @@ static int enqueue_iteration(qsm_tv_batch* B, size_t it, hipEvent_t closed, int 
     if ((rc = run_pass(B, 1, P_Y_FWD, B->gy, a))) return rc;
     if ((rc = run_pass(B, 2, B->method == 1 ? P_Z_RTS_SOLVE : P_Z_TV_SOLVE, B->gz, a))) return rc;
     if ((rc = run_pass(B, 3, P_Y_INV, B->gy, a))) return rc;
+    a.no_change = change_unread(B, it) ? 1 : 0;
     if ((rc = run_pass(B, 4, P_C2R_TV, B->gxc, a))) return rc;
     QSM_CHECK_LAUNCH();
     return QSM_OK;
@@ -831,11 +838,13 @@ static int build_iteration_graphs(qsm_tv_batch* B) {
 
 // Iteration `it` of a run: a graph replay where available, else the eager
 // launches of enqueue_iteration (the first iteration always: its kernels
-// differ, and RTS starts differently).  `closed` marks the point after which
+// differ, and RTS starts differently; the last one where only it forms its
+// relative change).  `closed` marks the point after which
 // iteration it-1's convergence state is in the host mirror: eagerly right
 // after the first pass of iteration it, after a replay at its end.
 static int launch_iteration(qsm_tv_batch* B, size_t it, hipEvent_t closed) {
-    if (it >= 2 && B->graph_state == 1) {
+    const bool last = it == B->params.max_iter && !(B->params.tol > 0.0);
+    if (it >= 2 && B->graph_state == 1 && !last) {
         QSM_HIP(hipGraphLaunch(B->gexec[(it - 1) & 1], B->stream));
         if (closed) QSM_HIP(hipEventRecord(closed, B->stream));
         return QSM_OK;
@@ -963,6 +972,7 @@ static int tv_batch_profile_impl(qsm_tv_batch* B, size_t iters, double* ms_out, 
         QSM_HIP(hipEventRecord(ev[3], st));
         run_groups(P_Y_INV, B->gy, a);
         QSM_HIP(hipEventRecord(ev[4], st));
+        a.no_change = change_unread(B, it) ? 1 : 0;
         run_groups(P_C2R_TV, B->gxc, a);
         QSM_HIP(hipEventRecord(ev[5], st));
         QSM_CHECK_LAUNCH();
