@@ -44,6 +44,11 @@ constexpr int eg_elems(int eg) { return eg & (kEgDense - 1); }
 // fill loads up to four columns from any column of a row.
 constexpr int kRowSlack = 4;
 
+// A TV batch whose arrays (kIterBytes a voxel) are larger than this runs the
+// non-temporal forms of its passes.
+constexpr size_t kIterBytes = 40;
+constexpr size_t kStreamBytes = (size_t)384 << 20;
+
 struct LaunchTable {
     int nvol;
     int start[kMaxVolumes + 1];  // start[v] = first block of entry v; start[nvol] = total
@@ -169,6 +174,7 @@ struct PassArgs {
     int sched;                // column-pass FFT schedule (y / z passes): 0 two-stage, 1 LDS-staged
     int xshift;               // x passes: 0 or 2 (shifted_rows(n, xshift) pair-rows per block)
     int no_change;            // TV C2R: nobody reads this iteration's relative change
+    int nt;                   // TV iteration: the batch's arrays do not fit the Infinity Cache (kStreamBytes)
 };
 
 // Axis lengths without compiled-length kernels that run fft_dense.hpp.

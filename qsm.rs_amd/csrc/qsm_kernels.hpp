@@ -41,8 +41,32 @@ __device__ __forceinline__ const QSM_GLOBAL T* glb(const T* p) { return (const Q
 
 // 8-byte complex access through a global pointer (one dwordx2 load/store).
 typedef float qsm_f2v __attribute__((ext_vector_type(2)));
+// One load / store, NT: with the non-temporal hint (first out of the caches).
+//
+// The TV iteration's passes come in an NT form for batches whose arrays (40
+// bytes a voxel: x and u twice, two spectra) are larger than the 256 MB
+// Infinity Cache (kStreamBytes; the host chooses).  Without a hint each array
+// evicts the next and nothing is left when it is read again; with it the dual
+// variable and f^, read again only an iteration later, and the spectrum's last
+// reading leave the cache to the spectrum and x, which the next pass reads.
+// Measured, us an iteration without and with: two 384x384x256 volumes (3.0
+// GB) 1085 and 1061 (the z pass 170 and 143), four 256x256x160 (1.7 GB) 545
+// and 526, one 250x250x200 (500 MB) 286 and 270, one 256x256x160 (419 MB) 155
+// and 154, one 256x256x144 (377 MB) 144 and 144.  Where it fits the hint
+// loses: 224x224x128 (257 MB) 101 and 104, 192x192x128 (189 MB) 78 and 86.
+template <bool NT, class T>
+__device__ __forceinline__ T ldx(const QSM_GLOBAL T* p) {
+    if constexpr (NT) return __builtin_nontemporal_load(p);
+    else return *p;
+}
+template <bool NT, class T>
+__device__ __forceinline__ void stx(QSM_GLOBAL T* p, T v) {
+    if constexpr (NT) __builtin_nontemporal_store(v, p);
+    else *p = v;
+}
+template <bool NT = false>
 __device__ __forceinline__ float2 ldg2(const QSM_GLOBAL float2* p) {
-    const qsm_f2v v = *(const QSM_GLOBAL qsm_f2v*)p;
+    const qsm_f2v v = ldx<NT>((const QSM_GLOBAL qsm_f2v*)p);
     return make_float2(v.x, v.y);
 }
 __device__ __forceinline__ void stg2(QSM_GLOBAL float2* p, float2 a) {
@@ -563,7 +587,7 @@ __device__ __forceinline__ int8_t shrink_sign(float v, float t) {
     return v > t ? (int8_t)1 : (v < -t ? (int8_t)-1 : (int8_t)0);
 }
 
-template <int CH, bool REC, bool W = false>
+template <int CH, bool REC, bool W, bool NT>
 __device__ __forceinline__ void tvdiv_compute(const TvDivRound<CH, W>& R, float2* lds, const VolDesc& V,
                                               int t0, int EMAX, int total,
                                               QSM_GLOBAL float* __restrict__ uo,
@@ -595,9 +619,9 @@ __device__ __forceinline__ void tvdiv_compute(const TvDivRound<CH, W>& R, float2
             const float zx = shrinkf(vx, ti), zy = shrinkf(vy, ti), zz = shrinkf(vz, ti);
             if (R.ok[c][h]) {
                 const int idx = R.idx[c][h];
-                uo[idx] = vx - zx;
-                uo[N + idx] = vy - zy;
-                uo[2 * N + idx] = vz - zz;
+                stx<NT>(uo + idx, vx - zx);
+                stx<NT>(uo + N + idx, vy - zy);
+                stx<NT>(uo + 2 * N + idx, vz - zz);
                 if constexpr (REC) {
                     // d z / d v of this update, for the unrolled adjoint
                     rec[idx] = shrink_sign(vx, t);
@@ -623,7 +647,7 @@ __device__ __forceinline__ void tvdiv_compute(const TvDivRound<CH, W>& R, float2
 // from x and u at i-1 (likewise y and z), so g never goes to memory.
 // Rounds of CH elements (2*CH voxels) are software-pipelined: the loads of
 // round r+1 are issued before round r is computed and stored.
-template <int EMAX, bool REC, bool W = false>
+template <int EMAX, bool REC, bool W = false, bool NT = false>
 __device__ __forceinline__ void fill_tvdiv(float2* lds, const VolDesc& V, int nx, int RB,
                                            const QSM_GLOBAL float* __restrict__ x,
                                            const QSM_GLOBAL float* __restrict__ u,
@@ -639,10 +663,10 @@ __device__ __forceinline__ void fill_tvdiv(float2* lds, const VolDesc& V, int nx
 #pragma unroll
     for (int r = 0; r < NR; r += 2) {
         if (r + 1 < NR) tvdiv_load<CH, W>(B, V, nx, (r + 1) * CH, EMAX, total, row0, nrows, x, u, w);
-        tvdiv_compute<CH, REC, W>(A, lds, V, r * CH, EMAX, total, uo, rec, wnorm);
+        tvdiv_compute<CH, REC, W, NT>(A, lds, V, r * CH, EMAX, total, uo, rec, wnorm);
         if (r + 1 < NR) {
             if (r + 2 < NR) tvdiv_load<CH, W>(A, V, nx, (r + 2) * CH, EMAX, total, row0, nrows, x, u, w);
-            tvdiv_compute<CH, REC, W>(B, lds, V, (r + 1) * CH, EMAX, total, uo, rec, wnorm);
+            tvdiv_compute<CH, REC, W, NT>(B, lds, V, (r + 1) * CH, EMAX, total, uo, rec, wnorm);
         }
     }
 }
@@ -706,26 +730,31 @@ __device__ __forceinline__ lanev<VW> vzero() {
     const float z[VW] = {};
     return vpack<VW>(z);
 }
-template <int VW>
+template <int VW, bool NT = false>
 __device__ __forceinline__ lanev<VW> ldv(const QSM_GLOBAL float* p) {
-    if constexpr (VW == 1) return *p;
-    else if constexpr (VW == 2) return ldg2((const QSM_GLOBAL float2*)p);
+    if constexpr (VW == 1) return ldx<NT>(p);
+    else if constexpr (VW == 2) return ldg2<NT>((const QSM_GLOBAL float2*)p);
     else {
-        const qsm_f4v v = *(const QSM_GLOBAL qsm_f4v*)p;
+        const qsm_f4v v = ldx<NT>((const QSM_GLOBAL qsm_f4v*)p);
         return make_float4(v.x, v.y, v.z, v.w);
     }
 }
-template <int VW>
+template <int VW, bool NT = false>
 __device__ __forceinline__ void stv(QSM_GLOBAL float* p, lanev<VW> v) {
-    if constexpr (VW == 1) *p = v;
-    else if constexpr (VW == 2) stg2((QSM_GLOBAL float2*)p, v);
-    else {
+    if constexpr (VW == 1) {
+        stx<NT>(p, v);
+    } else if constexpr (VW == 2) {
+        qsm_f2v w;
+        w.x = v.x;
+        w.y = v.y;
+        stx<NT>((QSM_GLOBAL qsm_f2v*)p, w);
+    } else {
         qsm_f4v w;
         w.x = v.x;
         w.y = v.y;
         w.z = v.z;
         w.w = v.w;
-        *(QSM_GLOBAL qsm_f4v*)p = w;
+        stx<NT>((QSM_GLOBAL qsm_f4v*)p, w);
     }
 }
 
@@ -749,7 +778,7 @@ __device__ __forceinline__ int tv_col(int lane, int m) {
 
 // Row r of the volume (r = j + k ny, k the plane): its own x and u, x on the
 // planes k +- 1 and u_z on plane k - 1 (periodic).
-template <int NX, int VW>
+template <int NX, int VW, bool NT>
 __device__ __forceinline__ void tvrow_load(TvRow<NX, VW>& R, int r, int k, int nz, int nxy, int N, int lane,
                                            const QSM_GLOBAL float* __restrict__ x,
                                            const QSM_GLOBAL float* __restrict__ u) {
@@ -764,8 +793,8 @@ __device__ __forceinline__ void tvrow_load(TvRow<NX, VW>& R, int r, int k, int n
 #pragma unroll
     for (int m = 0; m < C; ++m) {
         const int i = tv_col<NX, VW>(lane, m);
-        R.ux[m] = ldv<VW>(ur + i);
-        R.uy[m] = ldv<VW>(ur + N + i);
+        R.ux[m] = ldv<VW, NT>(ur + i);
+        R.uy[m] = ldv<VW, NT>(ur + N + i);
         R.uz[m] = ldv<VW>(ur + 2 * N + i);
         R.xzp[m] = ldv<VW>(xr + dzp + i);
         R.xzm[m] = ldv<VW>(xr + dzm + i);
@@ -792,7 +821,7 @@ __device__ __forceinline__ float tv_gv(float v, float t) { return tv_g(v, tv_cla
 // NX - 1 and 0 from lane broadcasts); only the rows above and below the wave's
 // rows, and y-wrapping rows, are loaded again.  Loads per voxel: 7 plus 3 /
 // (rows per wave), against 13.
-template <int NX, int RB>
+template <int NX, int RB, bool NT>
 __device__ __forceinline__ void fill_tvdiv_rows(float2* lds, const VolDesc& V, int row0, int nrows,
                                                 const QSM_GLOBAL float* __restrict__ x,
                                                 const QSM_GLOBAL float* __restrict__ u,
@@ -819,7 +848,7 @@ __device__ __forceinline__ void fill_tvdiv_rows(float2* lds, const VolDesc& V, i
     TvRow<NX, VW> A, B;
     vt hym_x[C], hym_uy[C], hyp_x[C];  // rows above / below the wave's rows
     if (r0 < nrows) {
-        tvrow_load<NX, VW>(A, r0, k, nz, nxy, N, lane, x, u);
+        tvrow_load<NX, VW, NT>(A, r0, k, nz, nxy, N, lane, x, u);
         // the row before the wave's first row, periodic in y
         const int ra = j > 0 ? r0 - 1 : r0 + ny - 1;
         const QSM_GLOBAL float* xr = x + ra * NX;
@@ -846,7 +875,7 @@ __device__ __forceinline__ void fill_tvdiv_rows(float2* lds, const VolDesc& V, i
             jn = 0;
             ++kn;
         }
-        if (q + 1 < nrw && r + 1 < nrows) tvrow_load<NX, VW>(nxt, r + 1, kn, nz, nxy, N, lane, x, u);
+        if (q + 1 < nrw && r + 1 < nrows) tvrow_load<NX, VW, NT>(nxt, r + 1, kn, nz, nxy, N, lane, x, u);
         if (q + 2 == nrw && ok) {
             // the row after the wave's last row rl = r + 1 (in-plane index
             // jn), periodic in y; issued one row ahead
@@ -958,9 +987,9 @@ __device__ __forceinline__ void fill_tvdiv_rows(float2* lds, const VolDesc& V, i
                 dd[e] = (gx[m][e] - gxm) * hx + (gyv[e] - vel<VW>(gym[m], e)) * hy + (gz - gzm) * hz;
             }
             if (ok && col_ok) {
-                stv<VW>(o, vpack<VW>(ox[m]));
-                stv<VW>(o + N, vpack<VW>(oy));
-                stv<VW>(o + 2 * N, vpack<VW>(oz));
+                stv<VW, NT>(o, vpack<VW>(ox[m]));
+                stv<VW, NT>(o + N, vpack<VW>(oy));
+                stv<VW, NT>(o + 2 * N, vpack<VW>(oz));
             }
             pgy[m] = vpack<VW>(gyv);
             d[m] = ok ? vpack<VW>(dd) : vzero<VW>();
@@ -998,29 +1027,29 @@ template <int VW>
 struct alignas(4) FloatsU {
     float v[VW];
 };
-template <int VW>
+template <int VW, bool NT = false>
 __device__ __forceinline__ FloatsU<VW> ldu(const QSM_GLOBAL float* p) {
     if constexpr (VW == 1) {
-        return FloatsU<VW>{{*p}};
+        return FloatsU<VW>{{ldx<NT>(p)}};
     } else {
         typedef float vt __attribute__((ext_vector_type(VW), aligned(4)));
-        const vt w = *(const QSM_GLOBAL vt*)p;
+        const vt w = ldx<NT>((const QSM_GLOBAL vt*)p);
         FloatsU<VW> r;
 #pragma unroll
         for (int e = 0; e < VW; ++e) r.v[e] = w[e];
         return r;
     }
 }
-template <int VW>
+template <int VW, bool NT>
 __device__ __forceinline__ void stu(QSM_GLOBAL float* p, const float (&a)[VW]) {
     if constexpr (VW == 1) {
-        *p = a[0];
+        stx<NT>(p, a[0]);
     } else {
         typedef float vt __attribute__((ext_vector_type(VW), aligned(4)));
         vt w;
 #pragma unroll
         for (int e = 0; e < VW; ++e) w[e] = a[e];
-        *(QSM_GLOBAL vt*)p = w;
+        stx<NT>((QSM_GLOBAL vt*)p, w);
     }
 }
 
@@ -1043,7 +1072,7 @@ struct TvAnyRow {
 // row's end values.  Rows need not be aligned.
 // One column per lane with the in-row neighbours loaded took 300 instructions
 // per row of 164 columns and 84 us of a pass whose bytes take 36 us.
-template <int VW>
+template <int VW, bool NT>
 __device__ __forceinline__ void fill_tvdiv_any(float2* lds, const VolDesc& V, int nx, int RB, int row0,
                                                int nrows, const QSM_GLOBAL float* __restrict__ x,
                                                const QSM_GLOBAL float* __restrict__ u,
@@ -1074,8 +1103,8 @@ __device__ __forceinline__ void fill_tvdiv_any(float2* lds, const VolDesc& V, in
             const QSM_GLOBAL float* xr = x + r * nx;
             const QSM_GLOBAL float* ur = u + r * nx;
             R.xc = ldu<VW>(xr + cu);
-            R.ux = ldu<VW>(ur + cu);
-            R.uy = ldu<VW>(ur + N + cu);
+            R.ux = ldu<VW, NT>(ur + cu);
+            R.uy = ldu<VW, NT>(ur + N + cu);
             R.uz = ldu<VW>(ur + 2 * N + cu);
             R.xzp = ldu<VW>(xr + dzp + cu);
             R.xzm = ldu<VW>(xr + dzm + cu);
@@ -1151,9 +1180,9 @@ __device__ __forceinline__ void fill_tvdiv_any(float2* lds, const VolDesc& V, in
                 QSM_GLOBAL float* o = uo + r * nx + cu;
                 float* l = ldsf + 2 * ((q >> 1) * nx + c) + (q & 1);
                 if (el >= VW - 1) {
-                    stu<VW>(o, ox);
-                    stu<VW>(o + N, oy);
-                    stu<VW>(o + 2 * N, oz);
+                    stu<VW, NT>(o, ox);
+                    stu<VW, NT>(o + N, oy);
+                    stu<VW, NT>(o + 2 * N, oz);
 #pragma unroll
                     for (int e = 0; e < VW; ++e) l[2 * e] = d[e];
                 } else {
@@ -1182,13 +1211,14 @@ __device__ __forceinline__ void fill_tvdiv_any(float2* lds, const VolDesc& V, in
 }
 
 // Columns per lane of fill_tvdiv_any: rows up to 256 columns in one group.
+template <bool NT>
 __device__ __forceinline__ void fill_tvdiv_runtime(float2* lds, const VolDesc& V, int nx, int RB, int row0, int nrows,
                                                    const QSM_GLOBAL float* __restrict__ x,
                                                    const QSM_GLOBAL float* __restrict__ u,
                                                    QSM_GLOBAL float* __restrict__ uo) {
-    if (nx <= 64) fill_tvdiv_any<1>(lds, V, nx, RB, row0, nrows, x, u, uo);
-    else if (nx <= 128) fill_tvdiv_any<2>(lds, V, nx, RB, row0, nrows, x, u, uo);
-    else fill_tvdiv_any<4>(lds, V, nx, RB, row0, nrows, x, u, uo);
+    if (nx <= 64) fill_tvdiv_any<1, NT>(lds, V, nx, RB, row0, nrows, x, u, uo);
+    else if (nx <= 128) fill_tvdiv_any<2, NT>(lds, V, nx, RB, row0, nrows, x, u, uo);
+    else fill_tvdiv_any<4, NT>(lds, V, nx, RB, row0, nrows, x, u, uo);
 }
 
 // First step of an NLTV Newton round after the first (src/inversion/
@@ -1368,7 +1398,7 @@ __device__ __forceinline__ int plane_fast_block(int lb, int ny, int nz, int R) {
 // record read, and the row of adj_tpart written).
 // RBS: the block takes shifted_rows(N, RBS) pair-rows (small volumes: more,
 // smaller blocks); the host sizes rows_x and the launch the same way.
-template <int N, int EG, int SRC, int RBS = 0>
+template <int N, int EG, int SRC, int RBS = 0, bool NT = false>
 __global__ __launch_bounds__(kThreads) void k_r2c_x(const VolDesc* __restrict__ vols, LaunchTable lt,
                                                     const float2* __restrict__ tw, int out_sel, int aux,
                                                     const VolStatus* status, VolStatus* status_rw,
@@ -1403,11 +1433,11 @@ __global__ __launch_bounds__(kThreads) void k_r2c_x(const VolDesc* __restrict__ 
     TwStage<N, EG> tws;
     tws.fetch(tw, V.px);
     if constexpr (SRC == SRC_TVDIV && tvdiv_rows_form(N, RBX)) {
-        fill_tvdiv_rows<N, RBX>(lds, V, row0, nrows, glb(V.x[aux]), glb(V.u[aux ^ 1]), glb(V.u[aux]));
+        fill_tvdiv_rows<N, RBX, NT>(lds, V, row0, nrows, glb(V.x[aux]), glb(V.u[aux ^ 1]), glb(V.u[aux]));
     } else if constexpr (SRC == SRC_TVDIV && N == 0 && eg_dense(EG)) {
-        fill_tvdiv_runtime(lds, V, nx, RB, row0, nrows, glb(V.x[aux]), glb(V.u[aux ^ 1]), glb(V.u[aux]));
+        fill_tvdiv_runtime<NT>(lds, V, nx, RB, row0, nrows, glb(V.x[aux]), glb(V.u[aux ^ 1]), glb(V.u[aux]));
     } else if constexpr (SRC == SRC_TVDIV) {
-        fill_tvdiv<EMAX, false>(lds, V, nx, RB, glb(V.x[aux]), glb(V.u[aux ^ 1]), glb(V.u[aux]), row0,
+        fill_tvdiv<EMAX, false, false, NT>(lds, V, nx, RB, glb(V.x[aux]), glb(V.u[aux ^ 1]), glb(V.u[aux]), row0,
                                 nrows, nullptr);
     } else if constexpr (SRC == SRC_TVDIV_REC) {
         const size_t N3 = (size_t)3 * V.nx * V.ny * V.nz;
@@ -1917,7 +1947,7 @@ __device__ __forceinline__ size_t q_nyq_base(const VolDesc& V, int ky) {
 // The per-iteration ops (SOLVE, SOLVE0, ADJ, RTS_SOLVE) at the lengths of
 // fft_col2.hpp: forward z from the load layout, the product in registers,
 // inverse z back to the load layout; two LDS exchanges in all.
-template <int N, int EG, int OP>
+template <int N, int EG, int OP, bool NT>
 __device__ __forceinline__ void z_tv_col2(const VolDesc& V, float2* lds, float2* twl, const TwStage<N, EG>& tws,
                                           int ky, int kx0, bool dpk) {
     constexpr int R0 = N / 16;
@@ -1952,7 +1982,7 @@ __device__ __forceinline__ void z_tv_col2(const VolDesc& V, float2* lds, float2*
         const QSM_GLOBAL float* __restrict__ Q = glb(V.q) + off;
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-            if constexpr (HAS_F) fr[r] = ldg2(F + R0 * r * kTile);
+            if constexpr (HAS_F) fr[r] = ldg2<NT>(F + R0 * r * kTile);
             if constexpr (Q_MEM) qr[r] = Q[R0 * r * kTile];
         }
     }
@@ -2017,7 +2047,7 @@ __device__ __forceinline__ void z_tv_col2(const VolDesc& V, float2* lds, float2*
     l16_store<R0>(v, buf, zs, kx0, nxh);
 }
 
-template <int N, int EG, int OP, int SCHED, int TW = kTile>
+template <int N, int EG, int OP, int SCHED, int TW = kTile, bool NT = false>
 __global__ __launch_bounds__(kThreads) void k_z_tv(const VolDesc* __restrict__ vols, LaunchTable lt,
                                                    const float2* __restrict__ tw,
                                                    const VolStatus* __restrict__ status) {
@@ -2050,7 +2080,7 @@ __global__ __launch_bounds__(kThreads) void k_z_tv(const VolDesc* __restrict__ v
     TwStage<N, EG> tws;
     tws.fetch(tw, V.pz);
     if constexpr (TWO) {
-        z_tv_col2<N, EG, OP>(V, lds, twl, tws, ky, kx0, dpk);
+        z_tv_col2<N, EG, OP, NT>(V, lds, twl, tws, ky, kx0, dpk);
         return;
     }
     if constexpr (OP == ZOP_TV_SOLVE0) {
@@ -2093,7 +2123,7 @@ __global__ __launch_bounds__(kThreads) void k_z_tv(const VolDesc* __restrict__ v
             const int kz = e >> L2;
             const int kx = kx0 + (e & (TW - 1));
             const bool in = e < total && kx < nxh;
-            if constexpr (HAS_F) fr[t] = in ? ldg2(F + kx + kz * TW) : make_float2(0.0f, 0.0f);
+            if constexpr (HAS_F) fr[t] = in ? ldg2<NT>(F + kx + kz * TW) : make_float2(0.0f, 0.0f);
             if constexpr (Q_MEM) qr[t] = in ? Q[kx + kz * TW] : 0.0f;
         }
     }
@@ -2253,7 +2283,7 @@ __device__ __forceinline__ void c2r_load(float2* lds, const VolDesc& V, int nx, 
 // every entry read once) and writes the full-spectrum elements they give:
 // k and N - k for 0 < k < N / 2, and for k = 0 the DC element and the
 // Nyquist element N / 2 (the imaginary parts of the packed column 0).
-template <int N, int RB>
+template <int N, int RB, bool NT>
 __device__ __forceinline__ void c2r_load_pairs(float2* lds, const QSM_GLOBAL float2* __restrict__ sa,
                                                const QSM_GLOBAL float2* __restrict__ sb, int row0, int step,
                                                int nrows) {
@@ -2270,8 +2300,8 @@ __device__ __forceinline__ void c2r_load_pairs(float2* lds, const QSM_GLOBAL flo
         // rows past the volume read its last row: in bounds, never stored
         const int ra = min(row0 + step * p, nrows - 1);
         const int rb = min((step == 2) ? row0 + step * p + 1 : row0 + step * p, nrows - 1);
-        a[t] = ldv<4>((const QSM_GLOBAL float*)(sa + k0 + (size_t)ra * NH));
-        b[t] = ldv<4>((const QSM_GLOBAL float*)(sb + k0 + (size_t)rb * NH));
+        a[t] = ldv<4, NT>((const QSM_GLOBAL float*)(sa + k0 + (size_t)ra * NH));
+        b[t] = ldv<4, NT>((const QSM_GLOBAL float*)(sb + k0 + (size_t)rb * NH));
     }
 #pragma unroll
     for (int t = 0; t < T; ++t) {
@@ -2298,12 +2328,12 @@ __device__ __forceinline__ void c2r_load_pairs(float2* lds, const QSM_GLOBAL flo
 }
 
 // c2r_load_pairs where it applies, else c2r_load.
-template <int N, int RBC, int EMAX>
+template <int N, int RBC, int EMAX, bool NT = false>
 __device__ __forceinline__ void c2r_load_rows(float2* lds, const VolDesc& V, int nx, int nxh, int RB,
                                               const QSM_GLOBAL float2* __restrict__ sa,
                                               const QSM_GLOBAL float2* __restrict__ sb, int row0, int step,
                                               int nrows) {
-    if constexpr (N > 0 && N % 4 == 0) c2r_load_pairs<N, RBC>(lds, sa, sb, row0, step, nrows);
+    if constexpr (N > 0 && N % 4 == 0) c2r_load_pairs<N, RBC, NT>(lds, sa, sb, row0, step, nrows);
     else c2r_load<N, EMAX>(lds, V, nx, nxh, RB, sa, sb, row0, step, nrows);
 }
 
@@ -2320,7 +2350,7 @@ __device__ __forceinline__ void c2r_load_rows(float2* lds, const VolDesc& V, int
 // C2R_X0: FP32 into x[0], 0 where mask == 0 (the RTS starting point).
 enum C2RMode : int { C2R_TV = 0, C2R_ADJ = 1, C2R_F64 = 2, C2R_F64_MASKED = 3, C2R_X0 = 4 };
 
-template <int N, int EG, int MODE, int RBS = 0>
+template <int N, int EG, int MODE, int RBS = 0, bool NT = false>
 __global__ __launch_bounds__(kThreads) void k_c2r_tv(const VolDesc* __restrict__ vols, LaunchTable lt,
                                                      const float2* __restrict__ tw, int parity,
                                                      const VolStatus* __restrict__ status, int no_change) {
@@ -2344,7 +2374,7 @@ __global__ __launch_bounds__(kThreads) void k_c2r_tv(const VolDesc* __restrict__
     const QSM_GLOBAL float2* s = glb(V.spec[SPEC_WORK]);
     TwStage<N, EG> tws;
     tws.fetch(tw, V.px);
-    c2r_load_rows<N, RBF, EMAX>(lds, V, nx, nxh, RB, s, s, row0, 2, nrows);
+    c2r_load_rows<N, RBF, EMAX, NT>(lds, V, nx, nxh, RB, s, s, row0, 2, nrows);
     if constexpr (MODE != C2R_TV) {
         tws.commit(twl);
         __syncthreads();

@@ -25,10 +25,14 @@ template <int N, int EG, int RBS>
 static void launch_rows_s(int kind, const LaunchTable& lt, const PassArgs& a) {
     const dim3 g(lt.start[lt.nvol]), b(kThreads);
     hipStream_t st = a.stream;
+    constexpr bool kNt = RBS == 0;
+    const bool nt = kNt && a.nt;
     switch (kind) {
         case P_R2C_TVDIV:
-            k_r2c_x<N, EG, SRC_TVDIV, RBS><<<g, b, 0, st>>>(a.vols, lt, a.tw, a.sel, a.parity, a.status,
-                                                       a.status_rw, a.mirror, 0);
+            if (nt) k_r2c_x<N, EG, SRC_TVDIV, RBS, kNt><<<g, b, 0, st>>>(a.vols, lt, a.tw, a.sel, a.parity, a.status,
+                                                                         a.status_rw, a.mirror, 0);
+            else k_r2c_x<N, EG, SRC_TVDIV, RBS><<<g, b, 0, st>>>(a.vols, lt, a.tw, a.sel, a.parity, a.status,
+                                                                a.status_rw, a.mirror, 0);
             break;
         case P_R2C_TVDIV_REC:
             k_r2c_x<N, EG, SRC_TVDIV_REC, RBS><<<g, b, 0, st>>>(a.vols, lt, a.tw, a.sel, a.parity, a.status,
@@ -47,7 +51,10 @@ static void launch_rows_s(int kind, const LaunchTable& lt, const PassArgs& a) {
         case P_R2C_F32: k_r2c_x<N, EG, SRC_F32, RBS><<<g, b, 0, st>>>(a.vols, lt, a.tw, a.sel, 0, a.status, nullptr, nullptr, 0); break;
         case P_R2C_ACC: k_r2c_x<N, EG, SRC_ACC, RBS><<<g, b, 0, st>>>(a.vols, lt, a.tw, a.sel, 0, nullptr, nullptr, nullptr, 0); break;
         case P_R2C_SPHERE: k_r2c_x<N, EG, SRC_SPHERE, RBS><<<g, b, 0, st>>>(a.vols, lt, a.tw, a.sel, a.ridx, a.status, nullptr, nullptr, 0); break;
-        case P_C2R_TV: k_c2r_tv<N, EG, C2R_TV, RBS><<<g, b, 0, st>>>(a.vols, lt, a.tw, a.parity, a.status, a.no_change); break;
+        case P_C2R_TV:
+            if (nt) k_c2r_tv<N, EG, C2R_TV, RBS, kNt><<<g, b, 0, st>>>(a.vols, lt, a.tw, a.parity, a.status, a.no_change);
+            else k_c2r_tv<N, EG, C2R_TV, RBS><<<g, b, 0, st>>>(a.vols, lt, a.tw, a.parity, a.status, a.no_change);
+            break;
         case P_C2R_ADJ: k_c2r_tv<N, EG, C2R_ADJ, RBS><<<g, b, 0, st>>>(a.vols, lt, a.tw, 0, nullptr, 0); break;
         case P_C2R_F64OUT: k_c2r_tv<N, EG, C2R_F64, RBS><<<g, b, 0, st>>>(a.vols, lt, a.tw, 0, nullptr, 0); break;
         case P_C2R_F64_MASKED: k_c2r_tv<N, EG, C2R_F64_MASKED, RBS><<<g, b, 0, st>>>(a.vols, lt, a.tw, 0, nullptr, 0); break;
@@ -99,6 +106,7 @@ static void launch_cols(int kind, const LaunchTable& lt, const PassArgs& a) {
         case P_Z_TV_SETUP: k_z_tv<N, EG, ZOP_TV_SETUP, 1, TW><<<g, b, 0, st>>>(a.vols, lt, a.tw, a.status); break;
         case P_Z_TV_SOLVE:
             if (a.sched) k_z_tv<N, EG, ZOP_TV_SOLVE, 1, TW><<<g, b, 0, st>>>(a.vols, lt, a.tw, a.status);
+            else if (a.nt) k_z_tv<N, EG, ZOP_TV_SOLVE, S0, TW, true><<<g, b, 0, st>>>(a.vols, lt, a.tw, a.status);
             else k_z_tv<N, EG, ZOP_TV_SOLVE, S0, TW><<<g, b, 0, st>>>(a.vols, lt, a.tw, a.status);
             break;
         case P_Z_TV_ADJ:

@@ -383,6 +383,7 @@ struct qsm_tv_batch {
     // other t (a negative lambda, say) the recording kernel, which forms
     // shrink itself, runs in its place with a scratch record.
     bool plain_shrink = false;
+    bool streams = false;  // larger than the Infinity Cache (kStreamBytes)
     bool field32 = false;  // the field is VolDesc::vs_local, in f32 (host entry points)
     void* host_out = nullptr;  // their result array, made ready while the device works
     size_t host_bytes = 0;
@@ -409,6 +410,7 @@ struct qsm_tv_batch {
         a.mirror = nullptr;
         a.sel = SPEC_WORK;
         a.sel2 = -1;
+        a.nt = streams ? 1 : 0;
         return a;
     }
     hipEvent_t ev[kWindow] = {};
@@ -581,6 +583,12 @@ static int tv_batch_create_impl(const qsm_tv_volume* vols, size_t n_vols, const 
         xshift[v] = (fixed && (npairs + r0 - 1) / r0 < 1024 && (r0 >> 2) >= 4) ? 2 : 0;
         cshift[v] = (fixed && (npairs + rc - 1) / rc < 1024 && (r0 >> 2) / 2 >= 4) ? 2 : 0;
     }
+    // (the quarter-row R2C pass has no non-temporal form: three 192x192x128
+    // volumes, 566 MB, took 203 us an iteration, 205 with the other passes' forms)
+    size_t voxels = 0;
+    for (size_t v = 0; v < n_vols; ++v)
+        if (!xshift[v]) voxels += vols[v].grid.nx * vols[v].grid.ny * vols[v].grid.nz;
+    B->streams = voxels * kIterBytes > kStreamBytes;
     for (size_t v = 0; v < n_vols; ++v) {
         VolDesc& V = B->h[v];
         std::memset(&V, 0, sizeof V);
