@@ -33,7 +33,7 @@ constexpr int kMaxDenseLen = 512;    // tiles of 16 columns up to 256, 8 above
 constexpr int kMaxDenseRadix = 256;  // above, only primes: chirp-z (fft_chirp.hpp)
 constexpr int kMaxRegRadix = 16;
 constexpr int kDenseElems = 16 * kThreads;  // elements of the largest tile
-constexpr int kDenseUnits = 4;              // units one wave holds (16 accumulators each)
+constexpr int kDenseUnits = 4;              // units one wave holds (16 accumulators each) of such a tile
 
 template <bool INV> struct Dft<6, INV> : DftSplit<2, 3, INV> {};
 
@@ -109,17 +109,18 @@ __host__ __device__ __forceinline__ int dense_r(int kk, int lane) { return 4 * k
 __host__ __device__ __forceinline__ int dense_q(int mt, int lane, int v) { return 16 * mt + 4 * (lane >> 4) + v; }
 
 // Register-radix stage in place, as fixed_stage_load / _store with run-time
-// geometry: B butterflies per thread at most.
-template <int R>
+// geometry: B butterflies per thread at most, in a tile of E elements per
+// thread (16, or 8: half tiles).
+template <int R, int E = kDenseElems / kThreads>
 struct RegStage {
-    static constexpr int B = (kDenseElems / kThreads + R - 1) / R;
+    static constexpr int B = (E + R - 1) / R;
 };
-template <int R, bool COLFAST, int LOG2C>
+template <int R, bool COLFAST, int LOG2C, int E = kDenseElems / kThreads>
 __host__ __device__ __forceinline__ void reg_stage_load(const float2* lds, int tid, const StageGeom& g,
-                                                        float2 (&v)[RegStage<R>::B][R]) {
+                                                        float2 (&v)[RegStage<R, E>::B][R]) {
     const int total = g.nb * g.ncols;
 #pragma unroll
-    for (int t = 0; t < RegStage<R>::B; ++t) {
+    for (int t = 0; t < RegStage<R, E>::B; ++t) {
         const int b = tid + t * kThreads;
         if (b < total) {
             int j, c;
@@ -130,12 +131,12 @@ __host__ __device__ __forceinline__ void reg_stage_load(const float2* lds, int t
         }
     }
 }
-template <int R, bool COLFAST, int LOG2C, bool INV>
+template <int R, bool COLFAST, int LOG2C, bool INV, int E = kDenseElems / kThreads>
 __host__ __device__ __forceinline__ void reg_stage_store(float2* lds, int tid, const StageGeom& g,
-                                                         float2 (&v)[RegStage<R>::B][R], const float2* tw) {
+                                                         float2 (&v)[RegStage<R, E>::B][R], const float2* tw) {
     const int total = g.nb * g.ncols;
 #pragma unroll
-    for (int t = 0; t < RegStage<R>::B; ++t) {
+    for (int t = 0; t < RegStage<R, E>::B; ++t) {
         const int b = tid + t * kThreads;
         if (b < total) {
             int j, c;
@@ -170,13 +171,14 @@ typedef float mfma_f4 __attribute__((ext_vector_type(4)));
 // unit's included): fetched a step ahead they held each step for an L2 round
 // trip.  Barriers: the caller's before, one between the reads and the writes,
 // one after.
-template <bool COLFAST, int LOG2C, bool INV>
+template <int E, bool COLFAST, int LOG2C, bool INV>
 __device__ __forceinline__ void dense_stage(float2* lds, const DenseGeom& g, const float2* tw,
                                             const float2* __restrict__ coef) {
     const int lane = (int)(threadIdx.x & 63);
     const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int bstep = kDenseBlock * 64;
-    mfma_f4 are[kDenseUnits], aim[kDenseUnits], bre[kDenseUnits], bim[kDenseUnits];
+    constexpr int UNITS = kDenseUnits * E * kThreads / kDenseElems;
+    mfma_f4 are[UNITS], aim[UNITS], bre[UNITS], bim[UNITS];
     const mfma_f4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
     float2 w[kDenseBlock];
     auto fetch = [&](int unit, int kb) {  // in bounds for every unit (mt < g.mt) and kb < g.kb
@@ -189,7 +191,7 @@ __device__ __forceinline__ void dense_stage(float2* lds, const DenseGeom& g, con
     fetch(wv, 0);
     const int se4 = 4 * g.se;
 #pragma unroll
-    for (int u = 0; u < kDenseUnits; ++u) {
+    for (int u = 0; u < UNITS; ++u) {
         const int unit = wv + u * (kThreads / 64);
         if (unit < g.units) {
             int nt, mt, in, out, ts;
@@ -251,7 +253,7 @@ __device__ __forceinline__ void dense_stage(float2* lds, const DenseGeom& g, con
     __syncthreads();
     const int so = g.Ns * g.es;
 #pragma unroll
-    for (int u = 0; u < kDenseUnits; ++u) {
+    for (int u = 0; u < UNITS; ++u) {
         const int unit = wv + u * (kThreads / 64);
         if (unit < g.units) {
             int nt, mt, in, out, ts;
@@ -277,42 +279,42 @@ __device__ __forceinline__ void dense_stage(float2* lds, const DenseGeom& g, con
     __syncthreads();
 }
 
-template <int R, bool COLFAST, int LOG2C, bool INV>
+template <int R, int E, bool COLFAST, int LOG2C, bool INV>
 __device__ __forceinline__ void reg_stage(float2* lds, const Plan& P, int s, int ncols, int es, int cs,
                                           const float2* tw) {
     const StageGeom g = plan_geom(P, s, ncols, es, cs);
-    float2 v[RegStage<R>::B][R];
-    reg_stage_load<R, COLFAST, LOG2C>(lds, threadIdx.x, g, v);
+    float2 v[RegStage<R, E>::B][R];
+    reg_stage_load<R, COLFAST, LOG2C, E>(lds, threadIdx.x, g, v);
     __syncthreads();
-    reg_stage_store<R, COLFAST, LOG2C, INV>(lds, threadIdx.x, g, v, tw);
+    reg_stage_store<R, COLFAST, LOG2C, INV, E>(lds, threadIdx.x, g, v, tw);
     __syncthreads();
 }
 
 // Full transform, in place in lds (ncols sequences of P.n elements at
 // e * es + c * cs).  tw: the twiddle table in LDS; twg: the bank in global
-// memory (the dense tables).  The caller has synchronised after filling the
-// tile; returns after a final barrier.
-template <bool COLFAST, int LOG2C, bool INV>
+// memory (the dense tables); E: the tile's elements per thread.  The caller has
+// synchronised after filling the tile; returns after a final barrier.
+template <int E, bool COLFAST, int LOG2C, bool INV>
 __device__ __forceinline__ void lds_fft_dense(float2* lds, const Plan& P, int ncols, int es, int cs,
                                               const float2* tw, const float2* __restrict__ twg) {
     for (int s = 0; s < P.nstages; ++s) {
         switch (P.radix[s]) {
-            case 2: reg_stage<2, COLFAST, LOG2C, INV>(lds, P, s, ncols, es, cs, tw); break;
-            case 3: reg_stage<3, COLFAST, LOG2C, INV>(lds, P, s, ncols, es, cs, tw); break;
-            case 4: reg_stage<4, COLFAST, LOG2C, INV>(lds, P, s, ncols, es, cs, tw); break;
-            case 5: reg_stage<5, COLFAST, LOG2C, INV>(lds, P, s, ncols, es, cs, tw); break;
-            case 6: reg_stage<6, COLFAST, LOG2C, INV>(lds, P, s, ncols, es, cs, tw); break;
-            case 7: reg_stage<7, COLFAST, LOG2C, INV>(lds, P, s, ncols, es, cs, tw); break;
-            case 8: reg_stage<8, COLFAST, LOG2C, INV>(lds, P, s, ncols, es, cs, tw); break;
-            case 9: reg_stage<9, COLFAST, LOG2C, INV>(lds, P, s, ncols, es, cs, tw); break;
-            case 10: reg_stage<10, COLFAST, LOG2C, INV>(lds, P, s, ncols, es, cs, tw); break;
-            case 11: reg_stage<11, COLFAST, LOG2C, INV>(lds, P, s, ncols, es, cs, tw); break;
-            case 12: reg_stage<12, COLFAST, LOG2C, INV>(lds, P, s, ncols, es, cs, tw); break;
-            case 13: reg_stage<13, COLFAST, LOG2C, INV>(lds, P, s, ncols, es, cs, tw); break;
-            case 14: reg_stage<14, COLFAST, LOG2C, INV>(lds, P, s, ncols, es, cs, tw); break;
-            case 15: reg_stage<15, COLFAST, LOG2C, INV>(lds, P, s, ncols, es, cs, tw); break;
-            case 16: reg_stage<16, COLFAST, LOG2C, INV>(lds, P, s, ncols, es, cs, tw); break;
-            default: dense_stage<COLFAST, LOG2C, INV>(lds, dense_geom(P, s, ncols, es, cs), tw, twg + P.dn_off[s]);
+            case 2: reg_stage<2, E, COLFAST, LOG2C, INV>(lds, P, s, ncols, es, cs, tw); break;
+            case 3: reg_stage<3, E, COLFAST, LOG2C, INV>(lds, P, s, ncols, es, cs, tw); break;
+            case 4: reg_stage<4, E, COLFAST, LOG2C, INV>(lds, P, s, ncols, es, cs, tw); break;
+            case 5: reg_stage<5, E, COLFAST, LOG2C, INV>(lds, P, s, ncols, es, cs, tw); break;
+            case 6: reg_stage<6, E, COLFAST, LOG2C, INV>(lds, P, s, ncols, es, cs, tw); break;
+            case 7: reg_stage<7, E, COLFAST, LOG2C, INV>(lds, P, s, ncols, es, cs, tw); break;
+            case 8: reg_stage<8, E, COLFAST, LOG2C, INV>(lds, P, s, ncols, es, cs, tw); break;
+            case 9: reg_stage<9, E, COLFAST, LOG2C, INV>(lds, P, s, ncols, es, cs, tw); break;
+            case 10: reg_stage<10, E, COLFAST, LOG2C, INV>(lds, P, s, ncols, es, cs, tw); break;
+            case 11: reg_stage<11, E, COLFAST, LOG2C, INV>(lds, P, s, ncols, es, cs, tw); break;
+            case 12: reg_stage<12, E, COLFAST, LOG2C, INV>(lds, P, s, ncols, es, cs, tw); break;
+            case 13: reg_stage<13, E, COLFAST, LOG2C, INV>(lds, P, s, ncols, es, cs, tw); break;
+            case 14: reg_stage<14, E, COLFAST, LOG2C, INV>(lds, P, s, ncols, es, cs, tw); break;
+            case 15: reg_stage<15, E, COLFAST, LOG2C, INV>(lds, P, s, ncols, es, cs, tw); break;
+            case 16: reg_stage<16, E, COLFAST, LOG2C, INV>(lds, P, s, ncols, es, cs, tw); break;
+            default: dense_stage<E, COLFAST, LOG2C, INV>(lds, dense_geom(P, s, ncols, es, cs), tw, twg + P.dn_off[s]);
         }
     }
 }

@@ -21,13 +21,13 @@ namespace qsm {
 constexpr int kMaxVolumes = 64;
 constexpr int kTile = 16;      // columns per y/z-pass tile (16 * 8 B = 128 B rows)
 constexpr int kLog2Tile = 4;
-// Run-time column lengths above 256 run in tiles of kTileLong columns;
+// Run-time column lengths above 256, and those in half tiles, run in tiles of
+// kTileLong columns;
 // compiled lengths, at most kWideTileMaxLen, in tiles of kTile.
 constexpr int kTileLong = 8;
 constexpr int kWideTileMaxLen = 512;
 constexpr int tile_log2(int tw) { return tw == 16 ? 4 : (tw == 8 ? 3 : -1); }
-// Added to a dense column kernel's launch size (emax_for) when it runs in
-// tiles of kTileLong columns.
+// Added to a dense column kernel's launch size (emax_for) above length 256.
 constexpr int kColLongTile = 256;
 // Elements per thread of the runtime-plan row kernels (tiles of
 // kThreads * kRowEmaxRt elements; the compiled ones take 16).
@@ -35,7 +35,7 @@ constexpr int kRowEmaxRt = 8;
 
 // Added to EG by the kernels that run fft_dense.hpp: in place in one tile of
 // 16 elements per thread (columns: tiles of kTile up to length 256, of
-// kTileLong up to 512).
+// kTileLong up to 512) or 8 (columns: half tiles of kTileLong up to 256).
 constexpr int kEgDense = 1024;
 constexpr bool eg_dense(int eg) { return eg >= kEgDense; }
 constexpr int eg_elems(int eg) { return eg & (kEgDense - 1); }

@@ -126,7 +126,7 @@ __device__ __forceinline__ void run_fft(float2* lds, const qsmfft::Plan& P, int 
     if constexpr (N > 0) {
         qsmfft::fixed_fft<N, NC ? NC : (COLFAST ? kTile : qsmfft::fixed_rows(N)), COLFAST, INV>(lds, twl);
     } else if constexpr (eg_dense(EG)) {
-        qsmfft::lds_fft_dense<COLFAST, LOG2C, INV>(lds, P, ncols, es, cs, twl, twg);
+        qsmfft::lds_fft_dense<EMAX, COLFAST, LOG2C, INV>(lds, P, ncols, es, cs, twl, twg);
     } else {
         // runtime-planned lengths (513 ... 1024, and chirp-z primes above 256):
         // out-of-place stages between the kernel's tile (kThreads * EMAX

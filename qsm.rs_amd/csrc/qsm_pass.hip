@@ -7,7 +7,7 @@
 #error "compile with -DQSM_PASS_N=<axis length> (0 for the runtime-plan kernels)"
 #endif
 #if QSM_PASS_N == 0 && !defined(QSM_GENERIC_PART)
-#error "the run-time-length kernels compile with -DQSM_GENERIC_PART=0..4"
+#error "the run-time-length kernels compile with -DQSM_GENERIC_PART=0..5"
 #endif
 
 namespace qsm {
@@ -140,16 +140,18 @@ void QSM_CAT(launch_fixed_, QSM_PASS_N)(int kind, const LaunchTable& lt, const P
     else launch_cols<QSM_PASS_N, 0>(kind, lt, a);
 }
 #elif QSM_GENERIC_PART == 0
-// The run-time-length kernels are compiled in five parts (this one with the
+// The run-time-length kernels are compiled in six parts (this one with the
 // runtime-plan row kernels and the dispatcher) so that they build in parallel.
 void launch_plan_cols(int kind, const LaunchTable& lt, const PassArgs& a);
 void launch_dense_rows(int kind, const LaunchTable& lt, const PassArgs& a);
 void launch_dense_cols(int kind, const LaunchTable& lt, const PassArgs& a);
+void launch_dense_cols_half(int kind, const LaunchTable& lt, const PassArgs& a);
 void launch_dense_cols_long(int kind, const LaunchTable& lt, const PassArgs& a);
 void launch_generic(int kind, int emax, const LaunchTable& lt, const PassArgs& a) {
     if (eg_dense(emax)) {
         if (is_row_kind(kind)) launch_dense_rows(kind, lt, a);
         else if (eg_elems(emax) > kColLongTile) launch_dense_cols_long(kind, lt, a);  // 257 ... 512
+        else if (eg_elems(emax) == 8) launch_dense_cols_half(kind, lt, a);            // half tiles
         else launch_dense_cols(kind, lt, a);                                          // <= 256
     } else if (is_row_kind(kind)) {
         launch_rows<0, 16>(kind, lt, a);
@@ -163,9 +165,13 @@ void launch_plan_cols(int kind, const LaunchTable& lt, const PassArgs& a) { laun
 void launch_dense_rows(int kind, const LaunchTable& lt, const PassArgs& a) { launch_rows<0, kEgDense + 16>(kind, lt, a); }
 #elif QSM_GENERIC_PART == 3
 void launch_dense_cols(int kind, const LaunchTable& lt, const PassArgs& a) { launch_cols<0, kEgDense + 16>(kind, lt, a); }
-#else
+#elif QSM_GENERIC_PART == 4
 void launch_dense_cols_long(int kind, const LaunchTable& lt, const PassArgs& a) {
     launch_cols<0, kEgDense + 16, kTileLong>(kind, lt, a);
+}
+#else
+void launch_dense_cols_half(int kind, const LaunchTable& lt, const PassArgs& a) {
+    launch_cols<0, kEgDense + 8, kTileLong>(kind, lt, a);
 }
 #endif
 

@@ -82,16 +82,36 @@ bool dense_length(int n) {
 // convolution length), which sizes the LDS tiles.
 int work_length(int n) { return dense_length(n) || direct_length(n) ? n : chirp_length(n); }
 
+// Dense column lengths up to 256 that take half tiles (kTileLong columns, 8
+// elements per thread): a z pass keeps 3 waves per SIMD instead of 2 (80 -> 62
+// us at 205, 82 -> 67 at 231), a y pass gains up to a tenth (27 -> 25 us at 250).
+// Not where a dense radix has fewer than 4 butterflies a column (8 columns then
+// fill half of a 16-wide matrix tile: the y pass at 211 29 -> 38 us), nor below
+// 128 rows (too little work per block: z at 66 13.6 -> 16.2 us).
+static bool half_tile(int n) {
+    int r[qsmfft::kMaxStages], st = 0;
+    if (n < 128 || n > 256 || !qsmfft::dense_factorize(n, r, &st)) return false;
+    for (int s = 0; s < st; ++s)
+        if (r[s] > qsmfft::kMaxRegRadix && n / r[s] < 4) return false;
+    return true;
+}
+
 // Columns per tile of a column pass of length n: kTile up to 256 and for the
 // compiled lengths, kTileLong above (a tile of 4096 elements at most, so four
-// blocks fit a CU's LDS).
-int col_tile(int n) { return has_fixed_kernels(n) || work_length(n) <= 256 ? kTile : kTileLong; }
+// blocks fit a CU's LDS) and in half tiles.
+int col_tile(int n) {
+    if (has_fixed_kernels(n)) return kTile;
+    return work_length(n) > 256 || half_tile(n) ? kTileLong : kTile;
+}
 
 // Launch size of a pass of length n (compiled kernels ignore it): the EG of
-// the kernels that serve it, plus kColLongTile for dense column kernels in
-// tiles of kTileLong columns.
+// the kernels that serve it, plus kColLongTile for dense column kernels above
+// 256, in tiles of kTileLong columns.
 int emax_for(int n, bool column) {
-    if (dense_length(n)) return kEgDense + 16 + (column && col_tile(n) == kTileLong ? kColLongTile : 0);
+    if (dense_length(n)) {
+        if (column && n > 256) return kEgDense + 16 + kColLongTile;
+        return kEgDense + (column && col_tile(n) == kTileLong ? 8 : 16);
+    }
     return column ? 32 : 16;
 }
 
