@@ -76,7 +76,7 @@ def alg_bytes(dims):
         16 * Nh,           # read + write half spectrum
         24 * Nh,           # spectrum r/w (16Nh) + f^ (8Nh); rho*inv_a/N is formed in-kernel
         16 * Nh,
-        8 * Nh + 8 * N,    # read spectrum + x_prev, write x
+        8 * Nh + 4 * N,    # read spectrum, write x (tol 0: x_prev is read in the last iteration only)
     ]
 
 

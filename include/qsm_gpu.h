@@ -162,7 +162,7 @@ const char* qsm_last_error_message(void);
 int qsm_backend_info(char* buf, size_t len);
 /* 1 if n is an axis length the GPU FFT supports, else 0: n <= 1024 factoring
  * into 2, 3, 5, 7, 11, 13, or any n <= 512 (a prime factor above 13 runs as a
- * chirp-z transform).  The reference (rustfft) transforms any length. */
+ * dense DFT factor, above 256 as a chirp-z transform).  The reference (rustfft) transforms any length. */
 int qsm_fft_length_supported(size_t n);
 
 /* ---- drop-in algorithm entry points (host pointers) -------------------- */
