@@ -12,9 +12,10 @@
  * failure on the calling thread.  Progress callbacks run on the calling
  * thread with exactly the reference's (current, total) sequence.
  *
- * Host-pointer entry points allocate their device memory per call.  The
- * batch entry points (qsm_tv_batch_*) take device pointers, keep their
- * workspace between runs and are the throughput path.
+ * Host-pointer entry points take their device memory per call, from what
+ * finished calls left (qsm_release_cached_memory).  The batch entry points
+ * (qsm_tv_batch_*) take device pointers, keep their workspace between runs and
+ * are the throughput path.
  */
 #ifndef QSM_GPU_H
 #define QSM_GPU_H
@@ -313,8 +314,10 @@ int qsm_memcpy_dtod(void* dst, const void* src, size_t bytes);
 int qsm_device_synchronize(void);
 /* The library keeps device workspaces (at most 2 GiB over all devices),
  * streams and pinned staging buffers (at most 16 MiB a device) of finished
- * calls for later ones; they are given back when the device runs out of
- * memory, and by this call. */
+ * calls for later ones.  They are given back when a call of this library
+ * finds no memory left (it then tries again), and by this call.  Other
+ * allocators do not see them: a program that needs the whole device for
+ * another library, or another process, calls this first. */
 void qsm_release_cached_memory(void);
 /* Achievable HBM rate reference: a one-element-per-thread device copy of
  * `bytes`, read + write counted, best of `reps` launches (GB/s). */

@@ -87,10 +87,10 @@ hipError_t lane_take(int dev, Lane& out) {
     }
     Lane l;
     l.dev = dev;
-    hipError_t e = hipStreamCreateWithFlags(&l.stream, hipStreamNonBlocking);
+    hipError_t e = with_trim([&] { return hipStreamCreateWithFlags(&l.stream, hipStreamNonBlocking); });
     if (e != hipSuccess) l.stream = nullptr;
     for (int i = 0; i < 2 && e == hipSuccess; ++i) {
-        e = hipHostMalloc((void**)&l.buf[i], kChunk, hipHostMallocDefault);
+        e = with_trim([&] { return hipHostMalloc((void**)&l.buf[i], kChunk, hipHostMallocDefault); });
         if (e != hipSuccess) l.buf[i] = nullptr;
         if (e == hipSuccess) {
             e = hipEventCreateWithFlags(&l.ev[i], hipEventDisableTiming);
@@ -230,12 +230,7 @@ hipError_t workspace_alloc(void** p, size_t bytes) {
             return hipSuccess;
         }
     }
-    e = hipMalloc(p, want);
-    if (e == hipErrorOutOfMemory) {
-        (void)hipGetLastError();
-        workspace_trim();
-        e = hipMalloc(p, want);
-    }
+    e = with_trim([&] { return hipMalloc(p, want); });
     if (e != hipSuccess) {
         *p = nullptr;
         return e;
@@ -306,7 +301,7 @@ hipError_t stream_take(hipStream_t* out) {
                 return hipSuccess;
             }
     }
-    e = hipStreamCreateWithFlags(out, hipStreamNonBlocking);
+    e = with_trim([&] { return hipStreamCreateWithFlags(out, hipStreamNonBlocking); });
     if (e != hipSuccess) {
         *out = nullptr;
         return e;
@@ -341,7 +336,9 @@ hipError_t pinned_take(void** p) {
             return hipSuccess;
         }
     }
-    const hipError_t e = hipHostMalloc(p, kPinnedBlock, hipHostMallocMapped | hipHostMallocCoherent | hipHostMallocPortable);
+    const hipError_t e = with_trim([&] {
+        return hipHostMalloc(p, kPinnedBlock, hipHostMallocMapped | hipHostMallocCoherent | hipHostMallocPortable);
+    });
     if (e != hipSuccess) *p = nullptr;
     return e;
 }

@@ -13,13 +13,27 @@ namespace qsm {
 // devices, the least recently freed go back first) and handed to a later
 // request of about its size on the same device.  The caller frees a block
 // only after it has waited for the work that uses it, so a kept block is idle
-// and any stream or thread may have it.  When the device has no memory left
-// the kept blocks are given back and the request is tried again.
+// and any stream or thread may have it.
 constexpr size_t kWorkspaceKept = (size_t)2 << 30;
 hipError_t workspace_alloc(void** p, size_t bytes);
 void workspace_free(void* p);
 // Gives every kept block, stream and pinned block back.
 void workspace_trim();
+
+// Runs a call that takes device or pinned memory.  Where it finds none left,
+// everything kept is given back and the call made once more, so that no call
+// of this library fails for want of memory that the library itself holds idle.
+// A failure that remains is the returned one only: HIP's last error, which the
+// next launch check would read, is cleared.
+template <class F>
+hipError_t with_trim(F&& call) {
+    hipError_t e = call();
+    if (e != hipErrorOutOfMemory) return e;
+    (void)hipGetLastError();
+    workspace_trim();
+    if ((e = call()) != hipSuccess) (void)hipGetLastError();
+    return e;
+}
 
 // A non-blocking stream of default priority, and back once it is idle.
 hipError_t stream_take(hipStream_t* s);

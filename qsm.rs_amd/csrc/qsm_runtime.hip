@@ -849,7 +849,8 @@ static int build_iteration_graphs(qsm_tv_batch* B) {
         hipGraph_t g = nullptr;
         const hipError_t e = hipStreamEndCapture(B->stream, &g);
         hipError_t ei = hipSuccess;
-        if (!rc && e == hipSuccess && g) ei = hipGraphInstantiate(&B->gexec[s], g, nullptr, nullptr, 0);
+        if (!rc && e == hipSuccess && g)
+            ei = with_trim([&] { return hipGraphInstantiate(&B->gexec[s], g, nullptr, nullptr, 0); });
         if (g) (void)hipGraphDestroy(g);
         if (rc) return rc;
         if (e != hipSuccess || !g || ei != hipSuccess) {
@@ -2238,7 +2239,12 @@ int qsm_device_alloc(size_t bytes, void** out) {
     g_err.clear();
     if (!out) return fail(QSM_EPARAM, "null output pointer");
     *out = nullptr;
-    QSM_HIP(hipMalloc(out, bytes ? bytes : 1));
+    const hipError_t e = with_trim([&] { return hipMalloc(out, bytes ? bytes : 1); });
+    if (e != hipSuccess) {
+        *out = nullptr;
+        return fail(e == hipErrorOutOfMemory ? QSM_ENOMEM : QSM_EHIP, "hipMalloc(%zu bytes): %s", bytes,
+                    hipGetErrorString(e));
+    }
     return QSM_OK;
 }
 

@@ -1,0 +1,178 @@
+// The library on a device that has no memory left.  This program defines the HIP calls that the library makes, so that
+// they end here and not in the runtime: memory is counted against a capacity
+// that the test sets, kernels do nothing.  No GPU is used.
+#include "qsm_gpu.h"
+
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <map>
+
+namespace {
+
+enum { kSuccess = 0, kOutOfMemory = 2 };
+constexpr size_t kMiB = (size_t)1 << 20, kStreamCost = kMiB, kGraphCost = kMiB;
+// (function-local, never destroyed: the library may free after main)
+struct Device {
+    size_t capacity = ~(size_t)0, used = 0, uploaded = 0;
+    std::map<void*, size_t> blocks;
+    int last_error = kSuccess, graph_launches = 0;
+    long next_id = 1;
+};
+Device& dev() {
+    static Device* d = new Device();
+    return *d;
+}
+bool charge(size_t bytes) {
+    Device& d = dev();
+    if (d.capacity - d.used < bytes) {
+        d.last_error = kOutOfMemory;
+        return false;
+    }
+    d.used += bytes;
+    return true;
+}
+void fill_up() { dev().capacity = dev().used; }
+
+int failures = 0;
+void check(bool ok, const char* what) {
+    std::printf("%s: %s\n", what, ok ? "ok" : "FAIL");
+    if (!ok) {
+        std::printf("  last message: %s\n", qsm_last_error_message());
+        ++failures;
+    }
+}
+
+}  // namespace
+
+struct Dim3 {
+    unsigned x, y, z;
+};
+extern "C" {
+int hipGetDevice(int* d) { *d = 0; return kSuccess; }
+int hipGetLastError() {
+    const int e = dev().last_error;
+    dev().last_error = kSuccess;
+    return e;
+}
+const char* hipGetErrorString(int e) { return e == kOutOfMemory ? "out of memory" : e ? "error" : "no error"; }
+int hipMalloc(void** p, size_t n) {
+    if (!charge(n)) return kOutOfMemory;
+    *p = reinterpret_cast<void*>(((size_t)1 << 40) + kMiB * 1024 * (size_t)dev().next_id++);
+    dev().blocks[*p] = n;
+    return kSuccess;
+}
+int hipFree(void* p) {
+    auto it = dev().blocks.find(p);
+    if (it == dev().blocks.end()) return 1;
+    dev().used -= it->second;
+    dev().blocks.erase(it);
+    return kSuccess;
+}
+int hipHostMalloc(void** p, size_t n, unsigned) { *p = std::calloc(n, 1); return *p ? kSuccess : kOutOfMemory; }
+int hipHostFree(void* p) { std::free(p); return kSuccess; }
+int hipHostGetDevicePointer(void** d, void* h, unsigned) { *d = h; return kSuccess; }
+int hipStreamCreateWithFlags(void** s, unsigned) {
+    if (!charge(kStreamCost)) return kOutOfMemory;
+    *s = reinterpret_cast<void*>(dev().next_id++);
+    return kSuccess;
+}
+int hipStreamDestroy(void*) { dev().used -= kStreamCost; return kSuccess; }
+int hipStreamSynchronize(void*) { return kSuccess; }
+int hipStreamWaitEvent(void*, void*, unsigned) { return kSuccess; }
+int hipStreamIsCapturing(void*, int* s) { *s = 0; return kSuccess; }
+int hipStreamBeginCapture(void*, int) { return kSuccess; }
+int hipStreamEndCapture(void*, void** g) { *g = reinterpret_cast<void*>(dev().next_id++); return kSuccess; }
+int hipGraphInstantiate(void** x, void*, void**, char*, size_t) {
+    if (!charge(kGraphCost)) return kOutOfMemory;
+    *x = reinterpret_cast<void*>(dev().next_id++);
+    return kSuccess;
+}
+int hipGraphDestroy(void*) { return kSuccess; }
+int hipGraphExecDestroy(void*) { dev().used -= kGraphCost; return kSuccess; }
+int hipGraphLaunch(void*, void*) { ++dev().graph_launches; return kSuccess; }
+int hipEventCreate(void** e) { *e = reinterpret_cast<void*>(dev().next_id++); return kSuccess; }
+int hipEventCreateWithFlags(void** e, unsigned) { return hipEventCreate(e); }
+int hipEventDestroy(void*) { return kSuccess; }
+int hipEventRecord(void*, void*) { return kSuccess; }
+int hipEventSynchronize(void*) { return kSuccess; }
+int hipEventElapsedTime(float* ms, void*, void*) { *ms = 1.0f; return kSuccess; }
+int hipDeviceSynchronize() { return kSuccess; }
+int hipMemcpy(void*, const void*, size_t n, int) { dev().uploaded += n; return kSuccess; }
+int hipMemcpyAsync(void*, const void*, size_t n, int, void*) { dev().uploaded += n; return kSuccess; }
+int hipLaunchKernel(const void*, Dim3, Dim3, void**, size_t, void*) { return kSuccess; }
+int __hipPushCallConfiguration(Dim3, Dim3, size_t, void*) { return kSuccess; }
+int __hipPopCallConfiguration(Dim3* g, Dim3* b, size_t* n, void** s) {
+    *g = *b = Dim3{1, 1, 1};
+    *n = 0;
+    *s = nullptr;
+    return kSuccess;
+}
+}
+
+namespace {
+
+double* fake(size_t i) { return reinterpret_cast<double*>(((size_t)1 << 36) + i * kMiB * 64); }
+void* const kUserStream = reinterpret_cast<void*>((size_t)77);
+const double kZ[3] = {0.0, 0.0, 1.0};
+
+// Two idle blocks of 32 MiB in the pool.
+void fill_pool() {
+    qsm_release_cached_memory();
+    dev().capacity = ~(size_t)0;
+    double gbps = 0.0;
+    check(qsm_hbm_copy_probe(32 * kMiB, 1, &gbps) == QSM_OK, "probe");
+}
+
+void device_memory() {
+    void* p = nullptr;
+    fill_pool();
+    const size_t kept = dev().used;
+    check(kept >= 64 * kMiB, "a finished call's blocks are kept");
+    fill_up();
+    check(qsm_device_alloc(48 * kMiB, &p) == QSM_OK && p, "an allocation that needs the kept blocks");
+    check(qsm_device_free(p) == QSM_OK && dev().used == 0, "freed");
+
+    fill_pool();
+    fill_up();
+    p = fake(1);
+    check(qsm_device_alloc(kept + kMiB, &p) == QSM_ENOMEM && !p, "an allocation beyond the device");
+    const qsm_grid g = {16, 16, 16, 1.0, 1.0, 1.0};
+    check(qsm_dipole_forward(fake(0), &g, kZ, fake(1), kUserStream) == QSM_OK, "the call after it");
+
+    // a stream of the library's own, beside the blocks that the call takes over
+    fill_pool();
+    check(qsm_dipole_forward(fake(0), &g, kZ, fake(1), kUserStream) == QSM_OK, "on the caller's stream");
+    fill_up();
+    check(qsm_dipole_forward(fake(0), &g, kZ, fake(1), nullptr) == QSM_OK, "on a stream that needs the kept blocks");
+
+    fill_pool();
+    qsm_tv_volume v = {};
+    v.grid = g;
+    v.bdir[2] = 1.0;
+    v.d_field = fake(0);
+    v.d_mask = reinterpret_cast<uint8_t*>(fake(1));
+    v.d_chi = fake(2);
+    const qsm_tv_params prm = {1e-3, 0.1, 0.0, 6};
+    qsm_tv_batch* b = nullptr;
+    check(qsm_tv_batch_create(&v, 1, &prm, nullptr, &b) == QSM_OK, "batch");
+    fill_up();
+    check(qsm_tv_batch_run(b, nullptr, nullptr) == QSM_OK && dev().graph_launches == 4,
+          "graphs that need the kept blocks");
+    qsm_tv_batch_destroy(b);
+    dev().capacity = ~(size_t)0;
+    qsm_release_cached_memory();
+    check(dev().used == 0, "everything given back");
+}
+
+}  // namespace
+
+int main(int argc, char** argv) {
+    if (argc == 2 && !std::strcmp(argv[1], "device")) {
+        device_memory();
+    } else {
+        return 2;
+    }
+    std::printf(failures ? "FAILED\n" : "ALL OK\n");
+    return failures ? 1 : 0;
+}

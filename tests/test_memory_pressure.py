@@ -1,0 +1,28 @@
+"""The library where memory runs out: what it keeps between calls is given back
+before a call of its own fails on the device.  HIP is replaced by the test
+program; no GPU is used."""
+import os
+import subprocess
+
+import pytest
+
+from conftest import PKG_DIR, ROOT
+
+
+@pytest.fixture(scope="module")
+def exe(tmp_path_factory):
+    out = tmp_path_factory.mktemp("memory") / "memory_test"
+    subprocess.run(["g++", "-std=c++17", "-O1", "-rdynamic", "-I", os.path.join(ROOT, "include"),
+                    os.path.join(ROOT, "tests", "native", "memory_test.cpp"), "-L", PKG_DIR, "-lqsm_gpu",
+                    "-Wl,-rpath," + PKG_DIR, "-o", str(out)], check=True)
+    return str(out)
+
+
+def _run(exe, *args):
+    r = subprocess.run([exe, *args], capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0 and "ALL OK" in r.stdout, r.stdout[-2000:] + r.stderr[-500:]
+    return r.stdout
+
+
+def test_kept_memory_is_given_back_to_own_calls(exe):
+    _run(exe, "device")
