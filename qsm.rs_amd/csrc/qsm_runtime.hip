@@ -138,20 +138,22 @@ const std::vector<float2>& fft_table(int kind, int n) {
     static std::mutex mu;
     static std::map<std::pair<int, int>, std::vector<float2>> tab;
     std::lock_guard<std::mutex> lk(mu);
-    std::vector<float2>& t = tab[{kind, n}];  // (references stay valid as the map grows)
-    if (t.empty()) {
-        if (kind == 0) {
-            for (int q = 0; q < n; ++q) t.push_back(twiddle_entry(q, n));
-        } else if (kind == 1) {
-            t.resize(qsmfft::dense_table_len(n));
-            qsmfft::dense_table(n, t.data());
-        } else {
-            std::vector<float2> f;
-            chirp_tables(n, chirp_length(n), t, f);
-            t.insert(t.end(), f.begin(), f.end());
-        }
+    auto it = tab.find({kind, n});
+    if (it != tab.end()) return it->second;
+    // formed whole before it is kept: a host allocation may fail on the way
+    std::vector<float2> t;
+    if (kind == 0) {
+        t.reserve(n);
+        for (int q = 0; q < n; ++q) t.push_back(twiddle_entry(q, n));
+    } else if (kind == 1) {
+        t.resize(qsmfft::dense_table_len(n));
+        qsmfft::dense_table(n, t.data());
+    } else {
+        std::vector<float2> f;
+        chirp_tables(n, chirp_length(n), t, f);
+        t.insert(t.end(), f.begin(), f.end());
     }
-    return t;
+    return tab.emplace(std::make_pair(kind, n), std::move(t)).first->second;  // (stays valid as the map grows)
 }
 
 // The tables of the lengths of a set of volumes, end to end.

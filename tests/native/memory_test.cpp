@@ -1,4 +1,5 @@
-// The library on a device that has no memory left.  This program defines the HIP calls that the library makes, so that
+// The library on a device that has no memory left, and on a host that has
+// none.  This program defines the HIP calls that the library makes, so that
 // they end here and not in the runtime: memory is counted against a capacity
 // that the test sets, kernels do nothing.  No GPU is used.
 #include "qsm_gpu.h"
@@ -6,7 +7,9 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <initializer_list>
 #include <map>
+#include <new>
 
 namespace {
 
@@ -43,7 +46,18 @@ void check(bool ok, const char* what) {
     }
 }
 
+long alloc_countdown = -1;  // host allocations until one fails; -1: none does
+
 }  // namespace
+
+void* operator new(size_t n) {
+    if (alloc_countdown > 0 && --alloc_countdown == 0) throw std::bad_alloc();
+    void* p = std::malloc(n ? n : 1);
+    if (!p) throw std::bad_alloc();
+    return p;
+}
+void operator delete(void* p) noexcept { std::free(p); }
+void operator delete(void* p, size_t) noexcept { std::free(p); }
 
 struct Dim3 {
     unsigned x, y, z;
@@ -165,11 +179,32 @@ void device_memory() {
     check(dev().used == 0, "everything given back");
 }
 
+// Bytes that a first call with axes of length n sends: the descriptor and the
+// FFT tables.  With fail > 0 that call's fail-th host allocation fails first.
+size_t table_upload(size_t n, long fail) {
+    const qsm_grid g = {n, n, n, 1.0, 1.0, 1.0};
+    if (fail > 0) {
+        alloc_countdown = fail;
+        try {
+            (void)qsm_dipole_forward(fake(0), &g, kZ, fake(1), kUserStream);
+        } catch (const std::bad_alloc&) {
+        }
+        alloc_countdown = -1;
+    }
+    dev().uploaded = 0;
+    check(qsm_dipole_forward(fake(0), &g, kZ, fake(1), kUserStream) == QSM_OK, "dipole");
+    return dev().uploaded;
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
     if (argc == 2 && !std::strcmp(argv[1], "device")) {
         device_memory();
+    } else if (argc == 3 && !std::strcmp(argv[1], "tables")) {
+        // lengths of every kind of table: register radices, dense, chirp-z
+        const long fail = std::atol(argv[2]);
+        for (size_t n : {40, 64, 82, 121, 263}) std::printf("upload %zu %zu\n", n, table_upload(n, fail));
     } else {
         return 2;
     }

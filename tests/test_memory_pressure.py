@@ -1,6 +1,7 @@
 """The library where memory runs out: what it keeps between calls is given back
-before a call of its own fails on the device.  HIP is replaced by the test
-program; no GPU is used."""
+before a call of its own fails on the device, and a host allocation that fails
+while a table is formed leaves no part of it behind.  HIP is replaced by the
+test program; no GPU is used."""
 import os
 import subprocess
 
@@ -26,3 +27,12 @@ def _run(exe, *args):
 
 def test_kept_memory_is_given_back_to_own_calls(exe):
     _run(exe, "device")
+
+
+# The allocations of a call come in this order: the volume's descriptor and
+# tables one axis at a time, each table growing in steps; 40 covers them all
+# for the shortest length and the tables of the longest.
+def test_table_whole_after_failed_allocation(exe):
+    want = _run(exe, "tables", "0")
+    for k in range(1, 41):
+        assert _run(exe, "tables", str(k)) == want, k
