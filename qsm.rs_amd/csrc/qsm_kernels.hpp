@@ -1172,8 +1172,11 @@ __device__ __forceinline__ void fill_tvdiv_any(float2* lds, const VolDesc& V, in
                 oy[e] = tv_clamp(vy, t);
                 oz[e] = tv_clamp(vz, t);
                 gy[e] = tv_g(vy, oy[e]);
-                d[e] = (gx[e] - (e > 0 ? gx[e > 0 ? e - 1 : 0] : gl)) * hx + (gy[e] - gym[e]) * hy +
-                       (tv_g(vz, oz[e]) - tv_gv(vzm, t)) * hz;
+                // (the products' rounding is spelled out: the copies of this row
+                // step, of which a row takes either by the rows of its block,
+                // contracted the sum differently)
+                const float dx = gx[e] - (e > 0 ? gx[e > 0 ? e - 1 : 0] : gl), dy = gy[e] - gym[e];
+                d[e] = fmaf(tv_g(vz, oz[e]) - tv_gv(vzm, t), hz, fmaf(dx, hx, dy * hy));
                 gym[e] = gy[e];
             }
             if (own) {

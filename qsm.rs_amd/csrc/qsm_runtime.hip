@@ -14,6 +14,7 @@
 #include <cstring>
 #include <atomic>
 #include <map>
+#include <numeric>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -260,19 +261,79 @@ static int default_rows_x(int nx) {
     return std::max(1, std::min(32, tile / work_length(nx)));
 }
 
-// xshift / cshift 2 (compiled and dense lengths): the R2C / TV C2R passes take a
-// quarter of their default rows per block, as the kernels launched with
-// PassArgs::xshift = 2 do (C2R: half the R2C pass's rows before its shift).
-PassBlocks fill_geometry(VolDesc& V, const qsm_grid& g, TwiddleBank& tb, int xshift = 0, int cshift = 0) {
+// Rows per block (pair-rows, or rows of the V-SHARP selection) of the x passes
+// of a dense length other than the TV C2R pass, for a launch over `rows` of
+// them.  As few as fill the launch's rounds of resident blocks (kRowBlocks: 148
+// registers leave three a CU): long blocks leave CUs idle, many short ones pay
+// for their start.  R2C pass at 20 columns and 20160 pair-rows 18 us with 28
+// rows, 20 with 32, 26 with 8; at 143 columns and 6912 pair-rows 22 us with 10
+// rows, 29 with 28 or 6; at 338 and 1536, 18 us with 2, 27 with 12.  With a dense
+// radix, where every CU still has a block, whole matrix tiles of 16 butterflies
+// if others were padded by more than an eighth (R2C pass at 239 columns and 6912
+// pair-rows: 40 us with 16 rows, 44 with 10, 69 with 4), else half a tile at
+// least (251 and 1536: 25 us with 8, 31 with 2).
+//
+// single: passes whose threads take single elements (all but the TV ones, whose
+// fill works row by row): two for each thread at least (V-SHARP of 12x144x96:
+// 177 us with 32 rows, 190 with 12); with a dense radix full blocks, which share
+// the coefficients among most rows, where there are 1.5 for every CU (356x144x96:
+// 593 us with 10 rows, 657 with 8; 398x64x48, 300 blocks: 457 with 10, 345 with 6).
+// The rows change no bit of any value.
+constexpr size_t kCus = 256, kRowBlocks = 3 * kCus;
+// The largest dense radix of a length in fft_dense.hpp's stages, 0: none.
+static int dense_radix(int n) {
+    int r[qsmfft::kMaxStages], st = 0;
+    return qsmfft::dense_factorize(n, r, &st) && st && r[0] > qsmfft::kMaxRegRadix ? r[0] : 0;  // (the largest comes first)
+}
+static int dense_rows_x(int n, size_t rows, bool single) {
+    const size_t most = default_rows_x(n) & ~1, rounds = (rows + kRowBlocks * most - 1) / (kRowBlocks * most);
+    const size_t least = single ? (2 * qsmfft::kThreads + n - 1) / n : 2;
+    const auto even = [](size_t k) { return (k + 1) & ~(size_t)1; };  // the same rows for each of the fill's four waves
+    size_t per = even(std::max((rows + kRowBlocks * rounds - 1) / (kRowBlocks * rounds), least));
+    if (const int R = dense_radix(n)) {
+        if (single && 2 * rows >= 3 * kCus * most) return (int)most;
+        const size_t nb = n / R, whole = 16 / std::gcd((size_t)16, nb), used = nb * per;
+        const size_t full = whole > most ? most
+                                         : std::min(std::max(whole, (per + whole / 2) / whole * whole), most / whole * whole);
+        if (rows < kCus * full) per = even(std::max(per, (8 + nb - 1) / nb));
+        else if (9 * used < 8 * ((used + 15) / 16 * 16)) per = even(full);  // (padded by more than an eighth)
+    }
+    return (int)std::min(per, most);
+}
+static size_t pair_rows(const qsm_grid& g) { return (g.ny * g.nz + 1) / 2; }
+
+// Pair-rows of the volumes of each x length, which share a launch.
+template <class VOLS>
+static std::map<size_t, size_t> length_pairs(const VOLS* vols, size_t n_vols) {
+    std::map<size_t, size_t> pairs;
+    for (size_t v = 0; v < n_vols; ++v) pairs[vols[v].grid.nx] += pair_rows(vols[v].grid);
+    return pairs;
+}
+
+// rows, single: for dense lengths, see dense_rows_x.  xshift / cshift 2
+// (compiled lengths): the R2C / TV C2R passes take a quarter of their default
+// rows per block, as the kernels launched with PassArgs::xshift = 2 do (C2R:
+// half the R2C pass's rows before its shift).
+PassBlocks fill_geometry(VolDesc& V, const qsm_grid& g, TwiddleBank& tb, size_t rows, bool single,
+                         int xshift = 0, int cshift = 0) {
     V.nx = (int)g.nx; V.ny = (int)g.ny; V.nz = (int)g.nz;
     V.nxh = (V.nx + 1) / 2;  // even nx: DC and Nyquist share column 0
-    V.rows_x = has_fixed_kernels(V.nx) ? qsmfft::shifted_rows(V.nx, xshift) : default_rows_x(V.nx) >> xshift;
-    if (dense_length(V.nx) && V.rows_x > 2) V.rows_x &= ~1;  // the same rows for each of the fill's four waves
-    // compiled and dense C2R kernels take half the R2C pass's pair-rows (the
-    // previous iterate stays in registers across the transform); the
-    // runtime-plan one its whole tile, whose 8 elements per thread cover it
-    V.rows_c = has_fixed_kernels(V.nx) || dense_length(V.nx) ? std::max(1, (default_rows_x(V.nx) >> cshift) / 2)
-                                                             : default_rows_x(V.nx);
+    if (has_fixed_kernels(V.nx)) V.rows_x = qsmfft::shifted_rows(V.nx, xshift);
+    else V.rows_x = dense_length(V.nx) ? dense_rows_x(V.nx, rows, single) : default_rows_x(V.nx);
+    // compiled C2R kernels take half the R2C pass's pair-rows (the previous
+    // iterate stays in registers across the transform), the others what their
+    // tile of 8 elements per thread holds (fewer did not pay: 9 us with 12 to 32
+    // rows, 16 with 4, at 20 columns and 6912 pair-rows), but with a dense radix
+    // no more than leave every CU a block (82 columns, 1536 pair-rows: 10.9 us
+    // with 4, 12.7 with 24).  The sums of the relative change follow these
+    // blocks, so they depend on the volume's own shape only.
+    if (has_fixed_kernels(V.nx)) {
+        V.rows_c = std::max(1, (default_rows_x(V.nx) >> cshift) / 2);
+    } else {
+        V.rows_c = std::max(1, std::min(32, qsmfft::kThreads * kRowEmaxRt / work_length(V.nx)));
+        if (dense_length(V.nx) && dense_radix(V.nx))
+            V.rows_c = std::min(V.rows_c, (int)std::max<size_t>(4, (pair_rows(g) + kCus - 1) / kCus));
+    }
     V.ntx = (V.nxh + kTile - 1) / kTile;
     V.ntx_long = (V.nxh + kTileLong - 1) / kTileLong;
     V.m_nx = qsmfft::magic_for((uint32_t)V.nx);
@@ -284,7 +345,7 @@ PassBlocks fill_geometry(VolDesc& V, const qsm_grid& g, TwiddleBank& tb, int xsh
     V.vsx = g.vsx; V.vsy = g.vsy; V.vsz = g.vsz;
     V.hx = (float)(1.0 / g.vsx); V.hy = (float)(1.0 / g.vsy); V.hz = (float)(1.0 / g.vsz);
     PassBlocks pb;
-    const int npairs = (V.ny * V.nz + 1) / 2;
+    const int npairs = (int)pair_rows(g);
     pb.xpass = (npairs + V.rows_x - 1) / V.rows_x;
     pb.cpass = (npairs + V.rows_c - 1) / V.rows_c;
     pb.ypass = (col_tile(V.ny) == kTile ? V.ntx : V.ntx_long) * V.nz;
@@ -546,7 +607,8 @@ static int tune_column_schedules(qsm_tv_batch* B) {
 // rts != null selects RTS: its rho, tol, max_iter replace params' (params
 // may then be null).
 // io: the host entry points' one volume, whose field and output are f32 on the
-// device (the volume's own d_field and d_chi are then null).
+// device (the volume's own d_field and d_chi are then null).  unrolled: the
+// batch of an unrolled solver.
 struct HostVolume {
     float* field = nullptr;
     float* chi = nullptr;
@@ -556,7 +618,7 @@ struct HostVolume {
 };
 static int tv_batch_create_impl(const qsm_tv_volume* vols, size_t n_vols, const qsm_tv_params* params_in,
                                 void* stream, qsm_tv_batch** out, const qsm_rts_params* rts = nullptr,
-                                const HostVolume* io = nullptr) {
+                                const HostVolume* io = nullptr, bool unrolled = false) {
     qsm_tv_params rts_as_tv{};
     if (rts) {
         if (!(rts->rho > 0) || std::isnan(rts->delta) || std::isnan(rts->mu))
@@ -590,7 +652,7 @@ static int tv_batch_create_impl(const qsm_tv_volume* vols, size_t n_vols, const 
     TwiddleBank tb;
     std::vector<int> lx, ly, lz, bx, bc, by, bz, bo;
     auto cleanup = [&](int rc) { batch_free(B); return rc; };
-    // A small volume of a compiled or dense x length, whose R2C pass would launch
+    // A small volume of a compiled x length, whose R2C pass would launch
     // fewer than 1024 blocks (128 for 128x128x64 against ~768 resident), runs
     // that pass with a quarter of the rows per block, and its TV C2R pass
     // likewise, where either keeps at least 4 pair-rows per block (fewer made
@@ -600,11 +662,14 @@ static int tv_batch_create_impl(const qsm_tv_volume* vols, size_t n_vols, const 
     std::vector<int> xshift(n_vols), cshift(n_vols);
     for (size_t v = 0; v < n_vols; ++v) {
         const int nx = (int)vols[v].grid.nx, r0 = default_rows_x(nx), rc = std::max(1, r0 / 2);
-        const long npairs = ((long)vols[v].grid.ny * (long)vols[v].grid.nz + 1) / 2;
-        const bool fixed = has_fixed_kernels(nx) || dense_length(nx);
+        const long npairs = (long)pair_rows(vols[v].grid);
+        const bool fixed = has_fixed_kernels(nx);
         xshift[v] = (fixed && (npairs + r0 - 1) / r0 < 1024 && (r0 >> 2) >= 4) ? 2 : 0;
         cshift[v] = (fixed && (npairs + rc - 1) / rc < 1024 && (r0 >> 2) / 2 >= 4) ? 2 : 0;
     }
+    // The unrolled solver sums the threshold's gradient block by block, so its
+    // rows are chosen by the volume's own shape, 8 a block or more.
+    std::map<size_t, size_t> pairs = length_pairs(vols, n_vols);
     // (the quarter-row R2C pass has no non-temporal form: three 192x192x128
     // volumes, 566 MB, took 203 us an iteration, 205 with the other passes' forms)
     size_t voxels = 0;
@@ -614,7 +679,8 @@ static int tv_batch_create_impl(const qsm_tv_volume* vols, size_t n_vols, const 
     for (size_t v = 0; v < n_vols; ++v) {
         VolDesc& V = B->h[v];
         std::memset(&V, 0, sizeof V);
-        PassBlocks pb = fill_geometry(V, vols[v].grid, tb, xshift[v], cshift[v]);
+        const size_t rows = unrolled ? std::max(pair_rows(vols[v].grid), 8 * kRowBlocks) : pairs[vols[v].grid.nx];
+        PassBlocks pb = fill_geometry(V, vols[v].grid, tb, rows, false, xshift[v], cshift[v]);
         const double* b = vols[v].bdir;
         double bn = std::sqrt(b[0] * b[0] + b[1] * b[1] + b[2] * b[2]);
         V.bx = b[0] / bn; V.by = b[1] / bn; V.bz = b[2] / bn;  // src/kernels/dipole.rs:39-43
@@ -1053,7 +1119,7 @@ static int unrolled_create_impl(const qsm_tv_volume* vols, size_t n_vols, const 
     qsm_tv_unrolled* U = new qsm_tv_unrolled();
     U->K = p.max_iter;
     auto cleanup = [&](int rc) { unrolled_free(U); return rc; };
-    int rc = tv_batch_create_impl(vols, n_vols, &p, stream, &U->B);
+    int rc = tv_batch_create_impl(vols, n_vols, &p, stream, &U->B, nullptr, nullptr, true);
     if (rc) return cleanup(rc);
     qsm_tv_batch* B = U->B;
     const size_t nrec = U->K > 1 ? U->K - 1 : 0;
@@ -1212,7 +1278,7 @@ static int spectral_apply(int zkind, int filt, double fa, const double* d_in, co
     VolDesc V;
     std::memset(&V, 0, sizeof V);
     TwiddleBank tb;
-    PassBlocks pb = fill_geometry(V, *grid, tb);
+    PassBlocks pb = fill_geometry(V, *grid, tb, pair_rows(*grid), true);
     V.bx = bdir[0] / bn; V.by = bdir[1] / bn; V.bz = bdir[2] / bn;
     V.field = d_in;
     V.adj_out = d_out;
@@ -1354,6 +1420,7 @@ static int vs_create_impl(const qsm_vsharp_volume* vols, size_t n_vols, const do
     B->h.resize(n_vols);
     TwiddleBank tb;
     std::vector<int> lx, ly, lz, bx, brows, by, by2, bz, bi;
+    std::map<size_t, size_t> pairs = length_pairs(vols, n_vols);
     int rc;
     if ((rc = dev_alloc(&B->d_radii, (size_t)R * (1 + n_vols)))) return cleanup(rc);
     B->allocs.push_back(B->d_radii);
@@ -1362,7 +1429,8 @@ static int vs_create_impl(const qsm_vsharp_volume* vols, size_t n_vols, const do
     for (size_t v = 0; v < n_vols; ++v) {
         VolDesc& V = B->h[v];
         std::memset(&V, 0, sizeof V);
-        PassBlocks pb = fill_geometry(V, vols[v].grid, tb);
+        // (the selection pass has twice as many rows as the others pair-rows)
+        PassBlocks pb = fill_geometry(V, vols[v].grid, tb, 2 * pairs[vols[v].grid.nx], true);
         V.field = vols[v].d_field;
         V.mask = vols[v].d_mask;
         V.out = vols[v].d_local;
@@ -1780,7 +1848,7 @@ int qsm_dipole_forward_noalloc(const double* d_chi, const qsm_grid* grid, const 
     VolDesc V;
     std::memset(&V, 0, sizeof V);
     TwiddleBank tb;
-    PassBlocks pb = fill_geometry(V, *grid, tb);
+    PassBlocks pb = fill_geometry(V, *grid, tb, pair_rows(*grid), true);
     const size_t spec_bytes = (size_t)V.nxh * V.ny * V.nz * sizeof(float2);
     if (spec_bytes > kScratchSpecBytes)
         return fail(QSM_EPARAM,
