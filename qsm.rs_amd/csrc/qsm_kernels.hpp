@@ -695,14 +695,16 @@ __host__ __device__ constexpr bool tvdiv_rows_form(int n, int rb) {
     return n > 0 && n <= 256 && rb >= 4;
 }
 
-// Columns per lane of the wave-row form (VW): 4 above 128 columns and 2 above
-// 64, one group of lanes for the row, so that every load and store moves 16 or
-// 8 bytes per lane.  Measured at 256, one column per lane against 2 and 4:
-// 277.9, 274.8 and 268.2 us per 4-volume launch; at 144 (three groups of 64
-// columns against 36 lanes of 4) 78.8 and 71.6 us for two 144x192x160 volumes,
-// at 160 81.4 and 79.0, at 176 91.7 and 88.1, at 192 the same.
+// Columns per lane of the wave-row form (VW): 4 above 128 columns and 2 from 66
+// to 128, one group of lanes for the row, so that every load and store moves 16
+// or 8 bytes per lane; 1 for other rows.  Measured at 256, one column per lane
+// against 2 and 4: 277.9, 274.8 and 268.2 us per 4-volume launch; at 144 (three
+// groups of 64 columns against 36 lanes of 4) 78.8 and 71.6 us for two
+// 144x192x160 volumes, at 160 81.4 and 79.0, at 176 91.7 and 88.1, at 192 the
+// same.  Two groups of 2 lose to three of 1 (150 columns: 142 registers against
+// 117, 23.2 us against 19.8 at 150x144x96).
 __host__ __device__ constexpr int tvdiv_rows_vw(int n) {
-    return n % 4 == 0 && n > 128 ? 4 : (n % 2 == 0 && n > 64 ? 2 : 1);
+    return n % 4 == 0 && n > 128 ? 4 : (n % 2 == 0 && n > 64 && n <= 128 ? 2 : 1);
 }
 
 template <int VW>
@@ -832,6 +834,7 @@ __device__ __forceinline__ void fill_tvdiv_rows(float2* lds, const VolDesc& V, i
     constexpr int C = TvRow<NX, VW>::C;
     constexpr int LV = (NX - G * (C - 1)) / VW;  // valid lanes of the last column group
     static_assert(kThreads == 256, "four waves per block");
+    static_assert(VW == 1 || C == 1, "several columns per lane: one group of lanes");
     const int ny = V.ny, nz = V.nz;
     const int nxy = NX * ny, N = nxy * nz;
     const float t = V.thr, hx = V.hx, hy = V.hy, hz = V.hz;
