@@ -840,10 +840,10 @@ __device__ __forceinline__ void fill_tvdiv_rows(float2* lds, const VolDesc& V, i
     const float t = V.thr, hx = V.hx, hy = V.hy, hz = V.hz;
     const int lane = (int)(threadIdx.x & 63);
     const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    // pair-rows [p0, p0 + nrw / 2) of this wave; the same count for every
-    // wave (a compile-time constant, so the row loop unrolls) when 4 | RB
-    const int p0 = (RB % 4 == 0) ? wv * (RB / 4) : (wv * RB) >> 2;
-    const int nrw = (RB % 4 == 0) ? RB / 2 : 2 * ((((wv + 1) * RB) >> 2) - p0);
+    // pair-rows [p0, p0 + nrw / 2) of this wave
+    static_assert(RB % 4 == 0, "the same rows for every wave");
+    const int p0 = wv * (RB / 4);
+    constexpr int nrw = RB / 2;
     const int r0 = row0 + 2 * p0;
     // plane and in-plane index of the wave's first row, then stepped
     int k = r0 / ny;
@@ -2352,9 +2352,9 @@ __device__ __forceinline__ void c2r_load_rows(float2* lds, const VolDesc& V, int
 // 119 instead of 179 for two 384x384x256 volumes.
 // MODE C2R_TV: as above.  C2R_ADJ: Re IFFT to adj_c (c-bar), nothing
 // else.  C2R_F64: Re IFFT widened to f64 into adj_out.
-// C2R_F64_MASKED: f64 into out, 0 where mask == 0 (src/utils/mask.rs:47-53).
-// C2R_X0: FP32 into x[0], 0 where mask == 0 (the RTS starting point).
-enum C2RMode : int { C2R_TV = 0, C2R_ADJ = 1, C2R_F64 = 2, C2R_F64_MASKED = 3, C2R_X0 = 4 };
+// C2R_X0: FP32 into x[0], 0 where mask == 0 (src/utils/mask.rs:47-53; the RTS
+// starting point, the closed-form inversions of host arrays).
+enum C2RMode : int { C2R_TV = 0, C2R_ADJ = 1, C2R_F64 = 2, C2R_X0 = 3 };
 
 template <int N, int EG, int MODE, int RBS = 0, bool NT = false>
 __global__ __launch_bounds__(kThreads) void k_c2r_tv(const VolDesc* __restrict__ vols, LaunchTable lt,
@@ -2397,18 +2397,12 @@ __global__ __launch_bounds__(kThreads) void k_c2r_tv(const VolDesc* __restrict__
                     QSM_GLOBAL float* __restrict__ o = glb(V.adj_c);
                     if (ra < nrows) o[i + (size_t)ra * nx] = z.x;
                     if (rb < nrows) o[i + (size_t)rb * nx] = z.y;
-                } else if constexpr (MODE == C2R_F64_MASKED || MODE == C2R_X0) {
+                } else if constexpr (MODE == C2R_X0) {
                     const QSM_GLOBAL uint8_t* __restrict__ m = glb(V.mask);
+                    QSM_GLOBAL float* __restrict__ o = glb(V.x[0]);
                     const size_t ia = i + (size_t)ra * nx, ib = i + (size_t)rb * nx;
-                    if constexpr (MODE == C2R_F64_MASKED) {
-                        QSM_GLOBAL double* __restrict__ o = glb(V.out);
-                        if (ra < nrows) o[ia] = m[ia] ? (double)z.x : 0.0;
-                        if (rb < nrows) o[ib] = m[ib] ? (double)z.y : 0.0;
-                    } else {
-                        QSM_GLOBAL float* __restrict__ o = glb(V.x[0]);
-                        if (ra < nrows) o[ia] = m[ia] ? z.x : 0.0f;
-                        if (rb < nrows) o[ib] = m[ib] ? z.y : 0.0f;
-                    }
+                    if (ra < nrows) o[ia] = m[ia] ? z.x : 0.0f;
+                    if (rb < nrows) o[ib] = m[ib] ? z.y : 0.0f;
                 } else {
                     QSM_GLOBAL double* __restrict__ o = glb(V.adj_out);
                     if (ra < nrows) o[i + (size_t)ra * nx] = (double)z.x;

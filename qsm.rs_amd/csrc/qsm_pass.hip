@@ -16,7 +16,7 @@ namespace qsm {
     return kind == P_R2C_TVDIV || kind == P_R2C_F64 || kind == P_R2C_U8 || kind == P_R2C_F32 ||
            kind == P_R2C_SPHERE || kind == P_C2R_TV || kind == P_C2R_VS_SELECT || kind == P_C2R_VS_OUT ||
            kind == P_R2C_TVDIV_REC || kind == P_R2C_TVADJ_FIRST || kind == P_R2C_TVADJ ||
-           kind == P_R2C_ACC || kind == P_C2R_ADJ || kind == P_C2R_F64OUT || kind == P_C2R_F64_MASKED ||
+           kind == P_R2C_ACC || kind == P_C2R_ADJ || kind == P_C2R_F64OUT ||
            kind == P_C2R_X0 || kind == P_R2C_X0 || kind == P_R2C_WRAPLAP || kind == P_R2C_TVDIV_W ||
            kind == P_R2C_NLTV_BND;
 }
@@ -57,7 +57,6 @@ static void launch_rows_s(int kind, const LaunchTable& lt, const PassArgs& a) {
             break;
         case P_C2R_ADJ: k_c2r_tv<N, EG, C2R_ADJ, RBS><<<g, b, 0, st>>>(a.vols, lt, a.tw, 0, nullptr, 0); break;
         case P_C2R_F64OUT: k_c2r_tv<N, EG, C2R_F64, RBS><<<g, b, 0, st>>>(a.vols, lt, a.tw, 0, nullptr, 0); break;
-        case P_C2R_F64_MASKED: k_c2r_tv<N, EG, C2R_F64_MASKED, RBS><<<g, b, 0, st>>>(a.vols, lt, a.tw, 0, nullptr, 0); break;
         case P_C2R_X0: k_c2r_tv<N, EG, C2R_X0, RBS><<<g, b, 0, st>>>(a.vols, lt, a.tw, 0, nullptr, 0); break;
         case P_R2C_X0: k_r2c_x<N, EG, SRC_X0, RBS><<<g, b, 0, st>>>(a.vols, lt, a.tw, a.sel, 0, nullptr, nullptr, nullptr, 0); break;
         case P_R2C_TVDIV_W:

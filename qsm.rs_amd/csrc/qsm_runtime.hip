@@ -1227,12 +1227,12 @@ static int unrolled_backward_impl(qsm_tv_unrolled* U, const double* const* d_chi
 // src/kernels/dipole.rs:24-72), device pointers, f64 in and out, FP32
 // transforms.  D is real and even after taking its Hermitian part, so the
 // operator is self-adjoint and the adjoint entry point runs the same passes.
-// zkind P_Z_DIPOLE (no mask, f64 out) or P_Z_FILTER (filter `filt` with
-// parameter `fa`, output masked by d_mask).
-// src_kind P_R2C_F64 (d_in as is) or P_R2C_WRAPLAP (masked wrapped
-// Laplacian of d_in); bdir may be null for filters that do not use D.
+// zkind P_Z_DIPOLE (d_in, d_out: f64 on the device, no mask) or P_Z_FILTER
+// (filter `filt` with parameter `fa`; hv: f32 field, mask and masked f32 output,
+// or the phase in d_in where src_kind is P_R2C_WRAPLAP, its masked wrapped
+// Laplacian); bdir may be null for filters that do not use D.
 // The five passes of one spectral round trip of a single volume: R2C of
-// src_kind, y, z pass zkind, inverse y, C2R to f64 (masked for filters).
+// src_kind, y, z pass zkind, inverse y, C2R pass out_kind.
 // Launch tables live on the stack.
 static void enqueue_round_trip(int src_kind, int zkind, int out_kind, const VolDesc& V, const PassBlocks& pb,
                                const VolDesc* d_vols, const float2* d_tw, hipStream_t st) {
@@ -1264,13 +1264,12 @@ static void enqueue_round_trip(int src_kind, int zkind, int out_kind, const VolD
     run(out_kind, V.nx, false, txc);
 }
 
-static int spectral_apply(int zkind, int filt, double fa, const double* d_in, const uint8_t* d_mask,
-                          const qsm_grid* grid, const double bdir_in[3], double* d_out, void* stream,
-                          int src_kind = P_R2C_F64, const HostVolume* hv = nullptr) {
+static int spectral_apply(int zkind, int filt, double fa, const double* d_in, const qsm_grid* grid,
+                          const double bdir_in[3], double* d_out, void* stream, int src_kind = P_R2C_F64,
+                          const HostVolume* hv = nullptr) {
     static const double z_axis[3] = {0.0, 0.0, 1.0};
     const double* bdir = bdir_in ? bdir_in : z_axis;
-    if (!hv && (!d_in || !grid || !d_out || (zkind == P_Z_FILTER && !d_mask)))
-        return fail(QSM_EPARAM, "null argument");
+    if (!hv && (!d_in || !grid || !d_out)) return fail(QSM_EPARAM, "null argument");
     int rc = validate_grid(grid);
     if (rc) return rc;
     const double bn = std::sqrt(bdir[0] * bdir[0] + bdir[1] * bdir[1] + bdir[2] * bdir[2]);
@@ -1282,8 +1281,6 @@ static int spectral_apply(int zkind, int filt, double fa, const double* d_in, co
     V.bx = bdir[0] / bn; V.by = bdir[1] / bn; V.bz = bdir[2] / bn;
     V.field = d_in;
     V.adj_out = d_out;
-    V.out = d_out;
-    V.mask = d_mask;
     if (hv) {
         V.vs_local = hv->field;
         V.mask = hv->mask;
@@ -1316,8 +1313,7 @@ static int spectral_apply(int zkind, int filt, double fa, const double* d_in, co
         if (e != hipSuccess) { st = nullptr; return done(fail(QSM_EHIP, "hipStreamCreate: %s", hipGetErrorString(e))); }
         own = true;
     }
-    enqueue_round_trip(src_kind, zkind, hv ? P_C2R_X0 : (zkind == P_Z_FILTER ? P_C2R_F64_MASKED : P_C2R_F64OUT), V,
-                       pb, d_vols, d_tw, st);
+    enqueue_round_trip(src_kind, zkind, hv ? P_C2R_X0 : P_C2R_F64OUT, V, pb, d_vols, d_tw, st);
     hipError_t le = hipGetLastError();
     if (le != hipSuccess) return done(fail(QSM_EHIP, "kernel launch: %s", hipGetErrorString(le)));
     if (hv) prefault(hv->out, hv->n * sizeof(double));
@@ -1787,13 +1783,13 @@ void qsm_tv_unrolled_destroy(qsm_tv_unrolled* h) { unrolled_free(h); }
 int qsm_dipole_forward(const double* d_chi, const qsm_grid* grid, const double bdir[3], double* d_field,
                        void* stream) {
     g_err.clear();
-    return spectral_apply(P_Z_DIPOLE, 0, 0.0, d_chi, nullptr, grid, bdir, d_field, stream);
+    return spectral_apply(P_Z_DIPOLE, 0, 0.0, d_chi, grid, bdir, d_field, stream);
 }
 
 int qsm_dipole_adjoint(const double* d_field, const qsm_grid* grid, const double bdir[3], double* d_chi,
                        void* stream) {
     g_err.clear();
-    return spectral_apply(P_Z_DIPOLE, 0, 0.0, d_field, nullptr, grid, bdir, d_chi, stream);
+    return spectral_apply(P_Z_DIPOLE, 0, 0.0, d_field, grid, bdir, d_chi, stream);
 }
 
 // ------------------------------------- dipole operator, no allocation ----
@@ -1862,7 +1858,6 @@ int qsm_dipole_forward_noalloc(const double* d_chi, const qsm_grid* grid, const 
     V.bx = bdir[0] / bn; V.by = bdir[1] / bn; V.bz = bdir[2] / bn;
     V.field = d_chi;
     V.adj_out = d_field;
-    V.out = d_field;
     V.spec[SPEC_WORK] = reinterpret_cast<float2*>(base + kScratchSpecOff);
     hipStream_t st = (hipStream_t)stream;
     // The R2C pass writes the whole spectrum, so nothing needs clearing.
@@ -1904,7 +1899,7 @@ static int filter_host(int filt, double fa, const double* field, const uint8_t* 
     } else if ((rc = host_volume_upload(hv, field, mask, N))) {
         return done(rc);
     }
-    if ((rc = spectral_apply(P_Z_FILTER, filt, fa, d_f64, nullptr, grid, bdir, nullptr, nullptr,
+    if ((rc = spectral_apply(P_Z_FILTER, filt, fa, d_f64, grid, bdir, nullptr, nullptr,
                              wrapped ? P_R2C_WRAPLAP : P_R2C_F32, &hv)))
         return done(rc);
     if ((rc = host_volume_download(hv, chi_out, N))) return done(rc);
