@@ -11,8 +11,10 @@
 namespace qsmfft {
 
 constexpr int kMaxDirectLen = 1024;
-// Lengths with a prime factor above 13 run as chirp-z transforms through a
-// convolution of length M >= 2n - 1 <= kMaxDirectLen, so up to this length.
+// Lengths that neither the stages of fft_dense.hpp (n <= 512, prime factors up
+// to 256) nor those of fft_core.hpp (prime factors up to 13) take, the primes 257
+// ... 509, run as chirp-z transforms through a convolution of length M >= 2n - 1
+// <= kMaxDirectLen, so up to this length.
 constexpr int kMaxChirpLen = kMaxDirectLen / 2;
 
 inline bool direct_length(int n) {
@@ -36,9 +38,8 @@ inline double stage_cost(int r) {
 
 // Convolution length of the chirp-z transform of length n: of the lengths
 // M >= 2n - 1 the stages handle directly (up to kMaxDirectLen), the one with
-// the least M * sum of its stage costs, so 512 = 8 8 8 is taken over
-// 468 = 4 3 3 13 for n = 232 (0 if there is none).  128, 256, 512 and 1024
-// count half: the runtime-plan kernels run them on compile-time stages.
+// the least M * sum of its stage costs (0 if there is none).  1024 counts half:
+// the runtime-plan kernels run it on compile-time stages.
 inline int chirp_length(int n) {
     int best = 0;
     double best_cost = 0.0;
@@ -48,7 +49,7 @@ inline int chirp_length(int n) {
         double c = 0.0;
         for (int i = 0; i < st; ++i) c += stage_cost(r[i]);
         c *= m;
-        if (m == 128 || m == 256 || m == 512 || m == 1024) c *= 0.5;
+        if (m == 1024) c *= 0.5;
         if (!best || c < best_cost) {
             best = m;
             best_cost = c;

@@ -28,7 +28,7 @@ constexpr int kMaxStages = 10;
 constexpr int kThreads = 256;  // threads per workgroup for every FFT kernel
 
 // Per-length plan.  Stored in device memory; read with uniform loads.
-// A length with a prime factor above 13 runs as a chirp-z (Bluestein)
+// A prime length above 256 runs as a chirp-z (Bluestein)
 // transform: bl_n is then the axis length, n the convolution length M the
 // stages run at, bl_chirp / bl_filt the offsets of its chirp and filter
 // tables (see bluestein_fft); bl_n = 0 for a direct transform.
