@@ -464,7 +464,8 @@ struct qsm_tv_batch {
     int method = 0;  // 0 TV-ADMM (src/inversion/tv.rs), 1 RTS (src/inversion/rts.rs)
     // The fused z/u update clamps to [-t, t], t = lambda / rho >= 0; for any
     // other t (a negative lambda, say) the recording kernel, which forms
-    // shrink itself, runs in its place with a scratch record.
+    // shrink itself, runs in its place with a scratch record, from the second
+    // iteration on.
     bool plain_shrink = false;
     bool streams = false;  // larger than the Infinity Cache (kStreamBytes)
     bool field32 = false;  // the field is VolDesc::vs_local, in f32 (host entry points)
@@ -835,9 +836,11 @@ static bool change_unread(const qsm_tv_batch* B, size_t it) {
 static int enqueue_iteration(qsm_tv_batch* B, size_t it, hipEvent_t closed, int rec = -1) {
     PassArgs a = B->args(B->d_status);
     a.parity = (int)((it - 1) & 1);
-    if (B->method == 1 && it == 1) {
-        // RTS starts from x0 != 0 with g = u = 0: the first step is x^ = f^
-        // (no z/u update and no divergence).
+    if (it == 1 && (B->method == 1 || B->plain_shrink)) {
+        // The first step is x^ = f^, from g = u = 0: no z/u update comes before
+        // it (src/inversion/admm.rs:76-145).  TV with t >= 0 runs the whole pass:
+        // on x_0 = u = 0 its update gives 0.  (shrink(0, t < 0) is -t, and RTS
+        // has x_0 != 0.)
         run_groups(P_Z_TV_SOLVE0, B->gz, a);
         run_groups(P_Y_INV, B->gy, a);
         run_groups(P_C2R_TV, B->gxc, a);
@@ -890,6 +893,7 @@ static int enqueue_setup(qsm_tv_batch* B) {
         const size_t N = (size_t)V.nx * V.ny * V.nz;
         launch_fill_zero(st, V.x[0], N);
         launch_fill_zero(st, V.u[1], 3 * N);
+        if (B->plain_shrink) launch_fill_zero(st, V.u[0], 3 * N);  // (what the second iteration reads)
     }
     launch_status_reset(st, B->d_status, B->nvol);
     PassArgs a = B->args(nullptr);
