@@ -17,6 +17,7 @@
 #include <cstring>
 #include <list>
 #include <mutex>
+#include <new>
 #include <unordered_map>
 #include <vector>
 
@@ -52,6 +53,19 @@ struct Store {
     std::vector<void*> pinned;
     std::vector<Lane> lanes;                                  // idle lanes
 };
+
+// Adds to one of the store's containers; false where the host has no memory for
+// that, and the caller gives the object back to the runtime instead.  (Nothing
+// here throws: these are the calls that free.)
+template <class F>
+bool kept_by(F&& add) noexcept {
+    try {
+        add();
+        return true;
+    } catch (const std::bad_alloc&) {
+        return false;
+    }
+}
 
 // Never destroyed: the runtime may be gone when static objects are.
 Store& store() {
@@ -112,10 +126,7 @@ void lane_give(Lane& l) {
         std::lock_guard<std::mutex> lk(s.mu);
         int have = 0;
         for (const Lane& k : s.lanes) have += k.dev == l.dev;
-        if (have < kLanesKept) {
-            s.lanes.push_back(l);
-            return;
-        }
+        if (have < kLanesKept && kept_by([&] { s.lanes.push_back(l); })) return;
     }
     lane_destroy(l);
 }
@@ -223,8 +234,8 @@ hipError_t workspace_alloc(void** p, size_t bytes) {
                 (best == s.kept.end() || it->bytes < best->bytes))
                 best = it;
         if (best != s.kept.end()) {
+            if (!kept_by([&] { s.live.emplace(best->p, *best); })) return hipErrorOutOfMemory;
             *p = best->p;
-            s.live[best->p] = *best;
             s.kept_bytes -= best->bytes;
             s.kept.erase(best);
             return hipSuccess;
@@ -235,34 +246,41 @@ hipError_t workspace_alloc(void** p, size_t bytes) {
         *p = nullptr;
         return e;
     }
-    std::lock_guard<std::mutex> lk(s.mu);
-    s.live[*p] = Block{*p, want, dev};
-    return hipSuccess;
+    bool known;
+    {
+        std::lock_guard<std::mutex> lk(s.mu);
+        known = kept_by([&] { s.live.emplace(*p, Block{*p, want, dev}); });
+    }
+    if (known) return hipSuccess;
+    (void)hipFree(*p);
+    *p = nullptr;
+    return hipErrorOutOfMemory;
 }
 
 void workspace_free(void* p) {
     if (!p) return;
     Store& s = store();
-    std::vector<void*> back;
+    std::list<Block> back, node;
+    const bool noted = kept_by([&] { node.emplace_back(); });
     {
         std::lock_guard<std::mutex> lk(s.mu);
         auto it = s.live.find(p);
         if (it == s.live.end()) return;  // not one of ours
         const Block b = it->second;
         s.live.erase(it);
-        if (b.bytes > kWorkspaceKept / 2) {
-            back.push_back(p);
-        } else {
-            s.kept.push_back(b);
+        if (noted && b.bytes <= kWorkspaceKept / 2) {
+            node.front() = b;
+            s.kept.splice(s.kept.end(), node);
             s.kept_bytes += b.bytes;
             while (s.kept_bytes > kWorkspaceKept) {
                 s.kept_bytes -= s.kept.front().bytes;
-                back.push_back(s.kept.front().p);
-                s.kept.pop_front();
+                back.splice(back.end(), s.kept, s.kept.begin());
             }
+            p = nullptr;
         }
     }
-    for (void* q : back) (void)hipFree(q);
+    if (p) (void)hipFree(p);
+    for (const Block& q : back) (void)hipFree(q.p);
 }
 
 void workspace_trim() {
@@ -306,9 +324,15 @@ hipError_t stream_take(hipStream_t* out) {
         *out = nullptr;
         return e;
     }
-    std::lock_guard<std::mutex> lk(s.mu);
-    s.stream_dev[*out] = dev;
-    return hipSuccess;
+    bool known;
+    {
+        std::lock_guard<std::mutex> lk(s.mu);
+        known = kept_by([&] { s.stream_dev.emplace(*out, dev); });
+    }
+    if (known) return hipSuccess;
+    (void)hipStreamDestroy(*out);
+    *out = nullptr;
+    return hipErrorOutOfMemory;
 }
 
 void stream_give(hipStream_t st) {
@@ -317,10 +341,9 @@ void stream_give(hipStream_t st) {
     {
         std::lock_guard<std::mutex> lk(s.mu);
         auto it = s.stream_dev.find(st);
-        if (it != s.stream_dev.end() && s.streams.size() < kStreamsKept) {
-            s.streams.emplace_back(it->second, st);
+        if (it != s.stream_dev.end() && s.streams.size() < kStreamsKept &&
+            kept_by([&] { s.streams.emplace_back(it->second, st); }))
             return;
-        }
         s.stream_dev.erase(st);
     }
     (void)hipStreamDestroy(st);
@@ -348,10 +371,7 @@ void pinned_give(void* p) {
     {
         Store& s = store();
         std::lock_guard<std::mutex> lk(s.mu);
-        if (s.pinned.size() < kPinnedKept) {
-            s.pinned.push_back(p);
-            return;
-        }
+        if (s.pinned.size() < kPinnedKept && kept_by([&] { s.pinned.push_back(p); })) return;
     }
     (void)hipHostFree(p);
 }

@@ -1837,9 +1837,8 @@ static int scratch_address(unsigned char** out) {
     return QSM_OK;
 }
 
-int qsm_dipole_forward_noalloc(const double* d_chi, const qsm_grid* grid, const double bdir[3],
+static int dipole_noalloc_impl(const double* d_chi, const qsm_grid* grid, const double bdir[3],
                                double* d_field, void* stream) {
-    g_err.clear();
     if (!d_chi || !grid || !bdir || !d_field) return fail(QSM_EPARAM, "null argument");
     int rc = validate_grid(grid);
     if (rc) return rc;
@@ -1872,6 +1871,16 @@ int qsm_dipole_forward_noalloc(const double* d_chi, const qsm_grid* grid, const 
     // the host-side tables above live on this stack frame: wait before returning
     QSM_HIP(hipStreamSynchronize(st));
     return QSM_OK;
+}
+
+int qsm_dipole_forward_noalloc(const double* d_chi, const qsm_grid* grid, const double bdir[3],
+                               double* d_field, void* stream) {
+    g_err.clear();
+    try {
+        return dipole_noalloc_impl(d_chi, grid, bdir, d_field, stream);
+    } catch (const std::bad_alloc&) {  // (the tables, before any device work)
+        return QSM_ENOMEM;
+    }
 }
 
 // Host-array wrapper of a closed-form inversion (filter kind, parameter).

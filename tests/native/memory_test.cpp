@@ -104,11 +104,57 @@ size_t table_upload(size_t n, long fail) {
     return dev().uploaded;
 }
 
+// Calls whose own host allocations fail, one after the other: handing a block
+// back must neither throw nor lose the block, and the entry point without device
+// allocations returns a status.
+template <class F>
+bool stays_in(F&& call) {
+    try {
+        call();
+    } catch (...) {
+        alloc_countdown = -1;
+        return false;
+    }
+    alloc_countdown = -1;
+    return true;
+}
+void host_memory() {
+    const qsm_grid g = {16, 16, 16, 1.0, 1.0, 1.0};
+    qsm_tv_volume v = {};
+    v.grid = g;
+    v.bdir[2] = 1.0;
+    v.d_field = fake(0);
+    v.d_mask = reinterpret_cast<uint8_t*>(fake(1));
+    v.d_chi = fake(2);
+    const qsm_tv_params prm = {1e-3, 0.1, 0.0, 3};
+    for (long fail = 1; fail <= 12; ++fail) {
+        qsm_release_cached_memory();
+        const size_t before = dev().used;
+        qsm_tv_batch* b = nullptr;
+        check(qsm_tv_batch_create(&v, 1, &prm, nullptr, &b) == QSM_OK, "batch");
+        check(stays_in([&] { alloc_countdown = fail; qsm_tv_batch_destroy(b); }), "destroy");
+        qsm_release_cached_memory();
+        check(dev().used == before, "every block back");
+    }
+    for (long fail = 1; fail <= 12; ++fail) {
+        int rc = -1;
+        check(stays_in([&] {
+                  alloc_countdown = fail;
+                  rc = qsm_dipole_forward_noalloc(fake(0), &g, kZ, fake(1), kUserStream);
+              }),
+              "without device allocations");
+        check(rc == QSM_OK || rc == QSM_ENOMEM, "its status");
+        check(qsm_dipole_forward_noalloc(fake(0), &g, kZ, fake(1), kUserStream) == QSM_OK, "and the next call");
+    }
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
     if (argc == 2 && !std::strcmp(argv[1], "device")) {
         device_memory();
+    } else if (argc == 2 && !std::strcmp(argv[1], "host")) {
+        host_memory();
     } else if (argc == 3 && !std::strcmp(argv[1], "tables")) {
         // lengths of every kind of table: register radices, dense, chirp-z
         const long fail = std::atol(argv[2]);

@@ -29,6 +29,10 @@ def test_kept_memory_is_given_back_to_own_calls(exe):
     _run(exe, "device")
 
 
+def test_failed_host_allocations_stay_inside(exe):
+    _run(exe, "host")
+
+
 # The allocations of a call come in this order: the volume's descriptor and
 # tables one axis at a time, each table growing in steps; 40 covers them all
 # for the shortest length and the tables of the longest.
