@@ -647,7 +647,12 @@ __device__ __forceinline__ void tvdiv_compute(const TvDivRound<CH, W>& R, float2
 // from x and u at i-1 (likewise y and z), so g never goes to memory.
 // Rounds of CH elements (2*CH voxels) are software-pipelined: the loads of
 // round r+1 are issued before round r is computed and stored.
-template <int EMAX, bool REC, bool W = false, bool NT = false>
+// RT: row length and rows known at run time only.  Such a block may fill a small
+// part of its tile, so the fills end with its elements: each round past them had
+// every thread load voxel 0 and its neighbours (six volumes of 16x64x48, 10
+// unrolled iterations and their gradient in blocks of 8 rows: 1.06 ms with those
+// rounds, 0.85 without).
+template <int EMAX, bool REC, bool W, bool NT, bool RT>
 __device__ __forceinline__ void fill_tvdiv(float2* lds, const VolDesc& V, int nx, int RB,
                                            const QSM_GLOBAL float* __restrict__ x,
                                            const QSM_GLOBAL float* __restrict__ u,
@@ -658,14 +663,17 @@ __device__ __forceinline__ void fill_tvdiv(float2* lds, const VolDesc& V, int nx
     constexpr int CH = (W || EMAX <= kRowEmaxRt) ? 1 : 2;
     constexpr int NR = (EMAX + CH - 1) / CH;
     const int total = RB * nx;
+    // round r holds elements of the block (a constant where N is)
+    auto has = [&](int r) { return r < NR && (!RT || r * CH * kThreads < total); };
     TvDivRound<CH, W> A, B;
     tvdiv_load<CH, W>(A, V, nx, 0, EMAX, total, row0, nrows, x, u, w);
 #pragma unroll
     for (int r = 0; r < NR; r += 2) {
-        if (r + 1 < NR) tvdiv_load<CH, W>(B, V, nx, (r + 1) * CH, EMAX, total, row0, nrows, x, u, w);
+        if (RT && !has(r)) break;
+        if (has(r + 1)) tvdiv_load<CH, W>(B, V, nx, (r + 1) * CH, EMAX, total, row0, nrows, x, u, w);
         tvdiv_compute<CH, REC, W, NT>(A, lds, V, r * CH, EMAX, total, uo, rec, wnorm);
-        if (r + 1 < NR) {
-            if (r + 2 < NR) tvdiv_load<CH, W>(A, V, nx, (r + 2) * CH, EMAX, total, row0, nrows, x, u, w);
+        if (has(r + 1)) {
+            if (has(r + 2)) tvdiv_load<CH, W>(A, V, nx, (r + 2) * CH, EMAX, total, row0, nrows, x, u, w);
             tvdiv_compute<CH, REC, W, NT>(B, lds, V, (r + 1) * CH, EMAX, total, uo, rec, wnorm);
         }
     }
@@ -1233,7 +1241,7 @@ __device__ __forceinline__ void fill_tvdiv_runtime(float2* lds, const VolDesc& V
 // still due); then g was overwritten with grad(x).  So: u' = u or
 // v - shrink(v, t w_old) with v = grad x + u, and the divergence source is
 // bdiv(grad x).
-template <int EMAX>
+template <int EMAX, bool RT>
 __device__ __forceinline__ void fill_nltv_boundary(float2* lds, const VolDesc& V, int nx, int RB,
                                                    const QSM_GLOBAL float* __restrict__ x,
                                                    const QSM_GLOBAL float* __restrict__ u,
@@ -1246,6 +1254,7 @@ __device__ __forceinline__ void fill_nltv_boundary(float2* lds, const VolDesc& V
     const int total = RB * nx;
 #pragma unroll
     for (int tt = 0; tt < EMAX; ++tt) {
+        if (RT && tt * kThreads >= total) break;
         const int e = threadIdx.x + tt * kThreads;
         const int p = e / nx;
         const int i = e - p * nx;
@@ -1308,7 +1317,7 @@ __device__ __forceinline__ float adj_sbar(float g, float so, int8_t q) {
     return q != 0 ? -g : so + g;
 }
 
-template <int EMAX, bool FIRST>
+template <int EMAX, bool FIRST, bool RT>
 __device__ __forceinline__ void fill_tvadj(float2* lds, const VolDesc& V, int nx, int RB, int row0,
                                            int nrows, int ck, int par, double& tsum) {
     const int ny = V.ny, nz = V.nz;
@@ -1323,6 +1332,7 @@ __device__ __forceinline__ void fill_tvadj(float2* lds, const VolDesc& V, int nx
     tsum = 0.0;
 #pragma unroll
     for (int t = 0; t < EMAX; ++t) {
+        if (RT && t * kThreads >= total) break;
         const int e = threadIdx.x + t * kThreads;
         const int p = e / nx;
         const int i = e - p * nx;
@@ -1443,24 +1453,24 @@ __global__ __launch_bounds__(kThreads) void k_r2c_x(const VolDesc* __restrict__ 
     } else if constexpr (SRC == SRC_TVDIV && N == 0 && eg_dense(EG)) {
         fill_tvdiv_runtime<NT>(lds, V, nx, RB, row0, nrows, glb(V.x[aux]), glb(V.u[aux ^ 1]), glb(V.u[aux]));
     } else if constexpr (SRC == SRC_TVDIV) {
-        fill_tvdiv<EMAX, false, false, NT>(lds, V, nx, RB, glb(V.x[aux]), glb(V.u[aux ^ 1]), glb(V.u[aux]), row0,
-                                nrows, nullptr);
+        fill_tvdiv<EMAX, false, false, NT, N == 0>(lds, V, nx, RB, glb(V.x[aux]), glb(V.u[aux ^ 1]), glb(V.u[aux]),
+                                                   row0, nrows, nullptr);
     } else if constexpr (SRC == SRC_TVDIV_REC) {
         const size_t N3 = (size_t)3 * V.nx * V.ny * V.nz;
-        fill_tvdiv<EMAX, true>(lds, V, nx, RB, glb(V.x[aux]), glb(V.u[aux ^ 1]), glb(V.u[aux]), row0,
-                               nrows, glb(V.ckpt) + (size_t)ck * N3);
+        fill_tvdiv<EMAX, true, false, false, N == 0>(lds, V, nx, RB, glb(V.x[aux]), glb(V.u[aux ^ 1]), glb(V.u[aux]),
+                                                     row0, nrows, glb(V.ckpt) + (size_t)ck * N3);
     } else if constexpr (SRC == SRC_TVDIV_W) {
-        fill_tvdiv<EMAX, false, true>(lds, V, nx, RB, glb(V.x[aux]), glb(V.u[aux ^ 1]), glb(V.u[aux]),
-                                      row0, nrows, nullptr, glb(V.nltv_w[ck]), (float)V.nltv_wnorm[ck]);
+        fill_tvdiv<EMAX, false, true, false, N == 0>(lds, V, nx, RB, glb(V.x[aux]), glb(V.u[aux ^ 1]), glb(V.u[aux]),
+                                                     row0, nrows, nullptr, glb(V.nltv_w[ck]), (float)V.nltv_wnorm[ck]);
     } else if constexpr (SRC == SRC_NLTV_BND) {
         // status_rw carries the convergence state of the round just ended
-        fill_nltv_boundary<EMAX>(lds, V, nx, RB, glb(V.x[aux]), glb(V.u[aux ^ 1]), glb(V.u[aux]), row0,
+        fill_nltv_boundary<EMAX, N == 0>(lds, V, nx, RB, glb(V.x[aux]), glb(V.u[aux ^ 1]), glb(V.u[aux]), row0,
                                  nrows, status_rw[gv].done != 0, glb(V.nltv_w[ck]),
                                  (float)V.nltv_wnorm[ck]);
     } else if constexpr (SRC == SRC_TVADJ_FIRST || SRC == SRC_TVADJ) {
         __shared__ double sh[kThreads / 64];
         double ts;
-        fill_tvadj<EMAX, SRC == SRC_TVADJ_FIRST>(lds, V, nx, RB, row0, nrows, ck, aux, ts);
+        fill_tvadj<EMAX, SRC == SRC_TVADJ_FIRST, N == 0>(lds, V, nx, RB, row0, nrows, ck, aux, ts);
         if constexpr (SRC == SRC_TVADJ) {
             const double bt = block_sum(ts, sh);
             if (threadIdx.x == 0) glb(V.adj_tpart)[(size_t)ck * V.adj_nblk + lb] = bt;

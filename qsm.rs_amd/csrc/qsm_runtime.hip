@@ -273,11 +273,15 @@ static int default_rows_x(int nx) {
 // pair-rows: 40 us with 16 rows, 44 with 10, 69 with 4), else half a tile at
 // least (251 and 1536: 25 us with 8, 31 with 2).
 //
-// single: passes whose threads take single elements (all but the TV ones, whose
-// fill works row by row): two for each thread at least (V-SHARP of 12x144x96:
-// 177 us with 32 rows, 190 with 12); with a dense radix full blocks, which share
-// the coefficients among most rows, where there are 1.5 for every CU (356x144x96:
-// 593 us with 10 rows, 657 with 8; 398x64x48, 300 blocks: 457 with 10, 345 with 6).
+// ROWS_SINGLE: passes whose threads take single elements (all but the TV ones,
+// whose fill works row by row): two for each thread at least (V-SHARP of
+// 12x144x96: 177 us with 32 rows, 190 with 12); with a dense radix full blocks,
+// which share the coefficients among most rows, where there are 1.5 for every CU
+// (356x144x96: 593 us with 10 rows, 657 with 8; 398x64x48, 300 blocks: 457 with
+// 10, 345 with 6).  ROWS_UNROLLED: `rows` are the volume's own, since the solver
+// sums the threshold's gradient block by block, so six at least for batches (six
+// volumes of 16x64x48, 10 iterations and their gradient: 0.87 ms with 6, 1.22
+// with 2; one volume the same with both).
 // The rows change no bit of any value.
 constexpr size_t kCus = 256, kRowBlocks = 3 * kCus;
 // The largest dense radix of a length in fft_dense.hpp's stages, 0: none.
@@ -285,9 +289,11 @@ static int dense_radix(int n) {
     int r[qsmfft::kMaxStages], st = 0;
     return qsmfft::dense_factorize(n, r, &st) && st && r[0] > qsmfft::kMaxRegRadix ? r[0] : 0;  // (the largest comes first)
 }
-static int dense_rows_x(int n, size_t rows, bool single) {
+enum RowUse { ROWS_TV, ROWS_UNROLLED, ROWS_SINGLE };
+static int dense_rows_x(int n, size_t rows, RowUse use) {
+    const bool single = use == ROWS_SINGLE;
     const size_t most = default_rows_x(n) & ~1, rounds = (rows + kRowBlocks * most - 1) / (kRowBlocks * most);
-    const size_t least = single ? (2 * qsmfft::kThreads + n - 1) / n : 2;
+    const size_t least = single ? (2 * qsmfft::kThreads + n - 1) / n : (use == ROWS_UNROLLED ? 6 : 2);
     const auto even = [](size_t k) { return (k + 1) & ~(size_t)1; };  // the same rows for each of the fill's four waves
     size_t per = even(std::max((rows + kRowBlocks * rounds - 1) / (kRowBlocks * rounds), least));
     if (const int R = dense_radix(n)) {
@@ -310,16 +316,16 @@ static std::map<size_t, size_t> length_pairs(const VOLS* vols, size_t n_vols) {
     return pairs;
 }
 
-// rows, single: for dense lengths, see dense_rows_x.  xshift / cshift 2
+// rows, use: for dense lengths, see dense_rows_x.  xshift / cshift 2
 // (compiled lengths): the R2C / TV C2R passes take a quarter of their default
 // rows per block, as the kernels launched with PassArgs::xshift = 2 do (C2R:
 // half the R2C pass's rows before its shift).
-PassBlocks fill_geometry(VolDesc& V, const qsm_grid& g, TwiddleBank& tb, size_t rows, bool single,
+PassBlocks fill_geometry(VolDesc& V, const qsm_grid& g, TwiddleBank& tb, size_t rows, RowUse use,
                          int xshift = 0, int cshift = 0) {
     V.nx = (int)g.nx; V.ny = (int)g.ny; V.nz = (int)g.nz;
     V.nxh = (V.nx + 1) / 2;  // even nx: DC and Nyquist share column 0
     if (has_fixed_kernels(V.nx)) V.rows_x = qsmfft::shifted_rows(V.nx, xshift);
-    else V.rows_x = dense_length(V.nx) ? dense_rows_x(V.nx, rows, single) : default_rows_x(V.nx);
+    else V.rows_x = dense_length(V.nx) ? dense_rows_x(V.nx, rows, use) : default_rows_x(V.nx);
     // compiled C2R kernels take half the R2C pass's pair-rows (the previous
     // iterate stays in registers across the transform), the others what their
     // tile of 8 elements per thread holds (fewer did not pay: 9 us with 12 to 32
@@ -668,8 +674,6 @@ static int tv_batch_create_impl(const qsm_tv_volume* vols, size_t n_vols, const 
         xshift[v] = (fixed && (npairs + r0 - 1) / r0 < 1024 && (r0 >> 2) >= 4) ? 2 : 0;
         cshift[v] = (fixed && (npairs + rc - 1) / rc < 1024 && (r0 >> 2) / 2 >= 4) ? 2 : 0;
     }
-    // The unrolled solver sums the threshold's gradient block by block, so its
-    // rows are chosen by the volume's own shape, 8 a block or more.
     std::map<size_t, size_t> pairs = length_pairs(vols, n_vols);
     // (the quarter-row R2C pass has no non-temporal form: three 192x192x128
     // volumes, 566 MB, took 203 us an iteration, 205 with the other passes' forms)
@@ -680,8 +684,8 @@ static int tv_batch_create_impl(const qsm_tv_volume* vols, size_t n_vols, const 
     for (size_t v = 0; v < n_vols; ++v) {
         VolDesc& V = B->h[v];
         std::memset(&V, 0, sizeof V);
-        const size_t rows = unrolled ? std::max(pair_rows(vols[v].grid), 8 * kRowBlocks) : pairs[vols[v].grid.nx];
-        PassBlocks pb = fill_geometry(V, vols[v].grid, tb, rows, false, xshift[v], cshift[v]);
+        const size_t rows = unrolled ? pair_rows(vols[v].grid) : pairs[vols[v].grid.nx];
+        PassBlocks pb = fill_geometry(V, vols[v].grid, tb, rows, unrolled ? ROWS_UNROLLED : ROWS_TV, xshift[v], cshift[v]);
         const double* b = vols[v].bdir;
         double bn = std::sqrt(b[0] * b[0] + b[1] * b[1] + b[2] * b[2]);
         V.bx = b[0] / bn; V.by = b[1] / bn; V.bz = b[2] / bn;  // src/kernels/dipole.rs:39-43
@@ -1281,7 +1285,7 @@ static int spectral_apply(int zkind, int filt, double fa, const double* d_in, co
     VolDesc V;
     std::memset(&V, 0, sizeof V);
     TwiddleBank tb;
-    PassBlocks pb = fill_geometry(V, *grid, tb, pair_rows(*grid), true);
+    PassBlocks pb = fill_geometry(V, *grid, tb, pair_rows(*grid), ROWS_SINGLE);
     V.bx = bdir[0] / bn; V.by = bdir[1] / bn; V.bz = bdir[2] / bn;
     V.field = d_in;
     V.adj_out = d_out;
@@ -1430,7 +1434,7 @@ static int vs_create_impl(const qsm_vsharp_volume* vols, size_t n_vols, const do
         VolDesc& V = B->h[v];
         std::memset(&V, 0, sizeof V);
         // (the selection pass has twice as many rows as the others pair-rows)
-        PassBlocks pb = fill_geometry(V, vols[v].grid, tb, 2 * pairs[vols[v].grid.nx], true);
+        PassBlocks pb = fill_geometry(V, vols[v].grid, tb, 2 * pairs[vols[v].grid.nx], ROWS_SINGLE);
         V.field = vols[v].d_field;
         V.mask = vols[v].d_mask;
         V.out = vols[v].d_local;
@@ -1847,7 +1851,7 @@ static int dipole_noalloc_impl(const double* d_chi, const qsm_grid* grid, const 
     VolDesc V;
     std::memset(&V, 0, sizeof V);
     TwiddleBank tb;
-    PassBlocks pb = fill_geometry(V, *grid, tb, pair_rows(*grid), true);
+    PassBlocks pb = fill_geometry(V, *grid, tb, pair_rows(*grid), ROWS_SINGLE);
     const size_t spec_bytes = (size_t)V.nxh * V.ny * V.nz * sizeof(float2);
     if (spec_bytes > kScratchSpecBytes)
         return fail(QSM_EPARAM,

@@ -36,3 +36,35 @@ def test_batch_of_one_length_equals_single(qsm, nx):
             assert np.array_equal(one[v], both[v]) and np.array_equal(one_e[v], both_e[v])
     for d in (df, dm, dx, de):
         d.free()
+
+
+# the unrolled solver's rows follow the volume alone (its sum over blocks gives
+# the gradient of lambda); blocks that fill a small part of their tile, and all of it.
+# The problem and the bars against the oracle are those of test_gpu_adjoint.py
+@pytest.mark.parametrize("nx", [20, 82, 143, 338])
+def test_unrolled_batch_of_one_length_equals_single(qsm, oracle, nx):
+    dims, nv = (nx, 13, 10), 3
+    n = int(np.prod(dims))
+    rng = np.random.default_rng(nx)
+    f, chi_true = rng.standard_normal((nv, n)) * 0.02, rng.standard_normal((nv, n)) * 0.01
+    m = (rng.random((nv, n)) < 0.85).astype(np.uint8)
+    vs, b, lam0, rho, K = (1.0, 1.0, 1.0), (0.1, -0.2, 1.0), 2e-3, 0.1, 5
+    cb = np.stack([2.0 * (oracle.tv_admm(f[v], m[v], dims, vs, b, lam0, rho, 0.0, K) - chi_true[v])
+                   for v in range(nv)])
+    g, p = qsm.Grid(dims, vs), qsm.TvParams(lambda_=lam0, rho=rho, tol=0.0, max_iter=K)
+    df, dm, dc = (qsm.DeviceArray.from_numpy(a.ravel()) for a in (f, m, cb))
+    dx, dg = qsm.DeviceArray(nv * n, np.float64), qsm.DeviceArray(nv * n, np.float64)
+    u = qsm.TvUnrolled([(g, b, df.ptr + 8 * n * v, dm.ptr + n * v, dx.ptr + 8 * n * v) for v in range(nv)], p)
+    u.forward()
+    lam = u.backward([dc.ptr + 8 * n * v for v in range(nv)], [dg.ptr + 8 * n * v for v in range(nv)])
+    u.close()
+    chi, grad = dx.numpy().reshape(nv, n), dg.numpy().reshape(nv, n)
+    for v in range(nv):
+        one = qsm.tv_unrolled_vjp(f[v], m[v], g, b, p, cb[v])
+        assert np.array_equal(one[0], chi[v]) and np.array_equal(one[1], grad[v]) and one[2] == lam[v]
+        xo, go, lo = oracle.tv_unrolled_vjp(f[v], m[v], dims, vs, b, lam0, rho, K, cb[v])
+        assert oracle.nrmse(chi[v], xo, m[v]) <= 2e-5
+        assert np.linalg.norm(grad[v] - go) <= 2e-3 * np.linalg.norm(go)
+        assert abs(lam[v] - lo) <= 5e-3 * abs(lo)
+    for d in (df, dm, dc, dx, dg):
+        d.free()
